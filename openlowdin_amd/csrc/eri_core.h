@@ -147,21 +147,35 @@ struct EriClass;
   };
 
 
+// Sum of N accumulators over aligned groups of `size` lanes (a power of
+// two); every lane of a group ends with the sums.
+template <int N, typename R>
+__device__ __forceinline__ void group_sum(R* acc, int size) {
+  for (int m = size >> 1; m > 0; m >>= 1) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) acc[k] += __shfl_xor(acc[k], m, 64);
+  }
+}
+
 // Contracted raw quartet (canonical orientation) for one lane.  The ket's
 // primitive pairs (per lane, vector loads) form the outer loop and are read
 // once; the bra's primitive pairs (wave-uniform, scalar loads) the inner
 // one.  VRR accumulates [e0|f0] over all primitive quartets, then one HRR.
+// nsplit > 1 (a power of two): nsplit neighbouring lanes share one quartet,
+// lane `sub` of them taking every nsplit-th primitive pair of the ket, and
+// their [e0|f0] are summed before the HRR.
 template <int LA, int LB, int LC, int LD, int RS = kBoysCols, int FO = 1 + LA + LB + LC + LD, typename BP,
           typename KP, typename TP>
 __device__ __forceinline__ void contracted_quartet_body(BP bprim, int nbp, KP kprim, int nkp, TP boys,
                                                    double ABx, double ABy, double ABz, double CDx,
-                                                   double CDy, double CDz, double* out) {
+                                                   double CDy, double CDz, double* out, int sub = 0,
+                                                   int nsplit = 1) {
   using C = EriClass<LA, LB, LC, LD>;
   constexpr int L = LA + LB + LC + LD;
   double acc[C::nacc];
 #pragma unroll
   for (int k = 0; k < C::nacc; ++k) acc[k] = 0.0;
-  for (int kp = 0; kp < nkp; ++kp) {
+  for (int kp = sub; kp < nkp; kp += nsplit) {
     const auto kq = kprim + kp * kPrimPairStride;
     const double q = kq[0], o2q = kq[1];
     const double Qx = kq[2], Qy = kq[3], Qz = kq[4];
@@ -185,6 +199,7 @@ __device__ __forceinline__ void contracted_quartet_body(BP bprim, int nbp, KP kp
                               roq * PQx, roq * PQy, roq * PQz, o2p, o2q, 0.5 * inv, rop, roq, acc);
     }
   }
+  if (nsplit > 1) group_sum<C::nacc>(acc, nsplit);
   C::template hrr<double>(acc, ABx, ABy, ABz, CDx, CDy, CDz, out);
 }
 
@@ -237,14 +252,15 @@ template <int LA, int LB, int LC, int LD, int RS = kBoysF32Cols, int FO = 1 + LA
           typename KP, typename TP>
 __device__ __forceinline__ void contracted_quartet_f32_body(BP bprim, int nbp, KP kprim, int nkp, TP boys,
                                                        double ABx, double ABy, double ABz, double CDx,
-                                                       double CDy, double CDz, double* out) {
+                                                       double CDy, double CDz, double* out, int sub = 0,
+                                                   int nsplit = 1) {
   using C = EriClass<LA, LB, LC, LD>;
   constexpr int L = LA + LB + LC + LD;
   constexpr int NOUT = ncart(LA) * ncart(LB) * ncart(LC) * ncart(LD);
   float acc[C::nacc];
 #pragma unroll
   for (int k = 0; k < C::nacc; ++k) acc[k] = 0.0f;
-  for (int kp = 0; kp < nkp; ++kp) {
+  for (int kp = sub; kp < nkp; kp += nsplit) {
     const auto kq = kprim + kp * kPrimPairStride;
     const float q = kq[0], o2q = kq[1];
     const float Qx = kq[2], Qy = kq[3], Qz = kq[4];
@@ -268,6 +284,7 @@ __device__ __forceinline__ void contracted_quartet_f32_body(BP bprim, int nbp, K
                              roq * PQx, roq * PQy, roq * PQz, o2p, o2q, 0.5f * inv, rop, roq, acc);
     }
   }
+  if (nsplit > 1) group_sum<C::nacc>(acc, nsplit);
   float o[NOUT];
   C::template hrr<float>(acc, (float)ABx, (float)ABy, (float)ABz, (float)CDx, (float)CDy, (float)CDz, o);
 #pragma unroll
@@ -285,8 +302,9 @@ constexpr int kMaxNaccFp32 = 300;
 template <int LA, int LB, int LC, int LD, typename BP, typename KP, typename TP>
 __device__ __forceinline__ void contracted_quartet(BP bprim, int nbp, KP kprim, int nkp, TP boys, double ABx,
                                                    double ABy, double ABz, double CDx, double CDy, double CDz,
-                                                   double* out) {
-  contracted_quartet_body<LA, LB, LC, LD>(bprim, nbp, kprim, nkp, boys, ABx, ABy, ABz, CDx, CDy, CDz, out);
+                                                   double* out, int sub = 0, int nsplit = 1) {
+  contracted_quartet_body<LA, LB, LC, LD>(bprim, nbp, kprim, nkp, boys, ABx, ABy, ABz, CDx, CDy, CDz, out, sub,
+                                          nsplit);
 }
 
 template <int LA, int LB, int LC, int LD>
@@ -297,8 +315,10 @@ struct Fp32Allowed {
 template <int LA, int LB, int LC, int LD, typename BP, typename KP>
 __device__ __forceinline__ void contracted_quartet_f32(BP bprim, int nbp, KP kprim, int nkp,
                                                        const float* __restrict__ boys, double ABx, double ABy,
-                                                       double ABz, double CDx, double CDy, double CDz, double* out) {
-  contracted_quartet_f32_body<LA, LB, LC, LD>(bprim, nbp, kprim, nkp, boys, ABx, ABy, ABz, CDx, CDy, CDz, out);
+                                                       double ABz, double CDx, double CDy, double CDz, double* out,
+                                                       int sub = 0, int nsplit = 1) {
+  contracted_quartet_f32_body<LA, LB, LC, LD>(bprim, nbp, kprim, nkp, boys, ABx, ABy, ABz, CDx, CDy, CDz, out, sub,
+                                              nsplit);
 }
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -553,7 +573,8 @@ __host__ __device__ constexpr bool strip_lds_boys32(int lds_n, int block, int an
 // ------------------------------------------------ J/K kernel, LDS strips
 // A workgroup owns one bra pair (a b) and streams up to t.j1 - t.j0 ket
 // pairs, one per thread per round (256 threads, or one wavefront of 64 for
-// the short ket runs of small molecules).  Every J/K update of a quartet except
+// the short ket runs of small molecules), or one per group of up to 64 lanes
+// where the primitive loop of one lane would be long (JKArgs::lmax).  Every J/K update of a quartet except
 // J_cd lands in row a or row b of G (J_ab; K_ac, K_ad in row a; K_bc, K_bd
 // in row b), so those are accumulated with LDS atomics in two row strips
 // (NA + NB) x n held for the whole ket stream and flushed to HBM once, with
@@ -634,7 +655,14 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
   unsigned int myq = 0, myp = 0, myq32 = 0;
   const double sbra = (P.sa != P.sb ? 2.0 : 1.0);
   const double hf = M.half_factor;
-  for (int j = t.j0 + tid; j < t.j1; j += blockDim.x) {
+  int nround = 0;
+  for (int jr = t.j0; jr < t.j1; jr += nround) {
+    // lanes per quartet of this round of kets, from the primitive count of
+    // its first ket (the kets come in descending order of it)
+    const int ls = a.lmax > 0 ? split_shift(P.nprim, pairs[M.off[a.cket] + jr].nprim, a.lmax) : 0;
+    nround = (int)blockDim.x >> ls;
+    const int j = jr + (tid >> ls), sub = tid & ((1 << ls) - 1);
+    if (j >= t.j1) continue;
     const PairInfo K = load_pair(pairs + M.off[a.cket] + j);
     bool lo = false;
     if (M.screen || M.mixed) {
@@ -642,25 +670,22 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
       if (M.screen && dn * P.Q * K.Q < a.eps) continue;
       lo = kF32 && M.mixed && dn * P.Qn * K.Qn < M.tau;
     }
-    myq += 1;
-    myp += (unsigned int)(P.nprim * K.nprim);
     double out[NA * NB * NC * ND];
     if constexpr (kF32) {
       if (lo) {
-        myq32 += 1;
         bool done = false;
         if constexpr (StripLdsBoys<LA, LB, LC, LD>::value) {
           if (ldsb32) {
             contracted_quartet_f32_body<LA, LB, LC, LD, kLdsBoys32Cols, 1>(
                 (const float*)bpf, P.nprim, (gcptr<float>)M.primf + (size_t)K.poff * kPrimPairStride, K.nprim,
-                (const float*)btab32, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
+                (const float*)btab32, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out, sub, 1 << ls);
             done = true;
           }
         }
         if (!done)
           contracted_quartet_f32<LA, LB, LC, LD>((const float*)bpf, P.nprim,
                                                  (gcptr<float>)M.primf + (size_t)K.poff * kPrimPairStride,
-                                                 K.nprim, a.boysf, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
+                                                 K.nprim, a.boysf, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out, sub, 1 << ls);
       }
     }
     if (!lo) {
@@ -670,15 +695,19 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
           contracted_quartet_body<LA, LB, LC, LD, kLdsBoysCols, 1>((const double*)bpd, P.nprim,
                                                                    prim + (size_t)K.poff * kPrimPairStride,
                                                                    K.nprim, (const double*)btab, P.ABx, P.ABy,
-                                                                   P.ABz, K.ABx, K.ABy, K.ABz, out);
+                                                                   P.ABz, K.ABx, K.ABy, K.ABz, out, sub, 1 << ls);
           done = true;
         }
       }
       if (!done)
         contracted_quartet<LA, LB, LC, LD>((const double*)bpd, P.nprim,
                                            prim + (size_t)K.poff * kPrimPairStride, K.nprim, a.boys,
-                                           P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
+                                           P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out, sub, 1 << ls);
     }
+    if (sub != 0) continue;   // the first lane of a group applies the quartet's updates
+    myq += 1;
+    myp += (unsigned int)(P.nprim * K.nprim);
+    if (lo) myq32 += 1;
     const double deg = sbra * (K.sa != K.sb ? 2.0 : 1.0) * ((a.same_class && j == t.bra) ? 1.0 : 2.0);
     double nc[NC], nd[ND];
 #pragma unroll

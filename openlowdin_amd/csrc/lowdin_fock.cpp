@@ -190,6 +190,7 @@ struct TaskSet {
     size_t off, count;
     int strip;        // intra: one workgroup per task with LDS row strips (1: 256 threads, 2: 64);
                       // 3: wave-cooperative kernel with row strips, 4: the same without strips
+    int lmax = 0;         // intra strips: JKArgs::lmax
   };
   std::vector<Launch> launches;
   std::vector<size_t> order;   // launch order: estimated cost, largest first
@@ -515,6 +516,23 @@ constexpr int kCoopDefaultL = 6;
 constexpr int kCoopDefaultWg = 4096;
 constexpr long kCoopMinRun = 4;
 
+// Strip launches are cut into about target_wg workgroups of 256 threads
+// (four times as many of one wavefront) of equal estimated cost, a quartet
+// counting kQuartetIters primitive quartets beside its own: more pieces cost
+// more in zeroed, filled and flushed LDS than the even load gains (C20H42:
+// 512 -> 4096 workgroups 20.9 -> 22.5 ms).
+constexpr double kQuartetIters = 12.0;
+// Lanes share a quartet when one lane would take more than lmax primitive
+// quartets one after another: that serial loop (up to 8^4 for cc-pVDZ carbon)
+// is what a small build waits for, and what leaves the lanes of a wavefront
+// and the waves of a workgroup uneven in a large one.  Long ket rows fill the
+// lanes by themselves, so lmax grows with the kets per bra.  Measured, lmax
+// 5000 (never shared) / 64 / 16: water 6-31G** 1066 / 782 / 569 us,
+// (H2O)10 3.51 / 3.31 / 3.22 ms, C20H42 21.1 / 20.7 / 22.0 ms (its (ss|ss)
+// alone 2.99 / 1.76 / 2.23 ms), 72 clusters in a batch 26.6 / 25.1 / 23.7 ms.
+constexpr double kSplitMin = 16.0, kSplitMax = 64.0;
+constexpr double kSplitKets = 32.0;   // kets per bra for each unit of lmax
+
 static inline int class_pair_id(int cx, int cy) { return cx * (cx + 1) / 2 + cy; }
 
 static void ensure_sig(Species& s, hipStream_t st) {
@@ -552,10 +570,28 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
     p.nshmax = std::max(p.nshmax, ns);
   }
   std::vector<double> cost;
-  auto task_cost = [&](const Task& t, int cx, int cy) {
-    const PairSet& ps = p.mols[t.flags]->sig;
-    return (double)ps.pairs[ps.off[cx] + t.bra].nprim * ps.pairs[ps.off[cy] + t.j0].nprim * (t.j1 - t.j0);
+  std::vector<std::pair<double, Task>> made;   // tasks of the launch at hand with their estimated costs
+  // runs of kets with equal primitive counts and the primitive counts summed
+  // up to each ket, per molecule and pair class
+  struct Run {
+    int j0, j1, np;
   };
+  std::vector<std::array<std::vector<Run>, kNumPairClasses>> runs(nm);
+  std::vector<std::vector<double>> psum(nm);
+  for (int m = 0; m < nm; ++m) {
+    const PairSet& ps = p.mols[m]->sig;
+    psum[m].assign(ps.pairs.size() + 1, 0.0);
+    for (int c = 0; c < kNumPairClasses; ++c)
+      for (int k = ps.off[c]; k < ps.off[c + 1]; ++k) {
+        std::vector<Run>& r = runs[m][c];
+        const int j = k - ps.off[c];
+        if (r.empty() || r.back().np != ps.pairs[k].nprim) r.push_back(Run{j, j, ps.pairs[k].nprim});
+        r.back().j1 = j + 1;
+        psum[m][k + 1] = psum[m][k] + ps.pairs[k].nprim;
+      }
+  }
+  std::vector<double> unit, upto;   // per run: cost of a quartet, cost of the kets before the run
+  std::vector<int> round;           // per run: kets a workgroup takes at once
   for (int cx = 0; cx < kNumPairClasses; ++cx) {
     for (int cy = 0; cy <= cx; ++cy) {
       const int la = kPairClassL[cx][0], lb = kPairClassL[cx][1];
@@ -589,39 +625,101 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
       const bool strip = coop || (strip_ok && (kd == 1 || kd == 3 || kd == 0));
       const bool wave64 = kd == 3 || (kd == 0 && total < 192 * nbras);
       const size_t from = ts.tasks.size();
-      // run length: at least enough kets to amortise zeroing and flushing the
-      // strips (which grow with n), at most 32768
-      const long cmin = coop ? kCoopMinRun : std::max(64L, std::min(256L, (long)((p.nmax / 2 + 63) / 64) * 64));
+      const int block = wave64 ? 64 : 256;
       const long tgt = coop_default ? kCoopDefaultWg : p.target_wg[class_pair_id(cx, cy)];
-      long chunk = (total + tgt - 1) / tgt;
-      chunk = std::max(cmin, std::min(32768L, coop ? ((chunk + 3) / 4) * 4 : ((chunk + 63) / 64) * 64));
+      made.clear();
+      double work = 0.0;   // primitive quartets of the launch
+      for (int m = 0; m < nm; ++m) {
+        const PairSet& ps = p.mols[m]->sig;
+        for (int i = 0; i < ps.off[cx + 1] - ps.off[cx]; ++i) {
+          const int nk = (cx == cy) ? i + 1 : ps.off[cy + 1] - ps.off[cy];
+          work += (psum[m][ps.off[cy] + nk] - psum[m][ps.off[cy]]) * ps.pairs[ps.off[cx] + i].nprim;
+        }
+      }
+      int lmax = 0;
+      if (strip && !coop) {
+        lmax = (int)std::max(kSplitMin, std::min(kSplitMax, (double)total / (kSplitKets * (double)nbras)));
+      }
+      const double flush = 8.0 + (double)(ncart_h(la) + ncart_h(lb)) * p.nmax / block;
+      const double goal = (wave64 ? 4.0 : 1.0) * (double)tgt;
+      const double cap = std::max((work + kQuartetIters * (double)total) / goal, 4.0 * block * flush);
+      const long chunk = std::max(kCoopMinRun, std::min(32768L, ((total + tgt - 1) / tgt + 3) / 4 * 4));
       for (int m = 0; m < nm; ++m) {
         const PairSet& ps = p.mols[m]->sig;
         const int nx = ps.off[cx + 1] - ps.off[cx], ny = ps.off[cy + 1] - ps.off[cy];
         if (nx == 0 || ny == 0) continue;
         const PairInfo* kets = ps.pairs.data() + ps.off[cy];
+        const std::vector<Run>& kr = runs[m][cy];
+        unit.resize(kr.size());
+        upto.resize(kr.size());
+        round.resize(kr.size());
+        int last = -1;   // primitive count of the bra the per-run costs are for
+        size_t rk = 0;
         for (int i = 0; i < nx; ++i) {
-          const int nk = (cx == cy) ? i + 1 : ny;
-          if (strip) {
+          const int nk = (cx == cy) ? i + 1 : ny, nbp = ps.pairs[ps.off[cx] + i].nprim;
+          if (coop) {
             const int pieces = (int)((nk + chunk - 1) / chunk);
             for (int q = 0; q < pieces; ++q) {
               const int j0 = (int)((long)nk * q / pieces), j1 = (int)((long)nk * (q + 1) / pieces);
-              if (j1 > j0) ts.tasks.push_back(Task{i, j0, j1, m});
+              if (j1 > j0) made.push_back({(double)nbp * kets[j0].nprim * (j1 - j0), Task{i, j0, j1, m}});
+            }
+          } else if (strip) {
+            // pieces of about equal cost, cut at whole rounds of the workgroup
+            if (nbp != last) {
+              double c = 0.0;
+              for (size_t r = 0; r < kr.size(); ++r) {
+                const int ls = split_shift(nbp, kr[r].np, lmax);
+                unit[r] = (double)nbp * kr[r].np + kQuartetIters * (double)(1 << ls);
+                round[r] = block >> ls;
+                upto[r] = c;
+                c += unit[r] * (kr[r].j1 - kr[r].j0);
+              }
+              last = nbp;
+              rk = 0;
+            }
+            if (cx != cy) rk = kr.size() - 1;
+            while (kr[rk].j1 < nk) ++rk;   // the run of the last ket
+            while (kr[rk].j0 >= nk) --rk;
+            const double all = upto[rk] + unit[rk] * (nk - kr[rk].j0);
+            if (all <= cap) {
+              made.push_back({all, Task{i, 0, nk, m}});
+              continue;
+            }
+            const double share = all / std::ceil(all / cap) * (1.0 - 1e-9);
+            double acc = 0.0;
+            int j0 = 0;
+            for (size_t r = 0; r <= rk; ++r) {
+              const int end = std::min(kr[r].j1, nk);
+              for (int j = kr[r].j0; j < end;) {
+                const int want = (int)std::min(1e9, std::ceil((share - acc) / unit[r]));
+                const int take = std::min(end - j, std::max(1, (want + round[r] - 1) / round[r]) * round[r]);
+                acc += take * unit[r];
+                j += take;
+                if (acc >= share || j == nk) {
+                  made.push_back({acc, Task{i, j0, j, m}});
+                  j0 = j;
+                  acc = 0.0;
+                }
+              }
             }
           } else {
+            const size_t at = ts.tasks.size();
             emit_tasks(ts.tasks, i, 0, nk, kets, m);
+            for (size_t k = at; k < ts.tasks.size(); ++k) {
+              const Task& t = ts.tasks[k];
+              made.push_back({(double)nbp * kets[t.j0].nprim * (t.j1 - t.j0), t});
+            }
+            ts.tasks.resize(at);
           }
         }
       }
-      std::stable_sort(ts.tasks.begin() + from, ts.tasks.end(),
-                       [&](const Task& x, const Task& y) { return task_cost(x, cx, cy) > task_cost(y, cx, cy); });
+      std::stable_sort(made.begin(), made.end(),
+                       [](const std::pair<double, Task>& x, const std::pair<double, Task>& y) { return x.first > y.first; });
+      for (const auto& t : made) ts.tasks.push_back(t.second);
       ts.launches.push_back({la, lb, lc, ld, cx, cy, 1, from, ts.tasks.size() - from,
-                             coop ? coop : (strip ? (wave64 ? 2 : 1) : 0)});
+                             coop ? coop : (strip ? (wave64 ? 2 : 1) : 0), lmax});
       // estimated cost of the launch: primitive quartets x class weight
-      const double w = 1.0 + (la + lb + lc + ld) * (la + lb + lc + ld);
-      double c = 0.0;
-      for (size_t t = from; t < ts.tasks.size(); ++t) c += w * task_cost(ts.tasks[t], cx, cy);
-      cost.push_back(c);
+      cost.push_back(work * (1.0 + (la + lb + lc + ld) * (la + lb + lc + ld)));
     }
   }
   ts.order.resize(ts.launches.size());
@@ -822,6 +920,7 @@ static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, int which,
     if (L.strip == 4) a.lds_n = 0;
     a.eps = p.eps;  // DBL_EPSILON by default (Libint2Iface.h:269-271)
     a.any_mixed = p.any_mixed ? 1 : 0;
+    a.lmax = L.lmax;
     if (timed) HIPCHK(hipEventRecord(p.launch_ev[2 * k], ls));
     const bool ok = L.strip >= 3 ? dispatch_jk_coop(L.la, L.lb, L.lc, L.ld, a, ls)
                     : L.strip    ? dispatch_jk_strip(L.la, L.lb, L.lc, L.ld, a, ls)

@@ -42,7 +42,18 @@ struct JKArgs {
   int block;               // strip kernel: threads per workgroup (0: 256)
   double eps;
   int any_mixed;           // some molecule of the launch runs mixed precision
+  int lmax;                // strip kernel: primitive quartets a lane takes one after another before
+                           // lanes share a quartet (0: one lane per quartet)
 };
+
+// log2 of the lanes that share a quartet of nbp x nkp primitive pairs: as few
+// as bring the serial loop of a lane down to lmax primitive quartets, at most
+// one wavefront and no more than the ket has primitive pairs.
+__host__ __device__ inline int split_shift(int nbp, int nkp, int lmax) {
+  int ls = 0;
+  while (ls < 6 && (1 << ls) < nkp && nbp * ((nkp + (1 << ls) - 1) >> ls) > lmax) ++ls;
+  return ls;
+}
 
 // Per molecule of a batched symmetrisation.
 struct SymDesc {
