@@ -231,7 +231,7 @@ int lowdin_fock_compute_2body_device(void* lint, const double* d_dens, double* d
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  The build's scratch -- descriptors, the shell-block norms of
  * D and the raw n x n accumulator -- lives in a file-scope device array of
- * the library (5.8 MB, one copy per GPU, held until the process ends), so
+ * the library (10.7 MB, one copy per GPU, held until the process ends), so
  * the basis is limited to 768 functions and 384 shells; larger ones are
  * refused with an error.  The species must have been built once by
  * LibintInterface_compute_2body_direct or lowdin_fock_compute_2body_device

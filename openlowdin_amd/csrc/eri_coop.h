@@ -262,6 +262,9 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
   const gptr<double> G = (gptr<double>)M.Graw;
   const PairInfo P = load_pair(pairs + M.off[a.cbra] + t.bra);
   const int n = M.n, ns = M.nshell;
+  const int npk = M.off[a.cket + 1] - M.off[a.cket];
+  const gcptr<double> Dp = (gcptr<double>)M.Dp + M.jpoff[a.cket];
+  const gptr<double> Jp = (gptr<double>)M.Jp + M.jpoff[a.cket];
   const int sn = a.lds_n;                 // strip width (0: no strips)
   double* sa = lds;
   double* sb = lds + NA * sn;
@@ -297,21 +300,19 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
     // J/K contraction of the (ab|cd) block (Libint2Iface.cpp:562-586)
     const double* out = R + Pg::kOut;
     const double deg = sbra * (K.sa != K.sb ? 2.0 : 1.0) * ((a.same_class && j == t.bra) ? 1.0 : 2.0);
-    for (int k = lane; k < NCD + NA * NC + NB * ND + NA * ND + NB * NC; k += 64) {
+    for (int k = lane; k < NCD; k += 64) R[oDcd + k] = Dp[(size_t)k * npk + j];
+    for (int k = lane; k < NA * NC + NB * ND + NA * ND + NB * NC; k += 64) {
       int r0, c0, o;
-      if (k < NCD) {
-        r0 = K.bfa + k / ND; c0 = K.bfb + k % ND; o = oDcd + k;
-      } else if (k < NCD + NA * NC) {
-        const int u = k - NCD;
-        r0 = P.bfa + u / NC; c0 = K.bfa + u % NC; o = oDac + u;
-      } else if (k < NCD + NA * NC + NB * ND) {
-        const int u = k - NCD - NA * NC;
+      if (k < NA * NC) {
+        r0 = P.bfa + k / NC; c0 = K.bfa + k % NC; o = oDac + k;
+      } else if (k < NA * NC + NB * ND) {
+        const int u = k - NA * NC;
         r0 = P.bfb + u / ND; c0 = K.bfb + u % ND; o = oDbd + u;
-      } else if (k < NCD + NA * NC + NB * ND + NA * ND) {
-        const int u = k - NCD - NA * NC - NB * ND;
+      } else if (k < NA * NC + NB * ND + NA * ND) {
+        const int u = k - NA * NC - NB * ND;
         r0 = P.bfa + u / ND; c0 = K.bfb + u % ND; o = oDad + u;
       } else {
-        const int u = k - NCD - NA * NC - NB * ND - NA * ND;
+        const int u = k - NA * NC - NB * ND - NA * ND;
         r0 = P.bfb + u / NC; c0 = K.bfa + u % NC; o = oDbc + u;
       }
       R[o] = D[(size_t)r0 * n + c0] * nrm[r0] * nrm[c0];
@@ -326,8 +327,7 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
       double s = 0.0;
 #pragma unroll 6
       for (int ab = 0; ab < NAB; ++ab) s += out[ab * NCD + lane] * R[oDab + ab];
-      const int fc = K.bfa + lane / ND, fd = K.bfb + lane % ND;
-      global_add(G + (size_t)fc * n + fd, deg * s * nrm[fc] * nrm[fd]);
+      global_add(Jp + (size_t)lane * npk + j, deg * s);
     }
     const double sk = deg * hf;
     if (lane < NA * NC) {  // K_ac = sum_bd (ab|cd) D_bd

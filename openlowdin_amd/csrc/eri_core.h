@@ -340,13 +340,16 @@ __device__ __forceinline__ double quartet_dnorm(gcptr<double> Dn, int ns, const 
 }
 
 // The J/K updates of one quartet's raw block (out), normalised and weighted
-// by deg: J_cd, K_ac, K_bd, K_ad and K_bc go to G with FP64 atomics; J_ab is
-// added into jab (unscaled by deg and the bra norms) for the caller to reduce.
+// by deg: K_ac, K_bd, K_ad and K_bc go to G with FP64 atomics, and so does
+// J_cd, to G or (Jp not null) to the packed accumulator at Jp, jstride doubles
+// from one element of the block to the next; J_ab is added into jab (unscaled
+// by deg and the bra norms) for the caller to reduce.
 // Libint2Iface.cpp:562-586 (exchange weight 0.5 * factor = half_factor).
 template <int LA, int LB, int LC, int LD>
 __device__ __forceinline__ void jk_quartet_update(const double* out, const PairInfo& P, const PairInfo& K, int n,
                                                   gcptr<double> D, gcptr<double> nrm, gptr<double> G,
-                                                  double deg, double half_factor, double* jab) {
+                                                  double deg, double half_factor, double* jab,
+                                                  gptr<double> Jp = nullptr, int jstride = 0) {
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   double na[NA], nb[NB], nc[NC], nd[ND];
 #pragma unroll
@@ -414,8 +417,13 @@ __device__ __forceinline__ void jk_quartet_update(const double* out, const PairI
 #pragma unroll
   for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
-    for (int id = 0; id < ND; ++id)
-      global_add(G + (size_t)(K.bfa + ic) * n + K.bfb + id, jcd[ic * ND + id] * sj * nc[ic] * nd[id]);
+    for (int id = 0; id < ND; ++id) {
+      const double v = jcd[ic * ND + id] * sj;
+      if (Jp)
+        global_add(Jp + (size_t)(ic * ND + id) * jstride, v);
+      else
+        global_add(G + (size_t)(K.bfa + ic) * n + K.bfb + id, v * nc[ic] * nd[id]);
+    }
 #pragma unroll
   for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
@@ -495,7 +503,9 @@ __global__ __launch_bounds__(256) void jk_kernel(JKArgs a) {
                                          P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
     const double deg = (P.sa != P.sb ? 2.0 : 1.0) * (K.sa != K.sb ? 2.0 : 1.0) *
                        ((a.same_class && j == t.bra) ? 1.0 : 2.0);
-    jk_quartet_update<LA, LB, LC, LD>(out, P, K, n, D, nrm, G, deg, M.half_factor, jab);
+    jk_quartet_update<LA, LB, LC, LD>(out, P, K, n, D, nrm, G, deg, M.half_factor, jab,
+                                      (gptr<double>)M.Jp + M.jpoff[a.cket] + j,
+                                      M.off[a.cket + 1] - M.off[a.cket]);
 #pragma unroll
     for (int k = 0; k < NA * NB; ++k) jab[k] *= deg;
   }
@@ -579,7 +589,9 @@ __host__ __device__ constexpr bool strip_lds_boys32(int lds_n, int block, int an
 // in row b), so those are accumulated with LDS atomics in two row strips
 // (NA + NB) x n held for the whole ket stream and flushed to HBM once, with
 // one global atomic per touched element.  J_cd, distinct for every ket, is
-// the only per-quartet global atomic.  The bra's primitive-pair records
+// the only per-quartet global atomic; it goes to the packed Jp, where the
+// lanes of a wavefront, which take neighbouring kets, add neighbouring
+// doubles.  The bra's primitive-pair records
 // (at most kMaxStripPrims, guaranteed by the host; FP64, and in mixed mode
 // also the FP32 copies) are staged in LDS once: every lane reads the same
 // record, an LDS broadcast.
@@ -601,6 +613,10 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
   const gptr<double> G = (gptr<double>)M.Graw;
   const PairInfo P = load_pair(pairs + M.off[a.cbra] + t.bra);
   const int n = M.n, ns = M.nshell;
+  // packed density and J blocks of the ket class
+  const int npk = M.off[a.cket + 1] - M.off[a.cket];
+  const gcptr<double> Dp = (gcptr<double>)M.Dp + M.jpoff[a.cket];
+  const gptr<double> Jp = (gptr<double>)M.Jp + M.jpoff[a.cket];
   double* sa = strip;
   double* sb = strip + NA * n;
   for (int k = tid; k < (NA + NB) * n; k += blockDim.x) strip[k] = 0.0;
@@ -716,9 +732,7 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
     for (int i = 0; i < ND; ++i) nd[i] = nrm[K.bfb + i];
     double dcd[NC * ND], dac[NA * NC], dbd[NB * ND], dad[NA * ND], dbc[NB * NC];
 #pragma unroll
-    for (int i = 0; i < NC; ++i)
-#pragma unroll
-      for (int k = 0; k < ND; ++k) dcd[i * ND + k] = D[(size_t)(K.bfa + i) * n + K.bfb + k] * nc[i] * nd[k];
+    for (int k = 0; k < NC * ND; ++k) dcd[k] = Dp[(size_t)k * npk + j];
 #pragma unroll
     for (int i = 0; i < NA; ++i)
 #pragma unroll
@@ -763,10 +777,7 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
             kbc[ib * NC + ic] += dad[ia * ND + id] * v;
           }
 #pragma unroll
-    for (int ic = 0; ic < NC; ++ic)
-#pragma unroll
-      for (int id = 0; id < ND; ++id)
-        global_add(G + (size_t)(K.bfa + ic) * n + K.bfb + id, jcd[ic * ND + id] * nc[ic] * nd[id]);
+    for (int k = 0; k < NC * ND; ++k) global_add(Jp + (size_t)k * npk + j, jcd[k]);
 #pragma unroll
     for (int ia = 0; ia < NA; ++ia) {
 #pragma unroll

@@ -177,6 +177,8 @@ struct PairSet {
   DevBuf<PairInfo> d_pairs;
   DevBuf<double> d_prims;
   DevBuf<float> d_primsf;           // the same records in FP32
+  DevBuf<int> d_pidx;               // nshell x nshell: pair of (sa, sb), -1 if none
+  int jpoff[kNumPairClasses + 1] = {0};   // MolDesc::jpoff
   bool q_ready = false;
 };
 
@@ -205,6 +207,7 @@ struct Species {
   std::vector<ShellInfo> shells;
   std::vector<double> pexp, pcoef;  // exponents; raw coefficient * N(alpha, l)
   std::vector<double> norma;
+  std::vector<int> fsh;             // shell of each function
   std::vector<std::array<double, 4>> particles;  // z, x, y, z
   int nbasis = 0;
   uint64_t generation = 0;          // bumps whenever a shell is added
@@ -215,6 +218,7 @@ struct Species {
   uint64_t dev_generation = ~0ull;
   DevBuf<ShellInfo> d_shells;
   DevBuf<double> d_pexp, d_pcoef, d_norma;
+  DevBuf<int> d_fsh;
 
   PairSet sig;        // significant pairs (intra builds), with Q
   PairSet all;        // every s1 <= s2 pair (coupling builds)
@@ -253,14 +257,14 @@ struct BuildPlan {
   bool valid = false;
   TaskSet ts;
   std::vector<size_t> off, shoff;       // packed n^2 / nshell^2 offsets; last = total
+  std::vector<size_t> jpo;              // packed pair-block (Dp, Jp) offsets; last = total
   int nmax = 0, nshmax = 0;
-  bool any_dn = false;                  // some molecule screens or runs mixed
   bool any_mixed = false;               // some molecule runs mixed precision
   std::vector<MolDesc> desc, desc_dev;  // wanted / on the device
   std::vector<SymDesc> sym, sym_dev;
   DevBuf<MolDesc> d_desc;
   DevBuf<SymDesc> d_sym;
-  DevBuf<double> d_Graw, d_Dn;
+  DevBuf<double> d_Graw, d_Dn, d_Dp, d_Jp;
   DevBuf<unsigned long long> d_cnt;
   DevBuf<unsigned int> d_task_counts;
   DevBuf<int> d_ranges;                 // per class launch: first task, task count
@@ -282,7 +286,6 @@ struct BuildPlan {
   hipGraphExec_t graph = nullptr;
   uint64_t graph_layout = ~0ull;
   hipStream_t graph_stream = nullptr;
-  bool graph_any_dn = false;
   bool graph_any_mixed = false;
   double graph_eps = 0.0;
 
@@ -318,6 +321,7 @@ static void ensure_device_basis(Species& s, hipStream_t st) {
   s.d_pexp.upload(s.pexp.data(), s.pexp.size(), st);
   s.d_pcoef.upload(s.pcoef.data(), s.pcoef.size(), st);
   s.d_norma.upload(s.norma.data(), s.norma.size(), st);
+  s.d_fsh.upload(s.fsh.data(), s.fsh.size(), st);
   s.dev_generation = s.generation;
 }
 
@@ -418,7 +422,9 @@ static uint64_t morton_key(const double* P, const double* lo) {
 //     (descending), so that the FP32 (small-bound) quartets form contiguous
 //     runs of kets, then along the Z-order curve within a decade.
 // Rewrites the primitive-pair records in that order.
-static void resort_by_q(PairSet& ps, hipStream_t st, bool by_q) {
+// Also lays out the packed density and J blocks of the pairs and the map from
+// shells to pairs (of this order).
+static void resort_by_q(PairSet& ps, int nshell, hipStream_t st, bool by_q) {
   std::vector<size_t> idx(ps.pairs.size());
   for (size_t k = 0; k < idx.size(); ++k) idx[k] = k;
   double lo[3] = {1e300, 1e300, 1e300};
@@ -458,6 +464,11 @@ static void resort_by_q(PairSet& ps, hipStream_t st, bool by_q) {
   ps.d_prims.upload(ps.prims.data(), ps.prims.size(), st);
   std::vector<float> pf(ps.prims.begin(), ps.prims.end());
   ps.d_primsf.upload(pf.data(), pf.size(), st);
+  std::vector<int> pidx((size_t)nshell * nshell, -1);
+  for (size_t k = 0; k < ps.pairs.size(); ++k) pidx[(size_t)ps.pairs[k].sa * nshell + ps.pairs[k].sb] = (int)k;
+  ps.d_pidx.upload(pidx.data(), pidx.size(), st);
+  for (int c = 0; c < kNumPairClasses; ++c)
+    ps.jpoff[c + 1] = ps.jpoff[c] + (ps.off[c + 1] - ps.off[c]) * ncart_h(kPairClassL[c][0]) * ncart_h(kPairClassL[c][1]);
   HIPCHK(hipStreamSynchronize(st));
 }
 
@@ -540,7 +551,7 @@ static void ensure_sig(Species& s, hipStream_t st) {
   if (!s.sig.valid) {
     build_pairset(s, s.pairlist, s.sig, st);
     compute_schwarz(s.sig, s.d_norma.p, st);
-    resort_by_q(s.sig, st, s.mixed != 0);
+    resort_by_q(s.sig, (int)s.shells.size(), st, s.mixed != 0);
     s.sig_mixed = s.mixed;
     s.sig_gen++;
   }
@@ -559,13 +570,14 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
   const int nm = (int)p.mols.size();
   p.off.assign(nm + 1, 0);
   p.shoff.assign(nm + 1, 0);
+  p.jpo.assign(nm + 1, 0);
   p.nmax = p.nshmax = 0;
-  p.any_dn = false;
   for (int m = 0; m < nm; ++m) {
     const Species& s = *p.mols[m];
     const int ns = (int)s.shells.size();
     p.off[m + 1] = p.off[m] + (size_t)s.nbasis * s.nbasis;
     p.shoff[m + 1] = p.shoff[m] + (size_t)ns * ns;
+    p.jpo[m + 1] = p.jpo[m] + (size_t)s.sig.jpoff[kNumPairClasses];
     p.nmax = std::max(p.nmax, s.nbasis);
     p.nshmax = std::max(p.nshmax, ns);
   }
@@ -737,6 +749,8 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
   p.d_task_counts.ensure(3 * std::max<size_t>(ts.tasks.size(), 1));
   p.d_Graw.ensure(std::max<size_t>(p.off[nm], 1));
   p.d_Dn.ensure(std::max<size_t>(p.shoff[nm], 1));
+  p.d_Dp.ensure(std::max<size_t>(p.jpo[nm], 1));
+  p.d_Jp.ensure(std::max<size_t>(p.jpo[nm], 1));
   p.d_desc.ensure(std::max(nm, 1));
   p.d_sym.ensure(std::max(nm, 1));
   p.desc_dev.clear();
@@ -931,19 +945,37 @@ static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, int which,
   if (join && fork) join_side_streams(st);
 }
 
-// Dnorm and zeroed G_raw (no memset: capturable).
+// Dnorm, packed densities and zeroed accumulators (no memset: capturable).
 static void enqueue_prologue(BuildPlan& p, hipStream_t st) {
-  const int nm = (int)p.mols.size();
-  if (p.any_dn) launch_dnorm_batch(p.d_desc.p, nm, p.nshmax, st);
-  launch_fill_zero(p.d_Graw.p, p.off[nm], st);
+  launch_prologue_batch(p.d_desc.p, (int)p.mols.size(), p.nmax, st);
 }
 
-// Per-launch counters and G = 0.25 (G_raw + G_raw^T).
+// G = 0.25 (G_raw + G_raw^T).
 static void enqueue_epilogue(BuildPlan& p, hipStream_t st) {
-  const int nm = (int)p.mols.size();
-  launch_reduce_counts_multi(p.d_task_counts.p, p.d_ranges.p, (int)p.ts.launches.size(), p.d_cnt.p, st);
-  launch_symmetrize_batch(p.d_sym.p, nm, p.nmax, st);
+  launch_symmetrize_batch(p.d_desc.p, p.d_sym.p, (int)p.mols.size(), p.nmax, st);
   HIPCHK(hipGetLastError());
+}
+
+// The descriptor fields a species itself determines.
+static void fill_desc(MolDesc& M, const Species& s, double factor) {
+  std::memset(&M, 0, sizeof(M));
+  M.pairs = s.sig.d_pairs.p;
+  M.prim = s.sig.d_prims.p;
+  M.primf = s.sig.d_primsf.p;
+  M.shells = s.d_shells.p;
+  M.norma = s.d_norma.p;
+  M.pidx = s.sig.d_pidx.p;
+  M.fsh = s.d_fsh.p;
+  for (int k = 0; k <= kNumPairClasses; ++k) {
+    M.off[k] = s.sig.off[k];
+    M.jpoff[k] = s.sig.jpoff[k];
+  }
+  M.n = s.nbasis;
+  M.nshell = (int)s.shells.size();
+  M.screen = s.is_electron ? 1 : 0;
+  M.mixed = s.mixed;
+  M.half_factor = 0.5 * factor;
+  M.tau = s.tau;
 }
 
 // Enqueue one build of plan p on stream st: packed densities dD -> packed
@@ -958,36 +990,20 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
   const int nm = (int)p.mols.size();
   p.desc.resize(nm);
   p.sym.resize(nm);
-  p.any_dn = false;
   p.any_mixed = false;
   p.eps = nm > 0 ? p.mols[0]->screen_eps : p.eps;
   for (int m = 1; m < nm; ++m) p.eps = std::min(p.eps, p.mols[m]->screen_eps);
   for (int m = 0; m < nm; ++m) {
     Species& s = *p.mols[m];
     MolDesc& M = p.desc[m];
-    std::memset(&M, 0, sizeof(M));
-    M.pairs = s.sig.d_pairs.p;
-    M.prim = s.sig.d_prims.p;
-    M.primf = s.sig.d_primsf.p;
+    fill_desc(M, s, factors[m]);
     M.D = dD_each ? dD_each[m] : dD + p.off[m];
     M.Dn = p.d_Dn.p + p.shoff[m];
-    M.shells = s.d_shells.p;
-    M.norma = s.d_norma.p;
     M.Graw = p.d_Graw.p + p.off[m];
-    for (int k = 0; k <= kNumPairClasses; ++k) M.off[k] = s.sig.off[k];
-    M.n = s.nbasis;
-    M.nshell = (int)s.shells.size();
-    M.screen = s.is_electron ? 1 : 0;
-    M.mixed = s.mixed;
-    M.half_factor = 0.5 * factors[m];
-    M.tau = s.tau;
-    p.any_dn = p.any_dn || M.screen || M.mixed;
+    M.Dp = p.d_Dp.p + p.jpo[m];
+    M.Jp = p.d_Jp.p + p.jpo[m];
     p.any_mixed = p.any_mixed || M.mixed;
-    SymDesc& Y = p.sym[m];
-    std::memset(&Y, 0, sizeof(Y));
-    Y.Graw = M.Graw;
-    Y.G = dG_each ? dG_each[m] : dG + p.off[m];
-    Y.n = s.nbasis;
+    p.sym[m].G = dG_each ? dG_each[m] : dG + p.off[m];
   }
   if (p.desc_dev.size() != p.desc.size() || std::memcmp(p.desc_dev.data(), p.desc.data(), nm * sizeof(MolDesc))) {
     HIPCHK(hipMemcpyAsync(p.d_desc.p, p.desc.data(), nm * sizeof(MolDesc), hipMemcpyHostToDevice, st));
@@ -1006,8 +1022,7 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
     // scratch-heavy classes stay outside it, on side stream 0: they are
     // enqueued after the prologue and before the graph launch, and joined
     // with it before the epilogue, so that they run beside the graph.
-    if (!p.graph || p.graph_layout != p.layout || p.graph_stream != st || p.graph_any_dn != p.any_dn ||
-        p.graph_any_mixed != p.any_mixed ||
+    if (!p.graph || p.graph_layout != p.layout || p.graph_stream != st || p.graph_any_mixed != p.any_mixed ||
         p.graph_eps != p.eps) {
       if (p.graph) HIPCHK(hipGraphExecDestroy(p.graph));
       p.graph = nullptr;
@@ -1026,7 +1041,6 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
       HIPCHK(e);
       p.graph_layout = p.layout;
       p.graph_stream = st;
-      p.graph_any_dn = p.any_dn;
       p.graph_any_mixed = p.any_mixed;
       p.graph_eps = p.eps;
     }
@@ -1045,18 +1059,20 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
 
 // ------------------------------------------------ build without allocation
 // lowdin_fock_compute_2body_device_noalloc keeps the scratch of a build --
-// the molecule and symmetrisation descriptors, the shell-block norms of D
-// and the raw accumulator G_raw -- in this file-scope device array instead
+// the molecule and symmetrisation descriptors, the shell-block norms of D,
+// the raw accumulator G_raw and the packed pair blocks -- in this file-scope device array instead
 // of library allocations.  Every GPU holds its own copy until the process
 // ends; calls that overlap on one GPU share it and race.
 constexpr int kNoAllocMaxN = 768;        // basis functions
 constexpr int kNoAllocMaxShells = 384;   // shells
 constexpr size_t kNoAllocDescBytes = 512;
+// doubles of the packed pair blocks: sum of NA NB over the pairs s1 >= s2
+constexpr size_t kNoAllocPairs = ((size_t)kNoAllocMaxN * kNoAllocMaxN + 6 * (size_t)kNoAllocMaxN) / 2;
 constexpr size_t kNoAllocScratchBytes =
     kNoAllocDescBytes + sizeof(double) * ((size_t)kNoAllocMaxShells * kNoAllocMaxShells +
-                                          (size_t)kNoAllocMaxN * kNoAllocMaxN);   // 5.8 MB
+                                          (size_t)kNoAllocMaxN * kNoAllocMaxN + 2 * kNoAllocPairs);   // 10.7 MB
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
-static_assert(sizeof(MolDesc) + sizeof(SymDesc) <= kNoAllocDescBytes, "descriptor slots");
+static_assert(sizeof(MolDesc) <= 256 && 256 + sizeof(SymDesc) <= kNoAllocDescBytes, "descriptor slots");
 
 // Device address of `scratch` on the current device (hipGetSymbolAddress
 // once per device; the host-side name of the array is not a device address).
@@ -1101,33 +1117,19 @@ static void enqueue_noalloc(BuildPlan& p, Species& s, const double* dD, double* 
   double* Dn = reinterpret_cast<double*>(scr + kNoAllocDescBytes);
   double* Graw = Dn + (size_t)kNoAllocMaxShells * kNoAllocMaxShells;
   MolDesc M;
-  std::memset(&M, 0, sizeof(M));
-  M.pairs = s.sig.d_pairs.p;
-  M.prim = s.sig.d_prims.p;
-  M.primf = s.sig.d_primsf.p;
+  fill_desc(M, s, factor);
   M.D = dD;
   M.Dn = Dn;
-  M.shells = s.d_shells.p;
-  M.norma = s.d_norma.p;
   M.Graw = Graw;
-  for (int k = 0; k <= kNumPairClasses; ++k) M.off[k] = s.sig.off[k];
-  M.n = s.nbasis;
-  M.nshell = (int)s.shells.size();
-  M.screen = s.is_electron ? 1 : 0;
-  M.mixed = s.mixed;
-  M.half_factor = 0.5 * factor;
-  M.tau = s.tau;
+  M.Dp = Graw + (size_t)kNoAllocMaxN * kNoAllocMaxN;
+  M.Jp = M.Dp + kNoAllocPairs;
   SymDesc Y;
-  std::memset(&Y, 0, sizeof(Y));
-  Y.Graw = Graw;
   Y.G = dG;
-  Y.n = s.nbasis;
   p.eps = s.screen_eps;
   hipLaunchKernelGGL(store_desc_kernel, dim3(1), dim3(1), 0, st, md, M, sd, Y);
-  if (M.screen || M.mixed) launch_dnorm_batch(md, 1, M.nshell, st);
-  launch_fill_zero(Graw, (size_t)M.n * M.n, st);
+  launch_prologue_batch(md, 1, M.n, st);
   enqueue_classes(p, st, false, 0, true, md, true);
-  launch_symmetrize_batch(sd, 1, M.n, st);
+  launch_symmetrize_batch(md, sd, 1, M.n, st);
   HIPCHK(hipGetLastError());
 }
 
@@ -1136,6 +1138,8 @@ static void collect_plan_stats(BuildPlan& p, hipStream_t st, double t0) {
   Context& c = ctx();
   const size_t nl = p.ts.launches.size();
   std::vector<unsigned long long> cnt(3 * std::max<size_t>(nl, 1));
+  launch_reduce_counts_multi(p.d_task_counts.p, p.d_ranges.p, (int)nl, p.d_cnt.p, st);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(cnt.data(), p.d_cnt.p, cnt.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
   float kms = 0.f;
@@ -1690,6 +1694,7 @@ void LibintInterface_add_shell(void* lint, double* alpha, double* coeff, double*
     lowdin::overlap_block(sh, sh, s->pexp.data(), s->pcoef.data(), blk);
     const int nc = lowdin::ncart_h(l);
     for (int i = 0; i < nc; ++i) s->norma.push_back(1.0 / std::sqrt(blk[i * nc + i]));
+    s->fsh.insert(s->fsh.end(), nc, (int)s->shells.size() - 1);
     s->nbasis += nc;
     s->generation++;
     s->sig.valid = false;
@@ -1980,7 +1985,7 @@ int lowdin_fock_compute_2body_device(void* lint, const double* d_dens, double* d
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c.stream;
     if (s->setup_each_build) s->sig.valid = false;
     lowdin::BuildPlan& p = lowdin::own_plan(*s);
-    lowdin::enqueue_plan(p, d_dens, d_result, &factor, st);
+    lowdin::enqueue_plan(p, d_dens, d_result, &factor, st, nullptr, nullptr, synchronize != 0);
     if (synchronize) {
       lowdin::collect_plan_stats(p, st, t0);
       s->stats = p.stats;
@@ -2200,7 +2205,7 @@ int lowdin_fock_batch_compute_2body_device(void* batch, const double* d_dens, do
     const double t0 = lowdin::now_ms();
     lowdin::ensure_context();
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c.stream;
-    lowdin::enqueue_plan(p, d_dens, d_result, factors, st);
+    lowdin::enqueue_plan(p, d_dens, d_result, factors, st, nullptr, nullptr, synchronize != 0);
     if (synchronize) lowdin::collect_plan_stats(p, st, t0);
     lowdin::g_last_error.clear();
     return 0;
@@ -2220,7 +2225,7 @@ int lowdin_fock_batch_compute_2body_device_ptrs(void* batch, const double* const
     const double t0 = lowdin::now_ms();
     lowdin::ensure_context();
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c.stream;
-    lowdin::enqueue_plan(p, nullptr, nullptr, factors, st, d_dens, d_result);
+    lowdin::enqueue_plan(p, nullptr, nullptr, factors, st, d_dens, d_result, synchronize != 0);
     if (synchronize) lowdin::collect_plan_stats(p, st, t0);
     lowdin::g_last_error.clear();
     return 0;

@@ -218,29 +218,60 @@ __global__ void symmetrize_kernel(const double* Graw, int n, double scale, doubl
   G[(size_t)i * n + k] = scale * 0.25 * (Graw[(size_t)i * n + k] + Graw[(size_t)k * n + i]);
 }
 
-// Sum the per-task (quartets, primitive quartets, FP32 quartets) triples of
-// one launch.
-// Dnorm of every molecule of a batch: blockIdx.y is the molecule.
-__global__ void dnorm_batch_kernel(const MolDesc* mols) {
+// What a build needs before its class launches, for every molecule of a batch
+// (blockIdx.y): G_raw and Jp cleared, the normalised density blocks of the
+// pairs packed into Dp, and (where the build screens or runs mixed precision)
+// the shell-block norms of D.  One launch: each part is far shorter than a
+// launch, so a small build pays for launches alone.
+__global__ void prologue_batch_kernel(const MolDesc* mols) {
   const MolDesc& M = mols[blockIdx.y];
-  const int nsh = M.nshell;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= nsh * nsh) return;
-  const int s1 = idx / nsh, s2 = idx % nsh;
-  const ShellInfo A = M.shells[s1], B = M.shells[s2];
-  const int n = M.n;
-  double m = 0.0;
-  for (int i = 0; i < ncart_(A.l); ++i)
-    for (int k = 0; k < ncart_(B.l); ++k) m = fmax(m, fabs(M.D[(size_t)(A.bf + i) * n + B.bf + k]));
-  M.Dn[idx] = m;
+  const int nsh = M.nshell, n = M.n, npairs = M.off[6], njp = M.jpoff[6];
+  const int first = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+  double* G = M.Graw;
+  double* Jp = M.Jp;
+  for (int k = first; k < n * n; k += stride) G[k] = 0.0;
+  for (int k = first; k < njp; k += stride) Jp[k] = 0.0;
+  for (int k = first; k < npairs; k += stride) {
+    const PairInfo* P = M.pairs + k;
+    const int la = P->la, lb = P->lb, c = la * (la + 1) / 2 + lb;
+    const int na = ncart_(la), nb = ncart_(lb), ncls = M.off[c + 1] - M.off[c];
+    const int bfa = P->bfa, bfb = P->bfb;
+    double* out = M.Dp + M.jpoff[c] + (k - M.off[c]);
+    for (int i = 0; i < na; ++i)
+      for (int j = 0; j < nb; ++j)
+        out[(size_t)(i * nb + j) * ncls] =
+            M.D[(size_t)(bfa + i) * n + bfb + j] * M.norma[bfa + i] * M.norma[bfb + j];
+  }
+  if (!(M.screen || M.mixed)) return;
+  for (int k = first; k < nsh * nsh; k += stride) {
+    const ShellInfo A = M.shells[k / nsh], B = M.shells[k % nsh];
+    double m = 0.0;
+    for (int i = 0; i < ncart_(A.l); ++i)
+      for (int j = 0; j < ncart_(B.l); ++j) m = fmax(m, fabs(M.D[(size_t)(A.bf + i) * n + B.bf + j]));
+    M.Dn[k] = m;
+  }
 }
 
-// G = 0.25 (Graw + Graw^T) of every molecule of a batch (blockIdx.z).
-__global__ void symmetrize_batch_kernel(const SymDesc* d) {
-  const SymDesc S = d[blockIdx.z];
-  const int i = blockIdx.y * blockDim.y + threadIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= S.n || j >= S.n) return;
-  S.G[(size_t)i * S.n + j] = 0.25 * (S.Graw[(size_t)i * S.n + j] + S.Graw[(size_t)j * S.n + i]);
+// J element (i, k) of the pair (shell of i, shell of k) if that orientation
+// is the pair's, else 0.
+__device__ inline double packed_j(const MolDesc& M, int i, int k) {
+  const int si = M.fsh[i], sk = M.fsh[k], q = M.pidx[si * M.nshell + sk];
+  if (q < 0) return 0.0;
+  const PairInfo* P = M.pairs + q;
+  const int c = P->la * (P->la + 1) / 2 + P->lb, ncls = M.off[c + 1] - M.off[c];
+  const int e = (i - P->bfa) * ncart_(P->lb) + (k - P->bfb);
+  return M.Jp[M.jpoff[c] + (size_t)e * ncls + (q - M.off[c])];
+}
+
+// G = 0.25 (Graw + Graw^T) of every molecule of a batch (blockIdx.z), G_raw
+// completed by the packed J_cd.
+__global__ void symmetrize_batch_kernel(const MolDesc* mols, const SymDesc* d) {
+  const MolDesc& M = mols[blockIdx.z];
+  const int i = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.x * blockDim.x + threadIdx.x;
+  const int n = M.n;
+  if (i >= n || k >= n) return;
+  const double J = (packed_j(M, i, k) + packed_j(M, k, i)) * (M.norma[i] * M.norma[k]);
+  d[blockIdx.z].G[(size_t)i * n + k] = 0.25 * (M.Graw[(size_t)i * n + k] + M.Graw[(size_t)k * n + i] + J);
 }
 
 // Vector-store fill; used instead of hipMemsetAsync so that a build can be
@@ -356,43 +387,11 @@ __global__ __launch_bounds__(1024) void reduce_counts_multi_kernel(const unsigne
   }
 }
 
-__global__ __launch_bounds__(1024) void reduce_counts_kernel(const unsigned int* counts, int ntasks,
-                                                             unsigned long long* out) {
-  __shared__ unsigned long long sq[1024], sp[1024], s3[1024];
-  unsigned long long q = 0, p = 0, q3 = 0;
-  for (int i = threadIdx.x; i < ntasks; i += blockDim.x) {
-    q += counts[3 * i];
-    p += counts[3 * i + 1];
-    q3 += counts[3 * i + 2];
-  }
-  sq[threadIdx.x] = q;
-  sp[threadIdx.x] = p;
-  s3[threadIdx.x] = q3;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      sq[threadIdx.x] += sq[threadIdx.x + w];
-      sp[threadIdx.x] += sp[threadIdx.x + w];
-      s3[threadIdx.x] += s3[threadIdx.x + w];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    out[0] = sq[0];
-    out[1] = sp[0];
-    out[2] = s3[0];
-  }
-}
-
 // ------------------------------------------------------------ launchers
 void launch_reduce_counts_multi(const unsigned int* counts, const int* ranges, int nlaunch, unsigned long long* out,
                                 hipStream_t s) {
   if (nlaunch > 0)
     hipLaunchKernelGGL(reduce_counts_multi_kernel, dim3(nlaunch), dim3(1024), 0, s, counts, ranges, out);
-}
-
-void launch_reduce_counts(const unsigned int* counts, int ntasks, unsigned long long* out, hipStream_t s) {
-  hipLaunchKernelGGL(reduce_counts_kernel, dim3(1), dim3(1024), 0, s, counts, ntasks, out);
 }
 
 void launch_pair_norms(const ShellInfo* sh, const double* pexp, const double* pcoef, int nsh, double* norms,
@@ -424,16 +423,16 @@ void launch_symmetrize(const double* Graw, int n, double scale, double* G, hipSt
   hipLaunchKernelGGL(symmetrize_kernel, grd, blk, 0, s, Graw, n, scale, G);
 }
 
-void launch_dnorm_batch(const MolDesc* mols, int nmol, int nshmax, hipStream_t s) {
-  if (nmol <= 0 || nshmax <= 0) return;
-  const int tot = nshmax * nshmax;
-  hipLaunchKernelGGL(dnorm_batch_kernel, dim3((tot + 255) / 256, nmol), dim3(256), 0, s, mols);
+void launch_prologue_batch(const MolDesc* mols, int nmol, int nmax, hipStream_t s) {
+  if (nmol <= 0 || nmax <= 0) return;
+  const int blocks = std::min((nmax * nmax + 255) / 256, 1024);
+  hipLaunchKernelGGL(prologue_batch_kernel, dim3(blocks, nmol), dim3(256), 0, s, mols);
 }
 
-void launch_symmetrize_batch(const SymDesc* d, int nmol, int nmax, hipStream_t s) {
+void launch_symmetrize_batch(const MolDesc* mols, const SymDesc* d, int nmol, int nmax, hipStream_t s) {
   if (nmol <= 0 || nmax <= 0) return;
   const dim3 blk(32, 8), grd((nmax + 31) / 32, (nmax + 7) / 8, nmol);
-  hipLaunchKernelGGL(symmetrize_batch_kernel, grd, blk, 0, s, d);
+  hipLaunchKernelGGL(symmetrize_batch_kernel, grd, blk, 0, s, mols, d);
 }
 
 void launch_fill_zero(double* p, size_t count, hipStream_t s) {
