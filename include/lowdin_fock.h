@@ -323,6 +323,8 @@ int lowdin_fock_batch_launch_profile(void* batch, int cap, int* classes, float* 
  * {2048, 8192, 32768}), by timing `reps` serialised builds per candidate on
  * the given inputs.  Classes of total angular momentum >= 6 run only the
  * wave-cooperative kernel (the per-lane kernels would spill to scratch).
+ * Small FP64 builds (up to about 4e6 candidate quartets) run as one launch over
+ * all classes whatever the choices.
  * Results are unchanged by the choice up to FP64 summation order. */
 int lowdin_fock_batch_autotune(void* batch, const double* d_dens, double* d_result, const double* factors,
                                void* stream, int reps);

@@ -31,6 +31,9 @@ namespace lowdin {
 template <int LA, int LB, int LC, int LD>
 struct CoopProgram;
 
+// Total angular momentum from which a class runs only these kernels.
+constexpr int kCoopL = 6;
+
 // Fixed slots of a wavefront's LDS region (doubles).
 constexpr int kCoopZero = 18;   // 18 and 19: always 0.0 (m and m+1 operands of absent terms)
 constexpr int kCoopAcc = 22;    // first contracted accumulator (20: target of idle lanes)
@@ -239,8 +242,11 @@ __device__ __forceinline__ void coop_quartet(double* R, const uint2* pg, gcptr<d
   }
 }
 
+// lds: the row strips, then one region per wavefront; wg: the workgroup's
+// counters; counts: the task's (null: none kept).
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
+__device__ __forceinline__ void jk_coop_body(const JKArgs& a, const Task& t, unsigned int* counts, double* lds,
+                                             unsigned int* wg) {
   using Pg = CoopProgram<LA, LB, LC, LD>;
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   constexpr int NAB = NA * NB, NCD = NC * ND;
@@ -248,12 +254,9 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
   constexpr int oDab = Pg::kRegion, oDcd = oDab + NAB, oDac = oDcd + NCD, oDbd = oDac + NA * NC,
                 oDad = oDbd + NB * ND, oDbc = oDad + NA * ND;
   static_assert(NAB <= 64, "one J_ab element per lane");
-  extern __shared__ double lds[];
-  __shared__ unsigned int wg_q, wg_p;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nw = blockDim.x >> 6;
-  const Task t = a.tasks[blockIdx.x];
   const MolDesc& M = a.mols[t.flags];
   const gcptr<PairInfo> pairs = (gcptr<PairInfo>)M.pairs;
   const gcptr<double> prim = (gcptr<double>)M.prim;
@@ -271,8 +274,8 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
   double* R = lds + (NA + NB) * sn + w * kWave;
   for (int k = tid; k < (NA + NB) * sn; k += blockDim.x) lds[k] = 0.0;
   if (tid == 0) {
-    wg_q = 0;
-    wg_p = 0;
+    wg[0] = 0;
+    wg[1] = 0;
   }
   if (lane < 2) R[kCoopZero + lane] = 0.0;
   // normalised bra density block; lane k < NAB owns J_ab element k
@@ -382,9 +385,9 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
     if (sn) atomicAdd(&sa[ia * sn + P.bfb + ib], v);
     else global_add(G + (size_t)(P.bfa + ia) * n + P.bfb + ib, v * nrm[P.bfa + ia]);
   }
-  if (a.counts && lane == 0) {
-    atomicAdd(&wg_q, myq);
-    atomicAdd(&wg_p, myp);
+  if (counts && lane == 0) {
+    atomicAdd(&wg[0], myq);
+    atomicAdd(&wg[1], myp);
   }
   __syncthreads();
   if (sn) {
@@ -403,11 +406,18 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
       }
     }
   }
-  if (a.counts && tid == 0) {
-    a.counts[3 * blockIdx.x] = wg_q;
-    a.counts[3 * blockIdx.x + 1] = wg_p;
-    a.counts[3 * blockIdx.x + 2] = 0;
+  if (counts && tid == 0) {
+    counts[0] = wg[0];
+    counts[1] = wg[1];
+    counts[2] = 0;
   }
+}
+
+template <int LA, int LB, int LC, int LD>
+__global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
+  extern __shared__ double lds[];
+  __shared__ unsigned int wg[2];
+  jk_coop_body<LA, LB, LC, LD>(a, a.tasks[blockIdx.x], a.counts ? a.counts + 3 * blockIdx.x : nullptr, lds, wg);
 }
 
 // Inter-species Coulomb coupling (Libint2Iface.cpp:1111-1294) of one class

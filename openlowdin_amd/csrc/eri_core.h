@@ -595,16 +595,16 @@ __host__ __device__ constexpr bool strip_lds_boys32(int lds_n, int block, int an
 // (at most kMaxStripPrims, guaranteed by the host; FP64, and in mixed mode
 // also the FP32 copies) are staged in LDS once: every lane reads the same
 // record, an LDS broadcast.
-template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_strip_kernel(JKArgs a) {
+// strip: rows of a (NA x n), then rows of b (NB x n), then the Boys columns;
+// bpd / bpf: the bra's FP64 and FP32 primitive-pair records; wg: the
+// workgroup's three counters; counts: the task's (null: none kept).  kF32:
+// with the FP32 quartets of mixed precision; kTab: with the Boys columns in
+// LDS where strip_lds_boys says so.
+template <int LA, int LB, int LC, int LD, bool kF32, bool kTab>
+__device__ __forceinline__ void jk_strip_body(const JKArgs& a, const Task& t, unsigned int* counts, double* strip,
+                                              double* bpd, float* bpf, unsigned int* wg) {
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-  constexpr bool kF32 = Fp32Allowed<LA, LB, LC, LD>::value;
-  extern __shared__ double strip[];  // rows of a (NA x n), then rows of b (NB x n)
-  __shared__ double bpd[kMaxStripPrims * kPrimPairStride];
-  __shared__ float bpf[kF32 ? kMaxStripPrims * kPrimPairStride : 1];   // FP32 bra records (mixed)
-  __shared__ unsigned int wg_q, wg_p, wg_q32;
   const int tid = threadIdx.x;
-  const Task t = a.tasks[blockIdx.x];
   const MolDesc& M = a.mols[t.flags];
   const gcptr<PairInfo> pairs = (gcptr<PairInfo>)M.pairs;
   const gcptr<double> prim = (gcptr<double>)M.prim;
@@ -620,11 +620,11 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
   double* sa = strip;
   double* sb = strip + NA * n;
   for (int k = tid; k < (NA + NB) * n; k += blockDim.x) strip[k] = 0.0;
-  const bool ldsb = strip_lds_boys<LA, LB, LC, LD>(a.lds_n, a.block);
+  const bool ldsb = kTab && strip_lds_boys<LA, LB, LC, LD>(a.lds_n, a.block);
   double* btab = strip + (NA + NB) * a.lds_n;
-  const bool ldsb32 = kF32 && strip_lds_boys32<LA, LB, LC, LD>(a.lds_n, a.block, a.any_mixed);
+  const bool ldsb32 = kF32 && kTab && strip_lds_boys32<LA, LB, LC, LD>(a.lds_n, a.block, a.any_mixed);
   float* btab32 = reinterpret_cast<float*>(btab + kBoysRows * kLdsBoysCols);
-  if constexpr (StripLdsBoys<LA, LB, LC, LD>::value) {
+  if constexpr (kTab) {
     constexpr int L = LA + LB + LC + LD;
     if (ldsb) {
       for (int k = tid; k < kBoysRows * kLdsBoysCols; k += blockDim.x) {
@@ -650,9 +650,9 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
     }
   }
   if (tid == 0) {
-    wg_q = 0;
-    wg_p = 0;
-    wg_q32 = 0;
+    wg[0] = 0;
+    wg[1] = 0;
+    wg[2] = 0;
   }
   __syncthreads();
   double na[NA], nb[NB];
@@ -690,7 +690,7 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
     if constexpr (kF32) {
       if (lo) {
         bool done = false;
-        if constexpr (StripLdsBoys<LA, LB, LC, LD>::value) {
+        if constexpr (kTab) {
           if (ldsb32) {
             contracted_quartet_f32_body<LA, LB, LC, LD, kLdsBoys32Cols, 1>(
                 (const float*)bpf, P.nprim, (gcptr<float>)M.primf + (size_t)K.poff * kPrimPairStride, K.nprim,
@@ -706,7 +706,7 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
     }
     if (!lo) {
       bool done = false;
-      if constexpr (StripLdsBoys<LA, LB, LC, LD>::value) {
+      if constexpr (kTab) {
         if (ldsb) {
           contracted_quartet_body<LA, LB, LC, LD, kLdsBoysCols, 1>((const double*)bpd, P.nprim,
                                                                    prim + (size_t)K.poff * kPrimPairStride,
@@ -799,10 +799,10 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
 #pragma unroll
     for (int ib = 0; ib < NB; ++ib)
       if (jab[ia * NB + ib] != 0.0) atomicAdd(&sa[ia * n + P.bfb + ib], jab[ia * NB + ib] * nb[ib]);
-  if (a.counts) {
-    atomicAdd(&wg_q, myq);
-    atomicAdd(&wg_p, myp);
-    atomicAdd(&wg_q32, myq32);
+  if (counts) {
+    atomicAdd(&wg[0], myq);
+    atomicAdd(&wg[1], myp);
+    atomicAdd(&wg[2], myq32);
   }
   __syncthreads();
   // flush: one global atomic per touched strip element (row norma applied here)
@@ -816,11 +816,22 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
       const double v = sb[r * n + c];
       if (v != 0.0) global_add(G + (size_t)(P.bfb + r) * n + c, v * nb[r]);
     }
-  if (a.counts && tid == 0) {
-    a.counts[3 * blockIdx.x] = wg_q;
-    a.counts[3 * blockIdx.x + 1] = wg_p;
-    a.counts[3 * blockIdx.x + 2] = wg_q32;
+  if (counts && tid == 0) {
+    counts[0] = wg[0];
+    counts[1] = wg[1];
+    counts[2] = wg[2];
   }
+}
+
+template <int LA, int LB, int LC, int LD>
+__global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_strip_kernel(JKArgs a) {
+  constexpr bool kF32 = Fp32Allowed<LA, LB, LC, LD>::value;
+  extern __shared__ double strip[];
+  __shared__ double bpd[kMaxStripPrims * kPrimPairStride];
+  __shared__ float bpf[kF32 ? kMaxStripPrims * kPrimPairStride : 1];
+  __shared__ unsigned int wg[3];
+  jk_strip_body<LA, LB, LC, LD, kF32, StripLdsBoys<LA, LB, LC, LD>::value>(
+      a, a.tasks[blockIdx.x], a.counts ? a.counts + 3 * blockIdx.x : nullptr, strip, bpd, bpf, wg);
 }
 
 // ------------------------------------------------------- coupling kernel

@@ -4,7 +4,8 @@ For every canonical quartet class (la lb|lc ld) with l <= LMAX, la >= lb,
 lc >= ld and pair class (la, lb) >= (lc, ld), this emits two device
 functions into ``gen/eri_<class>.inc`` (plus the Gaussian-geminal VRR
 ``g12vrr_<class>``, see G12Gen), three kernel translation units per class
-(``gen/k_<class>.hip``: Fock build, coupling and Schwarz kernels;
+(``gen/k_<class>.hip``: Fock build, coupling and Schwarz kernels, and
+``gen/k_fused.hip``: all classes of a small Fock build in one kernel;
 ``gen/s_<class>.hip``: integral store and first-quarter transform;
 ``gen/g_<class>.hip``: G12 Fock build and coupling), so that they compile in
 parallel, and the launch dispatch table ``gen/dispatch.h``:
@@ -712,6 +713,38 @@ void launch_gcp_%(k)s(const G12CouplingArgs& args, hipStream_t s) { launch_g12cp
 """
 
 
+FUSED_TU = """// Generated by gen_eri.py -- do not edit.
+// The J/K work of every quartet class as one launch (small builds).
+#include "../eri_fused.h"
+
+namespace lowdin {
+%(incs)s
+__global__ __launch_bounds__(64) void jk_fused_kernel(FusedArgs f) {
+  extern __shared__ double lds[];
+  __shared__ double bpd[kMaxStripPrims * kPrimPairStride];
+  __shared__ unsigned int wg[3];
+  const int b = blockIdx.x;
+  int seg = 0;
+  while (seg + 1 < f.nseg && b >= f.first[seg + 1]) ++seg;
+  const Task t = f.tasks[b];
+  unsigned int* counts = f.counts ? f.counts + 3 * (size_t)b : nullptr;
+  switch (f.cls[seg]) {
+%(cases)s  }
+}
+
+size_t jk_fused_lds(int nmax) {
+  int d = 0;
+%(sizes)s  return (size_t)d * sizeof(double);
+}
+
+void launch_jk_fused(const FusedArgs& f, hipStream_t s) {
+  if (f.nseg <= 0 || f.first[f.nseg] <= 0) return;
+  hipLaunchKernelGGL(jk_fused_kernel, dim3(f.first[f.nseg]), dim3(64), jk_fused_lds(f.lds_n), s, f);
+}
+}  // namespace lowdin
+"""
+
+
 def main(outdir):
     pcs, classes = canonical_classes()
     gdir = os.path.join(outdir, "gen")
@@ -755,6 +788,17 @@ def main(outdir):
         with open(os.path.join(gdir, "s_%s.hip" % k), "w") as fh:
             fh.write(STORE_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k})
         table[k] = {"L": L, "nacc": nacc, "vrr_flops": v.flops, "hrr_flops": h.flops}
+    incs, cases, sizes = [], [], []
+    for cl in classes:
+        k = "%d%d%d%d" % cl
+        incs.append('#include "eri_%s.inc"\nLOWDIN_ERI_CLASS(%d, %d, %d, %d)' % ((k,) + cl))
+        if sum(cl) >= COOP_MIN_L:
+            incs.append('#include "c_%s.inc"' % k)
+        cases.append("    case %d: fused_class<%d, %d, %d, %d>(f, seg, t, counts, lds, bpd, wg); break;\n"
+                     % ((int(k),) + cl))
+        sizes.append("  d = std::max(d, fused_doubles<%d, %d, %d, %d>(nmax));\n" % cl)
+    with open(os.path.join(gdir, "k_fused.hip"), "w") as fh:
+        fh.write(FUSED_TU % {"incs": "\n".join(incs), "cases": "".join(cases), "sizes": "".join(sizes)})
     with open(os.path.join(outdir, "ops_table.json"), "w") as fh:
         json.dump({"note": "floating-point operations of the generated Obara-Saika VRR (per primitive "
                            "quartet, excluding Boys) and HGP HRR (per contracted quartet)",

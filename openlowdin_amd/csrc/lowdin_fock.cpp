@@ -179,6 +179,7 @@ struct PairSet {
   DevBuf<float> d_primsf;           // the same records in FP32
   DevBuf<int> d_pidx;               // nshell x nshell: pair of (sa, sb), -1 if none
   int jpoff[kNumPairClasses + 1] = {0};   // MolDesc::jpoff
+  int maxprim = 0;                  // most primitive pairs of a pair
   bool q_ready = false;
 };
 
@@ -280,6 +281,7 @@ struct BuildPlan {
   std::vector<hipEvent_t> launch_ev;
   bool time_launches = false;
   bool serialize = false;               // all class launches on one side stream (clean per-class timing)
+  bool fused = false;                   // the tasks are those of one launch over all classes (jk_fused_kernel)
   bool inline_launch = false;           // class launches on the caller's stream (no side streams)
   bool use_graph = false;
   double eps = 2.220446049250313080847e-16;   // quartet screen threshold of the plan's launches
@@ -465,6 +467,8 @@ static void resort_by_q(PairSet& ps, int nshell, hipStream_t st, bool by_q) {
   std::vector<float> pf(ps.prims.begin(), ps.prims.end());
   ps.d_primsf.upload(pf.data(), pf.size(), st);
   std::vector<int> pidx((size_t)nshell * nshell, -1);
+  ps.maxprim = 0;
+  for (const PairInfo& P : ps.pairs) ps.maxprim = std::max(ps.maxprim, P.nprim);
   for (size_t k = 0; k < ps.pairs.size(); ++k) pidx[(size_t)ps.pairs[k].sa * nshell + ps.pairs[k].sb] = (int)k;
   ps.d_pidx.upload(pidx.data(), pidx.size(), st);
   for (int c = 0; c < kNumPairClasses; ++c)
@@ -544,6 +548,16 @@ constexpr double kQuartetIters = 12.0;
 constexpr double kSplitMin = 16.0, kSplitMax = 64.0;
 constexpr double kSplitKets = 32.0;   // kets per bra for each unit of lmax
 
+// A plan runs as one launch over all classes (jk_fused_kernel) up to this
+// many candidate quartets and tasks (one per bra and ket class).  Above, its
+// one wavefront per SIMD costs more than the side-by-side classes gain: class
+// launches against one launch, us: water 6-31G** 557 / 122, (H2O)3 887 / 219,
+// (H2O)6 1297 / 848, (H2O)10 2665 / 2833, C4H10 cc-pVDZ 1107 / 754, C7H16
+// 2442 / 3106; batches of 4 clusters 718 / 568, of 64 monomers and dimers
+// (1.5e6 quartets, 26000 tasks) 924 / 1352.
+constexpr double kFusedQuartets = 4.0e6, kFusedTasks = 8.0e3;
+constexpr long kFusedWg = 128;   // strip workgroups a class is cut into at least
+
 static inline int class_pair_id(int cx, int cy) { return cx * (cx + 1) / 2 + cy; }
 
 static void ensure_sig(Species& s, hipStream_t st) {
@@ -555,6 +569,22 @@ static void ensure_sig(Species& s, hipStream_t st) {
     s.sig_mixed = s.mixed;
     s.sig_gen++;
   }
+}
+
+// Whether a plan runs as one launch over all quartet classes.
+static bool want_fused(const BuildPlan& p) {
+  if (p.time_launches || p.serialize) return false;   // per-class times are wanted
+  double quartets = 0.0, tasks = 0.0;   // tasks: one per bra and ket class
+  for (const Species* s : p.mols) {
+    const PairSet& ps = s->sig;
+    if (s->mixed || ps.maxprim > kMaxStripPrims ||
+        (size_t)(2 * ncart_h(kMaxL)) * s->nbasis * sizeof(double) > kStripLdsMax)
+      return false;
+    quartets += 0.5 * (double)ps.pairs.size() * (double)ps.pairs.size();
+    for (int c = 0; c < kNumPairClasses; ++c) tasks += (double)(ps.off[c + 1] - ps.off[c]) * (c + 1);
+    if (quartets > kFusedQuartets || tasks > kFusedTasks) return false;
+  }
+  return true;
 }
 
 // Tasks of a plan, one class launch per (bra class, ket class <= bra class)
@@ -602,137 +632,143 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
         psum[m][k + 1] = psum[m][k] + ps.pairs[k].nprim;
       }
   }
+  p.fused = want_fused(p);
   std::vector<double> unit, upto;   // per run: cost of a quartet, cost of the kets before the run
   std::vector<int> round;           // per run: kets a workgroup takes at once
-  for (int cx = 0; cx < kNumPairClasses; ++cx) {
-    for (int cy = 0; cy <= cx; ++cy) {
-      const int la = kPairClassL[cx][0], lb = kPairClassL[cx][1];
-      const int lc = kPairClassL[cy][0], ld = kPairClassL[cy][1];
-      long total = 0, nbras = 0;
-      int maxbra = 0;   // largest bra primitive-pair count (staged in LDS by the strip kernel)
-      for (int m = 0; m < nm; ++m) {
-        const PairSet& ps = p.mols[m]->sig;
-        const int nx = ps.off[cx + 1] - ps.off[cx], ny = ps.off[cy + 1] - ps.off[cy];
-        if (nx && ny) {
-          total += (cx == cy) ? (long)nx * (nx + 1) / 2 : (long)nx * ny;
-          nbras += nx;
-          for (int i = ps.off[cx]; i < ps.off[cx + 1]; ++i) maxbra = std::max(maxbra, ps.pairs[i].nprim);
-        }
+  for (int id = 0; id < kNumClassPairs; ++id) {
+    // one launch starts its workgroups in task order: the classes with the
+    // longest chains (high angular momentum) first
+    const int at = p.fused ? kNumClassPairs - 1 - id : id;
+    int cx = 0;
+    while ((cx + 1) * (cx + 2) / 2 <= at) ++cx;
+    const int cy = at - cx * (cx + 1) / 2;
+    const int la = kPairClassL[cx][0], lb = kPairClassL[cx][1];
+    const int lc = kPairClassL[cy][0], ld = kPairClassL[cy][1];
+    long total = 0, nbras = 0;
+    int maxbra = 0;   // largest bra primitive-pair count (staged in LDS by the strip kernel)
+    for (int m = 0; m < nm; ++m) {
+      const PairSet& ps = p.mols[m]->sig;
+      const int nx = ps.off[cx + 1] - ps.off[cx], ny = ps.off[cy + 1] - ps.off[cy];
+      if (nx && ny) {
+        total += (cx == cy) ? (long)nx * (nx + 1) / 2 : (long)nx * ny;
+        nbras += nx;
+        for (int i = ps.off[cx]; i < ps.off[cx + 1]; ++i) maxbra = std::max(maxbra, ps.pairs[i].nprim);
       }
-      if (total == 0) continue;
-      // LDS strips pay off when a bra has enough kets to fill a workgroup
-      // (256 threads) for a while; short ket runs (small molecules) go to the
-      // wavefront kernel, one bra x 64 kets per wave.
-      int kd = p.kind[class_pair_id(cx, cy)];
-      // wave-cooperative kernel: by default from total L = kCoopDefaultL up
-      const bool coop_ok = has_jk_coop(la, lb, lc, ld);
-      const bool coop_default = kd < 4 && la + lb + lc + ld >= kCoopDefaultL;
-      const int coop = !coop_ok ? 0 : kd == 4 ? 3 : (kd == 5 || coop_default) ? 4 : 0;
-      if (kd >= 4) kd = 0;
-      const bool strip_ok = (size_t)(ncart_h(la) + ncart_h(lb)) * p.nmax * sizeof(double) <= kStripLdsMax &&
-                            maxbra <= kMaxStripPrims;
-      // untuned: strips wherever they fit, of 256 threads when a bra has on
-      // average >= 192 kets, else of one wavefront (short ket runs of small
-      // molecules would leave most of a 256-thread workgroup idle)
-      const bool strip = coop || (strip_ok && (kd == 1 || kd == 3 || kd == 0));
-      const bool wave64 = kd == 3 || (kd == 0 && total < 192 * nbras);
-      const size_t from = ts.tasks.size();
-      const int block = wave64 ? 64 : 256;
-      const long tgt = coop_default ? kCoopDefaultWg : p.target_wg[class_pair_id(cx, cy)];
-      made.clear();
-      double work = 0.0;   // primitive quartets of the launch
-      for (int m = 0; m < nm; ++m) {
-        const PairSet& ps = p.mols[m]->sig;
-        for (int i = 0; i < ps.off[cx + 1] - ps.off[cx]; ++i) {
-          const int nk = (cx == cy) ? i + 1 : ps.off[cy + 1] - ps.off[cy];
-          work += (psum[m][ps.off[cy] + nk] - psum[m][ps.off[cy]]) * ps.pairs[ps.off[cx] + i].nprim;
-        }
-      }
-      int lmax = 0;
-      if (strip && !coop) {
-        lmax = (int)std::max(kSplitMin, std::min(kSplitMax, (double)total / (kSplitKets * (double)nbras)));
-      }
-      const double flush = 8.0 + (double)(ncart_h(la) + ncart_h(lb)) * p.nmax / block;
-      const double goal = (wave64 ? 4.0 : 1.0) * (double)tgt;
-      const double cap = std::max((work + kQuartetIters * (double)total) / goal, 4.0 * block * flush);
-      const long chunk = std::max(kCoopMinRun, std::min(32768L, ((total + tgt - 1) / tgt + 3) / 4 * 4));
-      for (int m = 0; m < nm; ++m) {
-        const PairSet& ps = p.mols[m]->sig;
-        const int nx = ps.off[cx + 1] - ps.off[cx], ny = ps.off[cy + 1] - ps.off[cy];
-        if (nx == 0 || ny == 0) continue;
-        const PairInfo* kets = ps.pairs.data() + ps.off[cy];
-        const std::vector<Run>& kr = runs[m][cy];
-        unit.resize(kr.size());
-        upto.resize(kr.size());
-        round.resize(kr.size());
-        int last = -1;   // primitive count of the bra the per-run costs are for
-        size_t rk = 0;
-        for (int i = 0; i < nx; ++i) {
-          const int nk = (cx == cy) ? i + 1 : ny, nbp = ps.pairs[ps.off[cx] + i].nprim;
-          if (coop) {
-            const int pieces = (int)((nk + chunk - 1) / chunk);
-            for (int q = 0; q < pieces; ++q) {
-              const int j0 = (int)((long)nk * q / pieces), j1 = (int)((long)nk * (q + 1) / pieces);
-              if (j1 > j0) made.push_back({(double)nbp * kets[j0].nprim * (j1 - j0), Task{i, j0, j1, m}});
-            }
-          } else if (strip) {
-            // pieces of about equal cost, cut at whole rounds of the workgroup
-            if (nbp != last) {
-              double c = 0.0;
-              for (size_t r = 0; r < kr.size(); ++r) {
-                const int ls = split_shift(nbp, kr[r].np, lmax);
-                unit[r] = (double)nbp * kr[r].np + kQuartetIters * (double)(1 << ls);
-                round[r] = block >> ls;
-                upto[r] = c;
-                c += unit[r] * (kr[r].j1 - kr[r].j0);
-              }
-              last = nbp;
-              rk = 0;
-            }
-            if (cx != cy) rk = kr.size() - 1;
-            while (kr[rk].j1 < nk) ++rk;   // the run of the last ket
-            while (kr[rk].j0 >= nk) --rk;
-            const double all = upto[rk] + unit[rk] * (nk - kr[rk].j0);
-            if (all <= cap) {
-              made.push_back({all, Task{i, 0, nk, m}});
-              continue;
-            }
-            const double share = all / std::ceil(all / cap) * (1.0 - 1e-9);
-            double acc = 0.0;
-            int j0 = 0;
-            for (size_t r = 0; r <= rk; ++r) {
-              const int end = std::min(kr[r].j1, nk);
-              for (int j = kr[r].j0; j < end;) {
-                const int want = (int)std::min(1e9, std::ceil((share - acc) / unit[r]));
-                const int take = std::min(end - j, std::max(1, (want + round[r] - 1) / round[r]) * round[r]);
-                acc += take * unit[r];
-                j += take;
-                if (acc >= share || j == nk) {
-                  made.push_back({acc, Task{i, j0, j, m}});
-                  j0 = j;
-                  acc = 0.0;
-                }
-              }
-            }
-          } else {
-            const size_t at = ts.tasks.size();
-            emit_tasks(ts.tasks, i, 0, nk, kets, m);
-            for (size_t k = at; k < ts.tasks.size(); ++k) {
-              const Task& t = ts.tasks[k];
-              made.push_back({(double)nbp * kets[t.j0].nprim * (t.j1 - t.j0), t});
-            }
-            ts.tasks.resize(at);
-          }
-        }
-      }
-      std::stable_sort(made.begin(), made.end(),
-                       [](const std::pair<double, Task>& x, const std::pair<double, Task>& y) { return x.first > y.first; });
-      for (const auto& t : made) ts.tasks.push_back(t.second);
-      ts.launches.push_back({la, lb, lc, ld, cx, cy, 1, from, ts.tasks.size() - from,
-                             coop ? coop : (strip ? (wave64 ? 2 : 1) : 0), lmax});
-      // estimated cost of the launch: primitive quartets x class weight
-      cost.push_back(work * (1.0 + (la + lb + lc + ld) * (la + lb + lc + ld)));
     }
+    if (total == 0) continue;
+    // LDS strips pay off when a bra has enough kets to fill a workgroup
+    // (256 threads) for a while; short ket runs (small molecules) go to the
+    // wavefront kernel, one bra x 64 kets per wave.
+    int kd = p.fused ? 3 : p.kind[class_pair_id(cx, cy)];
+    // wave-cooperative kernel: by default from total L = kCoopDefaultL up
+    const bool coop_ok = has_jk_coop(la, lb, lc, ld);
+    const bool coop_default = kd < 4 && la + lb + lc + ld >= kCoopDefaultL;
+    const int coop = !coop_ok ? 0 : kd == 4 ? 3 : (kd == 5 || coop_default) ? 4 : 0;
+    if (kd >= 4) kd = 0;
+    const bool strip_ok = (size_t)(ncart_h(la) + ncart_h(lb)) * p.nmax * sizeof(double) <= kStripLdsMax &&
+                          maxbra <= kMaxStripPrims;
+    // untuned: strips wherever they fit, of 256 threads when a bra has on
+    // average >= 192 kets, else of one wavefront (short ket runs of small
+    // molecules would leave most of a 256-thread workgroup idle)
+    const bool strip = coop || (strip_ok && (kd == 1 || kd == 3 || kd == 0));
+    const bool wave64 = kd == 3 || (kd == 0 && total < 192 * nbras);
+    const size_t from = ts.tasks.size();
+    const int block = wave64 ? 64 : 256;
+    const long tgt = coop_default ? kCoopDefaultWg : p.fused ? kFusedWg : p.target_wg[class_pair_id(cx, cy)];
+    made.clear();
+    double work = 0.0;   // primitive quartets of the launch
+    for (int m = 0; m < nm; ++m) {
+      const PairSet& ps = p.mols[m]->sig;
+      for (int i = 0; i < ps.off[cx + 1] - ps.off[cx]; ++i) {
+        const int nk = (cx == cy) ? i + 1 : ps.off[cy + 1] - ps.off[cy];
+        work += (psum[m][ps.off[cy] + nk] - psum[m][ps.off[cy]]) * ps.pairs[ps.off[cx] + i].nprim;
+      }
+    }
+    int lmax = 0;
+    if (strip && !coop) {
+      lmax = (int)std::max(kSplitMin, std::min(kSplitMax, (double)total / (kSplitKets * (double)nbras)));
+    }
+    const double flush = 8.0 + (double)(ncart_h(la) + ncart_h(lb)) * p.nmax / block;
+    const double goal = (wave64 ? 4.0 : 1.0) * (double)tgt;
+    const double cap = std::max((work + kQuartetIters * (double)total) / goal, 4.0 * block * flush);
+    const long even = (total + tgt - 1) / tgt;   // kets of a cooperative task
+    const long chunk = p.fused ? even : std::max(kCoopMinRun, std::min(32768L, (even + 3) / 4 * 4));
+    for (int m = 0; m < nm; ++m) {
+      const PairSet& ps = p.mols[m]->sig;
+      const int nx = ps.off[cx + 1] - ps.off[cx], ny = ps.off[cy + 1] - ps.off[cy];
+      if (nx == 0 || ny == 0) continue;
+      const PairInfo* kets = ps.pairs.data() + ps.off[cy];
+      const std::vector<Run>& kr = runs[m][cy];
+      unit.resize(kr.size());
+      upto.resize(kr.size());
+      round.resize(kr.size());
+      int last = -1;   // primitive count of the bra the per-run costs are for
+      size_t rk = 0;
+      for (int i = 0; i < nx; ++i) {
+        const int nk = (cx == cy) ? i + 1 : ny, nbp = ps.pairs[ps.off[cx] + i].nprim;
+        if (coop) {
+          const int pieces = (int)((nk + chunk - 1) / chunk);
+          for (int q = 0; q < pieces; ++q) {
+            const int j0 = (int)((long)nk * q / pieces), j1 = (int)((long)nk * (q + 1) / pieces);
+            if (j1 > j0) made.push_back({(double)nbp * kets[j0].nprim * (j1 - j0), Task{i, j0, j1, m}});
+          }
+        } else if (strip) {
+          // pieces of about equal cost, cut at whole rounds of the workgroup
+          if (nbp != last) {
+            double c = 0.0;
+            for (size_t r = 0; r < kr.size(); ++r) {
+              const int ls = split_shift(nbp, kr[r].np, lmax);
+              unit[r] = (double)nbp * kr[r].np + kQuartetIters * (double)(1 << ls);
+              round[r] = block >> ls;
+              upto[r] = c;
+              c += unit[r] * (kr[r].j1 - kr[r].j0);
+            }
+            last = nbp;
+            rk = 0;
+          }
+          if (cx != cy) rk = kr.size() - 1;
+          while (kr[rk].j1 < nk) ++rk;   // the run of the last ket
+          while (kr[rk].j0 >= nk) --rk;
+          const double all = upto[rk] + unit[rk] * (nk - kr[rk].j0);
+          if (all <= cap) {
+            made.push_back({all, Task{i, 0, nk, m}});
+            continue;
+          }
+          const double share = all / std::ceil(all / cap) * (1.0 - 1e-9);
+          double acc = 0.0;
+          int j0 = 0;
+          for (size_t r = 0; r <= rk; ++r) {
+            const int end = std::min(kr[r].j1, nk);
+            for (int j = kr[r].j0; j < end;) {
+              const int want = (int)std::min(1e9, std::ceil((share - acc) / unit[r]));
+              const int take = std::min(end - j, std::max(1, (want + round[r] - 1) / round[r]) * round[r]);
+              acc += take * unit[r];
+              j += take;
+              if (acc >= share || j == nk) {
+                made.push_back({acc, Task{i, j0, j, m}});
+                j0 = j;
+                acc = 0.0;
+              }
+            }
+          }
+        } else {
+          const size_t at = ts.tasks.size();
+          emit_tasks(ts.tasks, i, 0, nk, kets, m);
+          for (size_t k = at; k < ts.tasks.size(); ++k) {
+            const Task& t = ts.tasks[k];
+            made.push_back({(double)nbp * kets[t.j0].nprim * (t.j1 - t.j0), t});
+          }
+          ts.tasks.resize(at);
+        }
+      }
+    }
+    std::stable_sort(made.begin(), made.end(),
+                     [](const std::pair<double, Task>& x, const std::pair<double, Task>& y) { return x.first > y.first; });
+    for (const auto& t : made) ts.tasks.push_back(t.second);
+    ts.launches.push_back({la, lb, lc, ld, cx, cy, 1, from, ts.tasks.size() - from,
+                           coop ? coop : (strip ? (wave64 ? 2 : 1) : 0), lmax});
+    // estimated cost of the launch: primitive quartets x class weight
+    cost.push_back(work * (1.0 + (la + lb + lc + ld) * (la + lb + lc + ld)));
   }
   ts.order.resize(ts.launches.size());
   for (size_t k = 0; k < ts.order.size(); ++k) ts.order[k] = k;
@@ -764,7 +800,7 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
 }
 
 static void ensure_plan(BuildPlan& p, hipStream_t st) {
-  bool stale = !p.valid || p.sig_gen.size() != p.mols.size();
+  bool stale = !p.valid || p.sig_gen.size() != p.mols.size() || p.fused != want_fused(p);
   for (size_t m = 0; m < p.mols.size(); ++m) {
     ensure_sig(*p.mols[m], st);
     if (!stale && p.sig_gen[m] != p.mols[m]->sig_gen) stale = true;
@@ -894,6 +930,23 @@ static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, int which,
                             const MolDesc* mols = nullptr, bool counts_off = false) {
   Context& c = ctx();
   const size_t nl = p.ts.launches.size();
+  if (p.fused && which != 2) {
+    FusedArgs f{};
+    f.tasks = p.ts.d_tasks.p;
+    f.mols = mols ? mols : p.d_desc.p;
+    f.boys = c.boys.p;
+    f.counts = counts_off ? nullptr : p.d_task_counts.p;
+    f.eps = p.eps;
+    f.lds_n = p.nmax;
+    for (const TaskSet::Launch& L : p.ts.launches) {
+      f.first[f.nseg] = (int)L.off;
+      f.cls[f.nseg] = 1000 * L.la + 100 * L.lb + 10 * L.lc + L.ld;
+      f.lmax[f.nseg++] = L.lmax;
+    }
+    f.first[f.nseg] = (int)p.ts.tasks.size();
+    launch_jk_fused(f, st);
+    return;
+  }
   bool any = false, any_heavy = false;
   for (size_t k = 0; k < nl; ++k) {
     any = any || which == 0 || (which == 1) != heavy_launch(p.ts.launches[k]);
@@ -1016,7 +1069,7 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
   const bool timed = p.time_launches && !p.use_graph;
   if (timed) ensure_launch_events(p);
   if (record) HIPCHK(hipEventRecord(c.ev0, st));
-  if (p.use_graph) {
+  if (p.use_graph && !p.fused) {
     // The graph holds the classes without a large private segment.  Kernels
     // in a graph run on the runtime's own streams (one per branch), so the
     // scratch-heavy classes stay outside it, on side stream 0: they are

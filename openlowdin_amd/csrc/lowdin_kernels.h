@@ -58,6 +58,25 @@ struct JKArgs {
                            // lanes share a quartet (0: one lane per quartet)
 };
 
+// The J/K launches of all quartet classes of a small build as one launch of
+// one-wavefront workgroups: workgroup b runs task b, whose class is that of
+// the segment seg with first[seg] <= b < first[seg + 1].
+constexpr int kMaxSegments = 21;
+struct FusedArgs {
+  const Task* tasks;
+  const MolDesc* mols;
+  const double* boys;
+  unsigned int* counts;    // as JKArgs::counts
+  double eps;
+  int nseg;
+  int lds_n;               // largest n of the launch
+  int first[kMaxSegments + 1];
+  int cls[kMaxSegments];   // 1000 la + 100 lb + 10 lc + ld
+  int lmax[kMaxSegments];
+};
+size_t jk_fused_lds(int nmax);   // dynamic LDS of a workgroup
+void launch_jk_fused(const FusedArgs& a, hipStream_t s);
+
 // log2 of the lanes that share a quartet of nbp x nkp primitive pairs: as few
 // as bring the serial loop of a lane down to lmax primitive quartets, at most
 // one wavefront and no more than the ket has primitive pairs.
