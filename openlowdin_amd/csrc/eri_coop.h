@@ -100,6 +100,43 @@ __device__ __forceinline__ double boys_one(double T, int m, const double* __rest
   return f;
 }
 
+// The HRR rounds: (ab|cd) at R + kOut from the contracted [e0|f0].
+template <int LA, int LB, int LC, int LD>
+__device__ __forceinline__ void coop_hrr(double* R, const uint2* pg, const PairInfo& P, const PairInfo& K, int lane) {
+  using Pg = CoopProgram<LA, LB, LC, LD>;
+  if (lane == 0) {
+    R[12] = P.ABx;
+    R[13] = P.ABy;
+    R[14] = P.ABz;
+    R[15] = K.ABx;
+    R[16] = K.ABy;
+    R[17] = K.ABz;
+  }
+  {
+    const uint2* q = pg + (Pg::kVrrRounds + Pg::kAccRounds) * 64;
+    uint2 dn[kCoopGroup];
+    coop_load<Pg::kHrrG[0], Pg::kHrrG[1]>(q, 0, dn);
+#pragma unroll 1
+    for (int g = 0; g < Pg::kHrrGroups; ++g) {
+      const unsigned c = coop_code<Pg::kHrrG[0], Pg::kHrrG[1]>(g);
+      const int nr = (int)(c & 7u) + 1;
+      const int cb = (c & 8u) ? 15 : 12;
+      uint2 d[kCoopGroup];
+#pragma unroll
+      for (int k = 0; k < kCoopGroup; ++k) d[k] = dn[k];
+      q += nr * 64;
+      if (g + 1 < Pg::kHrrGroups) coop_load<Pg::kHrrG[0], Pg::kHrrG[1]>(q, g + 1, dn);
+      double v[kCoopGroup];
+#pragma unroll
+      for (int k = 0; k < kCoopGroup; ++k)
+        if (k < nr) v[k] = lds_at(R, d[k].x & 0xffffu) + R[cb + (d[k].y & 3u)] * lds_at(R, d[k].x >> 16);
+#pragma unroll
+      for (int k = 0; k < kCoopGroup; ++k)
+        if (k < nr) lds_ref(R, d[k].y & 0xfff8u) = v[k];
+    }
+  }
+}
+
 // One contracted quartet of class (LA LB|LC LD), raw (unnormalised
 // functions), by one wavefront: the [e0|f0] accumulators are cleared, every
 // primitive quartet (bra primitive pairs bprim[0..nbp), ket kprim[0..nkp))
@@ -208,37 +245,126 @@ __device__ __forceinline__ void coop_quartet(double* R, const uint2* pg, gcptr<d
       }
     }
   }
-  // HRR groups
-  if (lane == 0) {
-    R[12] = P.ABx;
-    R[13] = P.ABy;
-    R[14] = P.ABz;
-    R[15] = K.ABx;
-    R[16] = K.ABy;
-    R[17] = K.ABz;
-  }
-  {
-    const uint2* q = pg + (Pg::kVrrRounds + Pg::kAccRounds) * 64;
-    uint2 dn[kCoopGroup];
-    coop_load<Pg::kHrrG[0], Pg::kHrrG[1]>(q, 0, dn);
-#pragma unroll 1
-    for (int g = 0; g < Pg::kHrrGroups; ++g) {
-      const unsigned c = coop_code<Pg::kHrrG[0], Pg::kHrrG[1]>(g);
-      const int nr = (int)(c & 7u) + 1;
-      const int cb = (c & 8u) ? 15 : 12;
-      uint2 d[kCoopGroup];
-#pragma unroll
-      for (int k = 0; k < kCoopGroup; ++k) d[k] = dn[k];
-      q += nr * 64;
-      if (g + 1 < Pg::kHrrGroups) coop_load<Pg::kHrrG[0], Pg::kHrrG[1]>(q, g + 1, dn);
-      double v[kCoopGroup];
-#pragma unroll
-      for (int k = 0; k < kCoopGroup; ++k)
-        if (k < nr) v[k] = lds_at(R, d[k].x & 0xffffu) + R[cb + (d[k].y & 3u)] * lds_at(R, d[k].x >> 16);
-#pragma unroll
-      for (int k = 0; k < kCoopGroup; ++k)
-        if (k < nr) lds_ref(R, d[k].y & 0xfff8u) = v[k];
+  coop_hrr<LA, LB, LC, LD>(R, pg, P, K, lane);
+}
+
+// What the J/K contraction of a cooperative quartet reads and adds to.
+struct CoopJk {
+  int n;
+  gcptr<double> D, nrm;
+  gptr<double> G;
+  gcptr<double> Dp;        // kPacked: packed ket densities and J accumulator (MolDesc::Dp,
+  gptr<double> Jp;         // Jp) of the ket class
+  int npk;                 // its pairs
+  double hf;               // 0.5 * exchange factor
+  double* sa;              // row strips (sn > 0)
+  double* sb;
+  int sn;
+};
+
+// J/K contraction of the (ab|cd) block at R + kOut with ket j of its class
+// (Libint2Iface.cpp:562-586); lane k < NA NB keeps J_ab element k in jab, the
+// normalised bra density block is at R + kRegion.
+template <bool kPacked, int LA, int LB, int LC, int LD>
+__device__ __forceinline__ void coop_jk_update(double* R, const CoopJk& u, const PairInfo& P, const PairInfo& K, int j,
+                                               double deg, int lane, double& jab) {
+  using Pg = CoopProgram<LA, LB, LC, LD>;
+  constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int NAB = NA * NB, NCD = NC * ND;
+  constexpr int oDab = Pg::kRegion, oDcd = oDab + NAB, oDac = oDcd + NCD, oDbd = oDac + NA * NC,
+                oDad = oDbd + NB * ND, oDbc = oDad + NA * ND;
+  const int n = u.n, sn = u.sn;
+  const gcptr<double> nrm = u.nrm;
+  const gptr<double> G = u.G;
+  double* sa = u.sa;
+  double* sb = u.sb;
+  const double hf = u.hf;
+  const double* out = R + Pg::kOut;
+  for (int k = lane; k < NCD; k += 64) {
+    if constexpr (kPacked) {
+      R[oDcd + k] = u.Dp[(size_t)k * u.npk + j];
+    } else {
+      const int fc = K.bfa + k / ND, fd = K.bfb + k % ND;
+      R[oDcd + k] = u.D[(size_t)fc * n + fd] * nrm[fc] * nrm[fd];
     }
+  }
+  for (int k = lane; k < NA * NC + NB * ND + NA * ND + NB * NC; k += 64) {
+    int r0, c0, o;
+    if (k < NA * NC) {
+      r0 = P.bfa + k / NC; c0 = K.bfa + k % NC; o = oDac + k;
+    } else if (k < NA * NC + NB * ND) {
+      const int v = k - NA * NC;
+      r0 = P.bfb + v / ND; c0 = K.bfb + v % ND; o = oDbd + v;
+    } else if (k < NA * NC + NB * ND + NA * ND) {
+      const int v = k - NA * NC - NB * ND;
+      r0 = P.bfa + v / ND; c0 = K.bfb + v % ND; o = oDad + v;
+    } else {
+      const int v = k - NA * NC - NB * ND - NA * ND;
+      r0 = P.bfb + v / NC; c0 = K.bfa + v % NC; o = oDbc + v;
+    }
+    R[o] = u.D[(size_t)r0 * n + c0] * nrm[r0] * nrm[c0];
+  }
+  if (lane < NAB) {
+    double s = 0.0;
+#pragma unroll 6
+    for (int cd = 0; cd < NCD; ++cd) s += out[lane * NCD + cd] * R[oDcd + cd];
+    jab += deg * s;
+  }
+  if (lane < NCD) {
+    double s = 0.0;
+#pragma unroll 6
+    for (int ab = 0; ab < NAB; ++ab) s += out[ab * NCD + lane] * R[oDab + ab];
+    if constexpr (kPacked) {
+      global_add(u.Jp + (size_t)lane * u.npk + j, deg * s);
+    } else {
+      const int fc = K.bfa + lane / ND, fd = K.bfb + lane % ND;
+      global_add(G + (size_t)fc * n + fd, deg * s * nrm[fc] * nrm[fd]);
+    }
+  }
+  const double sk = deg * hf;
+  if (lane < NA * NC) {  // K_ac = sum_bd (ab|cd) D_bd
+    const int ia = lane / NC, ic = lane % NC;
+    double s = 0.0;
+#pragma unroll 6
+    for (int ib = 0; ib < NB; ++ib)
+#pragma unroll 6
+      for (int id = 0; id < ND; ++id) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDbd + ib * ND + id];
+    const int fc = K.bfa + ic;
+    if (sn) atomicAdd(&sa[ia * sn + fc], sk * s * nrm[fc]);
+    else global_add(G + (size_t)(P.bfa + ia) * n + fc, sk * s * nrm[fc] * nrm[P.bfa + ia]);
+  }
+  if (lane < NB * ND) {  // K_bd = sum_ac (ab|cd) D_ac
+    const int ib = lane / ND, id = lane % ND;
+    double s = 0.0;
+#pragma unroll 6
+    for (int ia = 0; ia < NA; ++ia)
+#pragma unroll 6
+      for (int ic = 0; ic < NC; ++ic) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDac + ia * NC + ic];
+    const int fd = K.bfb + id;
+    if (sn) atomicAdd(&sb[ib * sn + fd], sk * s * nrm[fd]);
+    else global_add(G + (size_t)(P.bfb + ib) * n + fd, sk * s * nrm[fd] * nrm[P.bfb + ib]);
+  }
+  if (lane < NA * ND) {  // K_ad = sum_bc (ab|cd) D_bc
+    const int ia = lane / ND, id = lane % ND;
+    double s = 0.0;
+#pragma unroll 6
+    for (int ib = 0; ib < NB; ++ib)
+#pragma unroll 6
+      for (int ic = 0; ic < NC; ++ic) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDbc + ib * NC + ic];
+    const int fd = K.bfb + id;
+    if (sn) atomicAdd(&sa[ia * sn + fd], sk * s * nrm[fd]);
+    else global_add(G + (size_t)(P.bfa + ia) * n + fd, sk * s * nrm[fd] * nrm[P.bfa + ia]);
+  }
+  if (lane < NB * NC) {  // K_bc = sum_ad (ab|cd) D_ad
+    const int ib = lane / NC, ic = lane % NC;
+    double s = 0.0;
+#pragma unroll 6
+    for (int ia = 0; ia < NA; ++ia)
+#pragma unroll 6
+      for (int id = 0; id < ND; ++id) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDad + ia * ND + id];
+    const int fc = K.bfa + ic;
+    if (sn) atomicAdd(&sb[ib * sn + fc], sk * s * nrm[fc]);
+    else global_add(G + (size_t)(P.bfb + ib) * n + fc, sk * s * nrm[fc] * nrm[P.bfb + ib]);
   }
 }
 
@@ -249,10 +375,9 @@ __device__ __forceinline__ void jk_coop_body(const JKArgs& a, const Task& t, uns
                                              unsigned int* wg) {
   using Pg = CoopProgram<LA, LB, LC, LD>;
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-  constexpr int NAB = NA * NB, NCD = NC * ND;
+  constexpr int NAB = NA * NB;
   constexpr int kWave = coop_wave_doubles<LA, LB, LC, LD>();
-  constexpr int oDab = Pg::kRegion, oDcd = oDab + NAB, oDac = oDcd + NCD, oDbd = oDac + NA * NC,
-                oDad = oDbd + NB * ND, oDbc = oDad + NA * ND;
+  constexpr int oDab = Pg::kRegion;
   static_assert(NAB <= 64, "one J_ab element per lane");
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -265,9 +390,6 @@ __device__ __forceinline__ void jk_coop_body(const JKArgs& a, const Task& t, uns
   const gptr<double> G = (gptr<double>)M.Graw;
   const PairInfo P = load_pair(pairs + M.off[a.cbra] + t.bra);
   const int n = M.n, ns = M.nshell;
-  const int npk = M.off[a.cket + 1] - M.off[a.cket];
-  const gcptr<double> Dp = (gcptr<double>)M.Dp + M.jpoff[a.cket];
-  const gptr<double> Jp = (gptr<double>)M.Jp + M.jpoff[a.cket];
   const int sn = a.lds_n;                 // strip width (0: no strips)
   double* sa = lds;
   double* sb = lds + NA * sn;
@@ -286,7 +408,6 @@ __device__ __forceinline__ void jk_coop_body(const JKArgs& a, const Task& t, uns
   double jab = 0.0;
   unsigned int myq = 0, myp = 0;
   const double sbra = (P.sa != P.sb ? 2.0 : 1.0);
-  const double hf = M.half_factor;
   const gcptr<double> bprim = prim + (size_t)P.poff * kPrimPairStride;
   const uint2* pg = Pg::prog() + lane;   // this lane's column of the round table
   __syncthreads();
@@ -300,83 +421,12 @@ __device__ __forceinline__ void jk_coop_body(const JKArgs& a, const Task& t, uns
     myp += (unsigned int)(P.nprim * K.nprim);
     const gcptr<double> kprim = prim + (size_t)K.poff * kPrimPairStride;
     coop_quartet<LA, LB, LC, LD>(R, pg, bprim, P.nprim, kprim, K.nprim, a.boys, P, K, lane);
-    // J/K contraction of the (ab|cd) block (Libint2Iface.cpp:562-586)
-    const double* out = R + Pg::kOut;
     const double deg = sbra * (K.sa != K.sb ? 2.0 : 1.0) * ((a.same_class && j == t.bra) ? 1.0 : 2.0);
-    for (int k = lane; k < NCD; k += 64) R[oDcd + k] = Dp[(size_t)k * npk + j];
-    for (int k = lane; k < NA * NC + NB * ND + NA * ND + NB * NC; k += 64) {
-      int r0, c0, o;
-      if (k < NA * NC) {
-        r0 = P.bfa + k / NC; c0 = K.bfa + k % NC; o = oDac + k;
-      } else if (k < NA * NC + NB * ND) {
-        const int u = k - NA * NC;
-        r0 = P.bfb + u / ND; c0 = K.bfb + u % ND; o = oDbd + u;
-      } else if (k < NA * NC + NB * ND + NA * ND) {
-        const int u = k - NA * NC - NB * ND;
-        r0 = P.bfa + u / ND; c0 = K.bfb + u % ND; o = oDad + u;
-      } else {
-        const int u = k - NA * NC - NB * ND - NA * ND;
-        r0 = P.bfb + u / NC; c0 = K.bfa + u % NC; o = oDbc + u;
-      }
-      R[o] = D[(size_t)r0 * n + c0] * nrm[r0] * nrm[c0];
-    }
-    if (lane < NAB) {
-      double s = 0.0;
-#pragma unroll 6
-      for (int cd = 0; cd < NCD; ++cd) s += out[lane * NCD + cd] * R[oDcd + cd];
-      jab += deg * s;
-    }
-    if (lane < NCD) {
-      double s = 0.0;
-#pragma unroll 6
-      for (int ab = 0; ab < NAB; ++ab) s += out[ab * NCD + lane] * R[oDab + ab];
-      global_add(Jp + (size_t)lane * npk + j, deg * s);
-    }
-    const double sk = deg * hf;
-    if (lane < NA * NC) {  // K_ac = sum_bd (ab|cd) D_bd
-      const int ia = lane / NC, ic = lane % NC;
-      double s = 0.0;
-#pragma unroll 6
-      for (int ib = 0; ib < NB; ++ib)
-#pragma unroll 6
-        for (int id = 0; id < ND; ++id) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDbd + ib * ND + id];
-      const int fc = K.bfa + ic;
-      if (sn) atomicAdd(&sa[ia * sn + fc], sk * s * nrm[fc]);
-      else global_add(G + (size_t)(P.bfa + ia) * n + fc, sk * s * nrm[fc] * nrm[P.bfa + ia]);
-    }
-    if (lane < NB * ND) {  // K_bd = sum_ac (ab|cd) D_ac
-      const int ib = lane / ND, id = lane % ND;
-      double s = 0.0;
-#pragma unroll 6
-      for (int ia = 0; ia < NA; ++ia)
-#pragma unroll 6
-        for (int ic = 0; ic < NC; ++ic) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDac + ia * NC + ic];
-      const int fd = K.bfb + id;
-      if (sn) atomicAdd(&sb[ib * sn + fd], sk * s * nrm[fd]);
-      else global_add(G + (size_t)(P.bfb + ib) * n + fd, sk * s * nrm[fd] * nrm[P.bfb + ib]);
-    }
-    if (lane < NA * ND) {  // K_ad = sum_bc (ab|cd) D_bc
-      const int ia = lane / ND, id = lane % ND;
-      double s = 0.0;
-#pragma unroll 6
-      for (int ib = 0; ib < NB; ++ib)
-#pragma unroll 6
-        for (int ic = 0; ic < NC; ++ic) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDbc + ib * NC + ic];
-      const int fd = K.bfb + id;
-      if (sn) atomicAdd(&sa[ia * sn + fd], sk * s * nrm[fd]);
-      else global_add(G + (size_t)(P.bfa + ia) * n + fd, sk * s * nrm[fd] * nrm[P.bfa + ia]);
-    }
-    if (lane < NB * NC) {  // K_bc = sum_ad (ab|cd) D_ad
-      const int ib = lane / NC, ic = lane % NC;
-      double s = 0.0;
-#pragma unroll 6
-      for (int ia = 0; ia < NA; ++ia)
-#pragma unroll 6
-        for (int id = 0; id < ND; ++id) s += out[((ia * NB + ib) * NC + ic) * ND + id] * R[oDad + ia * ND + id];
-      const int fc = K.bfa + ic;
-      if (sn) atomicAdd(&sb[ib * sn + fc], sk * s * nrm[fc]);
-      else global_add(G + (size_t)(P.bfb + ib) * n + fc, sk * s * nrm[fc] * nrm[P.bfb + ib]);
-    }
+    // made here, not before the loop: kept live through the quartet these
+    // scalars cost (dd|pp) a wave per SIMD (0.95 -> 1.23 ms for C20H42)
+    const CoopJk u{n, D, nrm, G, (gcptr<double>)M.Dp + M.jpoff[a.cket], (gptr<double>)M.Jp + M.jpoff[a.cket],
+                   M.off[a.cket + 1] - M.off[a.cket], M.half_factor, sa, sb, sn};
+    coop_jk_update<true, LA, LB, LC, LD>(R, u, P, K, j, deg, lane, jab);
   }
   // J_ab of this wavefront (lane-owned elements)
   if (lane < NAB && jab != 0.0) {
@@ -420,32 +470,12 @@ __global__ __launch_bounds__(256, 2) void jk_coop_kernel(JKArgs a) {
   jk_coop_body<LA, LB, LC, LD>(a, a.tasks[blockIdx.x], a.counts ? a.counts + 3 * blockIdx.x : nullptr, lds, wg);
 }
 
-// Inter-species Coulomb coupling (Libint2Iface.cpp:1111-1294) of one class
-// with one wavefront per quartet: the quartet as above, then the drop of
-// raw integrals below a.drop and the two contractions of coupling_scatter
-// (eri_core.h) split over the lanes -- lane k < NA NB sums result element
-// (a b) on the bra species over the ket density's element set, lane k <
-// NC ND element (c d) on the ket species over the bra density's.  A
-// workgroup owns one coupling task (a bra pair and up to 64 ket pairs);
-// its wavefronts take the kets in turn.  No private segment: the state of
-// a quartet lives in the wavefront's LDS region.
+// Weights of the bra density of a cooperative coupling task, into its
+// wavefront's region.
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(256, 2) void coupling_coop_kernel(CouplingArgs a) {
-  using Pg = CoopProgram<LA, LB, LC, LD>;
-  constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-  constexpr int NAB = NA * NB, NCD = NC * ND;
-  constexpr int kWave = coop_wave_doubles<LA, LB, LC, LD>();
-  constexpr int oWb = Pg::kRegion, oWk = oWb + NAB;   // bra and ket density weights
-  static_assert(NAB <= 64 && NCD <= 64, "one result element per lane");
-  static_assert(oWk + NCD <= kWave, "weights inside the wavefront's region");
-  extern __shared__ double lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nw = blockDim.x >> 6;
-  const Task t = a.tasks[blockIdx.x];
-  const PairInfo P = load_pair((gcptr<PairInfo>)a.bra + t.bra);
-  double* R = lds + w * kWave;
-  if (lane < 2) R[kCoopZero + lane] = 0.0;
+__device__ __forceinline__ void coop_coupling_weights(double* R, const CouplingArgs& a, const PairInfo& P, int lane) {
+  constexpr int NB = ncart(LB), NAB = ncart(LA) * NB;
+  constexpr int oWb = CoopProgram<LA, LB, LC, LD>::kRegion;
   const bool bdiag = P.sa == P.sb;
   // weights of the bra density (result on the ket species): element set
   // ia <= ib within a diagonal shell pair, doubled off the function
@@ -458,51 +488,91 @@ __global__ __launch_bounds__(256, 2) void coupling_coop_kernel(CouplingArgs a) {
       v = (fa != fb ? 2.0 : 1.0) * a.dbra[(size_t)fa * a.nbra + fb] * a.nbra_norma[fa] * a.nbra_norma[fb];
     R[oWb + lane] = v;
   }
+}
+
+// The drop of raw integrals below a.drop and the two contractions of
+// coupling_scatter (eri_core.h) for the (ab|cd) block at R + kOut, split over
+// the lanes; coop_coupling_weights has left the bra density's weights.
+template <int LA, int LB, int LC, int LD>
+__device__ __forceinline__ void coop_coupling_update(double* R, const CouplingArgs& a, const PairInfo& P,
+                                                     const PairInfo& K, int lane) {
+  using Pg = CoopProgram<LA, LB, LC, LD>;
+  constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int NAB = NA * NB, NCD = NC * ND;
+  constexpr int oWb = Pg::kRegion, oWk = oWb + NAB;   // bra and ket density weights
+  static_assert(NAB <= 64 && NCD <= 64, "one result element per lane");
+  static_assert(oWk + NCD <= coop_wave_doubles<LA, LB, LC, LD>(), "weights inside the wavefront's region");
+  const double drop = a.drop;
+  const bool bdiag = P.sa == P.sb;
+  const double* out = R + Pg::kOut;
+  const bool kdiag = K.sa == K.sb;
+  if (a.rbra) {
+    if (lane < NCD) {
+      const int ic = lane / ND, id = lane % ND;
+      const int fc = K.bfa + ic, fd = K.bfb + id;
+      double v = 0.0;
+      if (!kdiag || ic <= id)
+        v = (fc != fd ? 2.0 : 1.0) * a.dket[(size_t)fc * a.nket + fd] * a.nket_norma[fc] * a.nket_norma[fd];
+      R[oWk + lane] = v;
+    }
+    if (lane < NAB) {
+      const int ia = lane / NB, ib = lane % NB;
+      if (!(bdiag && ia > ib)) {
+        double s = 0.0;
+        for (int k = 0; k < NCD; ++k) {
+          const double x = out[lane * NCD + k];
+          s += R[oWk + k] * (fabs(x) < drop ? 0.0 : x);
+        }
+        const int fa = P.bfa + ia, fb = P.bfb + ib;
+        const int r = fa > fb ? fa : fb, c = fa > fb ? fb : fa;
+        unsafeAtomicAdd(&a.rbra[(size_t)r * a.nbra + c], s * a.nbra_norma[fa] * a.nbra_norma[fb]);
+      }
+    }
+  }
+  if (a.rket && lane < NCD) {
+    const int ic = lane / ND, id = lane % ND;
+    if (!(kdiag && ic > id)) {
+      double s = 0.0;
+      for (int k = 0; k < NAB; ++k) {
+        const double x = out[k * NCD + lane];
+        s += R[oWb + k] * (fabs(x) < drop ? 0.0 : x);
+      }
+      const int fc = K.bfa + ic, fd = K.bfb + id;
+      const int r = fc > fd ? fc : fd, c = fc > fd ? fd : fc;
+      unsafeAtomicAdd(&a.rket[(size_t)r * a.nket + c], s * a.nket_norma[fc] * a.nket_norma[fd]);
+    }
+  }
+}
+
+// Inter-species Coulomb coupling (Libint2Iface.cpp:1111-1294) of one class
+// with one wavefront per quartet: the quartet as above, then the drop of
+// raw integrals below a.drop and the two contractions of coupling_scatter
+// (eri_core.h) split over the lanes -- lane k < NA NB sums result element
+// (a b) on the bra species over the ket density's element set, lane k <
+// NC ND element (c d) on the ket species over the bra density's.  A
+// workgroup owns one coupling task (a bra pair and up to 64 ket pairs);
+// its wavefronts take the kets in turn.  No private segment: the state of
+// a quartet lives in the wavefront's LDS region.
+template <int LA, int LB, int LC, int LD>
+__global__ __launch_bounds__(256, 2) void coupling_coop_kernel(CouplingArgs a) {
+  using Pg = CoopProgram<LA, LB, LC, LD>;
+  constexpr int kWave = coop_wave_doubles<LA, LB, LC, LD>();
+  extern __shared__ double lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nw = blockDim.x >> 6;
+  const Task t = a.tasks[blockIdx.x];
+  const PairInfo P = load_pair((gcptr<PairInfo>)a.bra + t.bra);
+  double* R = lds + w * kWave;
+  if (lane < 2) R[kCoopZero + lane] = 0.0;
+  coop_coupling_weights<LA, LB, LC, LD>(R, a, P, lane);
   const gcptr<double> bprim = (gcptr<double>)a.bprim + (size_t)P.poff * kPrimPairStride;
   const uint2* pg = Pg::prog() + lane;
-  const double drop = a.drop;
   for (int j = t.j0 + w; j < t.j1; j += nw) {
     const PairInfo K = load_pair((gcptr<PairInfo>)a.ket + j);
     const gcptr<double> kprim = (gcptr<double>)a.kprim + (size_t)K.poff * kPrimPairStride;
     coop_quartet<LA, LB, LC, LD>(R, pg, bprim, P.nprim, kprim, K.nprim, a.boys, P, K, lane);
-    const double* out = R + Pg::kOut;
-    const bool kdiag = K.sa == K.sb;
-    if (a.rbra) {
-      if (lane < NCD) {
-        const int ic = lane / ND, id = lane % ND;
-        const int fc = K.bfa + ic, fd = K.bfb + id;
-        double v = 0.0;
-        if (!kdiag || ic <= id)
-          v = (fc != fd ? 2.0 : 1.0) * a.dket[(size_t)fc * a.nket + fd] * a.nket_norma[fc] * a.nket_norma[fd];
-        R[oWk + lane] = v;
-      }
-      if (lane < NAB) {
-        const int ia = lane / NB, ib = lane % NB;
-        if (!(bdiag && ia > ib)) {
-          double s = 0.0;
-          for (int k = 0; k < NCD; ++k) {
-            const double x = out[lane * NCD + k];
-            s += R[oWk + k] * (fabs(x) < drop ? 0.0 : x);
-          }
-          const int fa = P.bfa + ia, fb = P.bfb + ib;
-          const int r = fa > fb ? fa : fb, c = fa > fb ? fb : fa;
-          unsafeAtomicAdd(&a.rbra[(size_t)r * a.nbra + c], s * a.nbra_norma[fa] * a.nbra_norma[fb]);
-        }
-      }
-    }
-    if (a.rket && lane < NCD) {
-      const int ic = lane / ND, id = lane % ND;
-      if (!(kdiag && ic > id)) {
-        double s = 0.0;
-        for (int k = 0; k < NAB; ++k) {
-          const double x = out[k * NCD + lane];
-          s += R[oWb + k] * (fabs(x) < drop ? 0.0 : x);
-        }
-        const int fc = K.bfa + ic, fd = K.bfb + id;
-        const int r = fc > fd ? fc : fd, c = fc > fd ? fd : fc;
-        unsafeAtomicAdd(&a.rket[(size_t)r * a.nket + c], s * a.nket_norma[fc] * a.nket_norma[fd]);
-      }
-    }
+    coop_coupling_update<LA, LB, LC, LD>(R, a, P, K, lane);
   }
 }
 

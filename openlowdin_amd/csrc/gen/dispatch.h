@@ -106,9 +106,6 @@ void launch_gcp_2120(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2120(const JKArgs&, hipStream_t);
 bool launch_cpc_2120(const CouplingArgs&, hipStream_t);
 void coop_attr_2120();
-void launch_jk_2121(const JKArgs&, hipStream_t);
-void launch_jks_2121(const JKArgs&, hipStream_t);
-void launch_cp_2121(const CouplingArgs&, hipStream_t);
 void launch_st_2121(const StoreArgs&, hipStream_t);
 void launch_cst_2121(const CouplingStoreArgs&, hipStream_t);
 void launch_gjk_2121(const G12Args&, hipStream_t);
@@ -133,9 +130,6 @@ void launch_gcp_2210(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2210(const JKArgs&, hipStream_t);
 bool launch_cpc_2210(const CouplingArgs&, hipStream_t);
 void coop_attr_2210();
-void launch_jk_2211(const JKArgs&, hipStream_t);
-void launch_jks_2211(const JKArgs&, hipStream_t);
-void launch_cp_2211(const CouplingArgs&, hipStream_t);
 void launch_st_2211(const StoreArgs&, hipStream_t);
 void launch_cst_2211(const CouplingStoreArgs&, hipStream_t);
 void launch_gjk_2211(const G12Args&, hipStream_t);
@@ -143,9 +137,6 @@ void launch_gcp_2211(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2211(const JKArgs&, hipStream_t);
 bool launch_cpc_2211(const CouplingArgs&, hipStream_t);
 void coop_attr_2211();
-void launch_jk_2220(const JKArgs&, hipStream_t);
-void launch_jks_2220(const JKArgs&, hipStream_t);
-void launch_cp_2220(const CouplingArgs&, hipStream_t);
 void launch_st_2220(const StoreArgs&, hipStream_t);
 void launch_cst_2220(const CouplingStoreArgs&, hipStream_t);
 void launch_gjk_2220(const G12Args&, hipStream_t);
@@ -153,9 +144,6 @@ void launch_gcp_2220(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2220(const JKArgs&, hipStream_t);
 bool launch_cpc_2220(const CouplingArgs&, hipStream_t);
 void coop_attr_2220();
-void launch_jk_2221(const JKArgs&, hipStream_t);
-void launch_jks_2221(const JKArgs&, hipStream_t);
-void launch_cp_2221(const CouplingArgs&, hipStream_t);
 void launch_st_2221(const StoreArgs&, hipStream_t);
 void launch_cst_2221(const CouplingStoreArgs&, hipStream_t);
 void launch_gjk_2221(const G12Args&, hipStream_t);
@@ -163,9 +151,6 @@ void launch_gcp_2221(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2221(const JKArgs&, hipStream_t);
 bool launch_cpc_2221(const CouplingArgs&, hipStream_t);
 void coop_attr_2221();
-void launch_jk_2222(const JKArgs&, hipStream_t);
-void launch_jks_2222(const JKArgs&, hipStream_t);
-void launch_cp_2222(const CouplingArgs&, hipStream_t);
 void launch_st_2222(const StoreArgs&, hipStream_t);
 void launch_cst_2222(const CouplingStoreArgs&, hipStream_t);
 void launch_gjk_2222(const G12Args&, hipStream_t);
@@ -195,13 +180,8 @@ inline bool dispatch_jk(int la, int lb, int lc, int ld, const JKArgs& a, hipStre
     case 2110: launch_jk_2110(a, s); return true;
     case 2111: launch_jk_2111(a, s); return true;
     case 2120: launch_jk_2120(a, s); return true;
-    case 2121: launch_jk_2121(a, s); return true;
     case 2200: launch_jk_2200(a, s); return true;
     case 2210: launch_jk_2210(a, s); return true;
-    case 2211: launch_jk_2211(a, s); return true;
-    case 2220: launch_jk_2220(a, s); return true;
-    case 2221: launch_jk_2221(a, s); return true;
-    case 2222: launch_jk_2222(a, s); return true;
     default: return false;
   }
 }
@@ -221,13 +201,8 @@ inline bool dispatch_jk_strip(int la, int lb, int lc, int ld, const JKArgs& a, h
     case 2110: launch_jks_2110(a, s); return true;
     case 2111: launch_jks_2111(a, s); return true;
     case 2120: launch_jks_2120(a, s); return true;
-    case 2121: launch_jks_2121(a, s); return true;
     case 2200: launch_jks_2200(a, s); return true;
     case 2210: launch_jks_2210(a, s); return true;
-    case 2211: launch_jks_2211(a, s); return true;
-    case 2220: launch_jks_2220(a, s); return true;
-    case 2221: launch_jks_2221(a, s); return true;
-    case 2222: launch_jks_2222(a, s); return true;
     default: return false;
   }
 }
@@ -288,13 +263,8 @@ inline bool dispatch_cp(int la, int lb, int lc, int ld, const CouplingArgs& a, h
     case 2110: launch_cp_2110(a, s); return true;
     case 2111: launch_cp_2111(a, s); return true;
     case 2120: launch_cp_2120(a, s); return true;
-    case 2121: launch_cp_2121(a, s); return true;
     case 2200: launch_cp_2200(a, s); return true;
     case 2210: launch_cp_2210(a, s); return true;
-    case 2211: launch_cp_2211(a, s); return true;
-    case 2220: launch_cp_2220(a, s); return true;
-    case 2221: launch_cp_2221(a, s); return true;
-    case 2222: launch_cp_2222(a, s); return true;
     default: return false;
   }
 }

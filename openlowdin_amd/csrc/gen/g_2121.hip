@@ -6,6 +6,7 @@ namespace lowdin {
 #include "eri_2121.inc"
 LOWDIN_ERI_CLASS(2, 1, 2, 1)
 LOWDIN_G12_CLASS(2, 1, 2, 1)
+#include "c_2121.inc"
 
 void launch_gjk_2121(const G12Args& args, hipStream_t s) { launch_g12_t<2, 1, 2, 1>(args, s); }
 void launch_gcp_2121(const G12CouplingArgs& args, hipStream_t s) { launch_g12cp_t<2, 1, 2, 1>(args, s); }

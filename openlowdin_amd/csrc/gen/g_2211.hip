@@ -6,6 +6,7 @@ namespace lowdin {
 #include "eri_2211.inc"
 LOWDIN_ERI_CLASS(2, 2, 1, 1)
 LOWDIN_G12_CLASS(2, 2, 1, 1)
+#include "c_2211.inc"
 
 void launch_gjk_2211(const G12Args& args, hipStream_t s) { launch_g12_t<2, 2, 1, 1>(args, s); }
 void launch_gcp_2211(const G12CouplingArgs& args, hipStream_t s) { launch_g12cp_t<2, 2, 1, 1>(args, s); }

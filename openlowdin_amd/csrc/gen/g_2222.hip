@@ -6,6 +6,7 @@ namespace lowdin {
 #include "eri_2222.inc"
 LOWDIN_ERI_CLASS(2, 2, 2, 2)
 LOWDIN_G12_CLASS(2, 2, 2, 2)
+#include "c_2222.inc"
 
 void launch_gjk_2222(const G12Args& args, hipStream_t s) { launch_g12_t<2, 2, 2, 2>(args, s); }
 void launch_gcp_2222(const G12CouplingArgs& args, hipStream_t s) { launch_g12cp_t<2, 2, 2, 2>(args, s); }

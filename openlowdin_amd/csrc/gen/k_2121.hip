@@ -7,9 +7,6 @@ namespace lowdin {
 LOWDIN_ERI_CLASS(2, 1, 2, 1)
 #include "c_2121.inc"
 
-void launch_jk_2121(const JKArgs& args, hipStream_t s) { launch_jk_t<2, 1, 2, 1>(args, s); }
-void launch_jks_2121(const JKArgs& args, hipStream_t s) { launch_jk_strip_t<2, 1, 2, 1>(args, s); }
-void launch_cp_2121(const CouplingArgs& args, hipStream_t s) { launch_cp_t<2, 1, 2, 1>(args, s); }
 void launch_schwarz_21(PairInfo* pairs, int npairs, const double* prim, const double* boys, const double* norma, hipStream_t s) { launch_schwarz_t<2, 1>(pairs, npairs, prim, boys, norma, s); }
 bool launch_jkc_2121(const JKArgs& args, hipStream_t s) { return launch_jk_coop_t<2, 1, 2, 1>(args, s); }
 bool launch_cpc_2121(const CouplingArgs& args, hipStream_t s) { return launch_cp_coop_t<2, 1, 2, 1>(args, s); }

@@ -7,9 +7,6 @@ namespace lowdin {
 LOWDIN_ERI_CLASS(2, 2, 1, 1)
 #include "c_2211.inc"
 
-void launch_jk_2211(const JKArgs& args, hipStream_t s) { launch_jk_t<2, 2, 1, 1>(args, s); }
-void launch_jks_2211(const JKArgs& args, hipStream_t s) { launch_jk_strip_t<2, 2, 1, 1>(args, s); }
-void launch_cp_2211(const CouplingArgs& args, hipStream_t s) { launch_cp_t<2, 2, 1, 1>(args, s); }
 bool launch_jkc_2211(const JKArgs& args, hipStream_t s) { return launch_jk_coop_t<2, 2, 1, 1>(args, s); }
 bool launch_cpc_2211(const CouplingArgs& args, hipStream_t s) { return launch_cp_coop_t<2, 2, 1, 1>(args, s); }
 void coop_attr_2211() { coop_attr_t<2, 2, 1, 1>(); }

@@ -7,9 +7,6 @@ namespace lowdin {
 LOWDIN_ERI_CLASS(2, 2, 2, 0)
 #include "c_2220.inc"
 
-void launch_jk_2220(const JKArgs& args, hipStream_t s) { launch_jk_t<2, 2, 2, 0>(args, s); }
-void launch_jks_2220(const JKArgs& args, hipStream_t s) { launch_jk_strip_t<2, 2, 2, 0>(args, s); }
-void launch_cp_2220(const CouplingArgs& args, hipStream_t s) { launch_cp_t<2, 2, 2, 0>(args, s); }
 bool launch_jkc_2220(const JKArgs& args, hipStream_t s) { return launch_jk_coop_t<2, 2, 2, 0>(args, s); }
 bool launch_cpc_2220(const CouplingArgs& args, hipStream_t s) { return launch_cp_coop_t<2, 2, 2, 0>(args, s); }
 void coop_attr_2220() { coop_attr_t<2, 2, 2, 0>(); }

@@ -7,9 +7,6 @@ namespace lowdin {
 LOWDIN_ERI_CLASS(2, 2, 2, 1)
 #include "c_2221.inc"
 
-void launch_jk_2221(const JKArgs& args, hipStream_t s) { launch_jk_t<2, 2, 2, 1>(args, s); }
-void launch_jks_2221(const JKArgs& args, hipStream_t s) { launch_jk_strip_t<2, 2, 2, 1>(args, s); }
-void launch_cp_2221(const CouplingArgs& args, hipStream_t s) { launch_cp_t<2, 2, 2, 1>(args, s); }
 bool launch_jkc_2221(const JKArgs& args, hipStream_t s) { return launch_jk_coop_t<2, 2, 2, 1>(args, s); }
 bool launch_cpc_2221(const CouplingArgs& args, hipStream_t s) { return launch_cp_coop_t<2, 2, 2, 1>(args, s); }
 void coop_attr_2221() { coop_attr_t<2, 2, 2, 1>(); }

@@ -7,9 +7,6 @@ namespace lowdin {
 LOWDIN_ERI_CLASS(2, 2, 2, 2)
 #include "c_2222.inc"
 
-void launch_jk_2222(const JKArgs& args, hipStream_t s) { launch_jk_t<2, 2, 2, 2>(args, s); }
-void launch_jks_2222(const JKArgs& args, hipStream_t s) { launch_jk_strip_t<2, 2, 2, 2>(args, s); }
-void launch_cp_2222(const CouplingArgs& args, hipStream_t s) { launch_cp_t<2, 2, 2, 2>(args, s); }
 void launch_schwarz_22(PairInfo* pairs, int npairs, const double* prim, const double* boys, const double* norma, hipStream_t s) { launch_schwarz_t<2, 2>(pairs, npairs, prim, boys, norma, s); }
 bool launch_jkc_2222(const JKArgs& args, hipStream_t s) { return launch_jk_coop_t<2, 2, 2, 2>(args, s); }
 bool launch_cpc_2222(const CouplingArgs& args, hipStream_t s) { return launch_cp_coop_t<2, 2, 2, 2>(args, s); }

@@ -674,14 +674,19 @@ namespace lowdin {
 #include "eri_%(k)s.inc"
 LOWDIN_ERI_CLASS(%(a)d, %(b)d, %(c)d, %(d)d)
 %(coopinc)s
+%(lanefn)s%(schwfn)s%(coopfn)s}  // namespace lowdin
+"""
+
+LANE_FN = """\
 void launch_jk_%(k)s(const JKArgs& args, hipStream_t s) { launch_jk_t<%(a)d, %(b)d, %(c)d, %(d)d>(args, s); }
 void launch_jks_%(k)s(const JKArgs& args, hipStream_t s) { launch_jk_strip_t<%(a)d, %(b)d, %(c)d, %(d)d>(args, s); }
 void launch_cp_%(k)s(const CouplingArgs& args, hipStream_t s) { launch_cp_t<%(a)d, %(b)d, %(c)d, %(d)d>(args, s); }
-%(schwfn)s%(coopfn)s}  // namespace lowdin
 """
 
 # classes with a wave-cooperative J/K kernel (total L >= 5)
 COOP_MIN_L = 5
+# classes without per-lane Fock and coupling kernels (kCoopL of eri_coop.h)
+COOP_ONLY_L = 6
 
 
 STORE_TU = """// Generated by gen_eri.py -- do not edit.
@@ -706,7 +711,7 @@ namespace lowdin {
 #include "eri_%(k)s.inc"
 LOWDIN_ERI_CLASS(%(a)d, %(b)d, %(c)d, %(d)d)
 LOWDIN_G12_CLASS(%(a)d, %(b)d, %(c)d, %(d)d)
-
+%(coopinc)s
 void launch_gjk_%(k)s(const G12Args& args, hipStream_t s) { launch_g12_t<%(a)d, %(b)d, %(c)d, %(d)d>(args, s); }
 void launch_gcp_%(k)s(const G12CouplingArgs& args, hipStream_t s) { launch_g12cp_t<%(a)d, %(b)d, %(c)d, %(d)d>(args, s); }
 }  // namespace lowdin
@@ -779,12 +784,13 @@ def main(outdir):
                       "void coop_attr_%s() { coop_attr_t<%d, %d, %d, %d>(); }\n"
                       % (k, la, lb, lc, ld, k, la, lb, lc, ld, k, la, lb, lc, ld))
         with open(os.path.join(gdir, "k_%s.hip" % k), "w") as fh:
-            fh.write(KERNEL_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k,
+            lane = "" if la + lb + lc + ld >= COOP_ONLY_L else LANE_FN % {"a": la, "b": lb, "c": lc, "d": ld, "k": k}
+            fh.write(KERNEL_TU % {"lanefn": lane, "a": la, "b": lb, "c": lc, "d": ld, "k": k,
                                   "schw": ", Schwarz" if diag else "", "schwfn": schwfn,
                                   "coopnote": ", wave-cooperative J/K and coupling" if coop else "",
                                   "coopinc": coopinc, "coopfn": coopfn})
         with open(os.path.join(gdir, "g_%s.hip" % k), "w") as fh:
-            fh.write(G12_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k})
+            fh.write(G12_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k, "coopinc": coopinc})
         with open(os.path.join(gdir, "s_%s.hip" % k), "w") as fh:
             fh.write(STORE_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k})
         table[k] = {"L": L, "nacc": nacc, "vrr_flops": v.flops, "hrr_flops": h.flops}
@@ -808,9 +814,10 @@ def main(outdir):
              "namespace lowdin {"]
     for (la, lb, lc, ld) in classes:
         k = "%d%d%d%d" % (la, lb, lc, ld)
-        lines.append("void launch_jk_%s(const JKArgs&, hipStream_t);" % k)
-        lines.append("void launch_jks_%s(const JKArgs&, hipStream_t);" % k)
-        lines.append("void launch_cp_%s(const CouplingArgs&, hipStream_t);" % k)
+        if la + lb + lc + ld < COOP_ONLY_L:
+            lines.append("void launch_jk_%s(const JKArgs&, hipStream_t);" % k)
+            lines.append("void launch_jks_%s(const JKArgs&, hipStream_t);" % k)
+            lines.append("void launch_cp_%s(const CouplingArgs&, hipStream_t);" % k)
         lines.append("void launch_st_%s(const StoreArgs&, hipStream_t);" % k)
         lines.append("void launch_cst_%s(const CouplingStoreArgs&, hipStream_t);" % k)
         lines.append("void launch_gjk_%s(const G12Args&, hipStream_t);" % k)
@@ -822,14 +829,15 @@ def main(outdir):
     for (la, lb) in pcs:
         lines.append("void launch_schwarz_%d%d(PairInfo*, int, const double*, const double*, const double*, hipStream_t);"
                      % (la, lb))
+    lane_classes = [c for c in classes if sum(c) < COOP_ONLY_L]
     lines.append("inline bool dispatch_jk(int la, int lb, int lc, int ld, const JKArgs& a, hipStream_t s) {")
     lines.append("  switch (la * 1000 + lb * 100 + lc * 10 + ld) {")
-    for (la, lb, lc, ld) in classes:
+    for (la, lb, lc, ld) in lane_classes:
         lines.append("    case %d: launch_jk_%d%d%d%d(a, s); return true;" % (la * 1000 + lb * 100 + lc * 10 + ld, la, lb, lc, ld))
     lines.append("    default: return false;\n  }\n}")
     lines.append("inline bool dispatch_jk_strip(int la, int lb, int lc, int ld, const JKArgs& a, hipStream_t s) {")
     lines.append("  switch (la * 1000 + lb * 100 + lc * 10 + ld) {")
-    for (la, lb, lc, ld) in classes:
+    for (la, lb, lc, ld) in lane_classes:
         lines.append("    case %d: launch_jks_%d%d%d%d(a, s); return true;" % (la * 1000 + lb * 100 + lc * 10 + ld, la, lb, lc, ld))
     lines.append("    default: return false;\n  }\n}")
     lines.append("// wave-cooperative J/K kernel; false when the class has none or the launch")
@@ -856,7 +864,7 @@ def main(outdir):
     lines.append("    default: return false;\n  }\n}")
     lines.append("inline bool dispatch_cp(int la, int lb, int lc, int ld, const CouplingArgs& a, hipStream_t s) {")
     lines.append("  switch (la * 1000 + lb * 100 + lc * 10 + ld) {")
-    for (la, lb, lc, ld) in classes:
+    for (la, lb, lc, ld) in lane_classes:
         lines.append("    case %d: launch_cp_%d%d%d%d(a, s); return true;" % (la * 1000 + lb * 100 + lc * 10 + ld, la, lb, lc, ld))
     lines.append("    default: return false;\n  }\n}")
     lines.append("inline bool dispatch_store(int la, int lb, int lc, int ld, const StoreArgs& a, hipStream_t s) {")

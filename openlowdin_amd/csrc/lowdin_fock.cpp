@@ -231,10 +231,19 @@ struct Species {
     TaskSet* tasks;
   };
   std::map<uint64_t, CouplingKey> coupling_tasks;  // keyed by the other species' uid
+  struct G12CouplingKey {
+    uint64_t gen_self = 0, gen_other = 0;
+    int nterm = -1;
+    TaskSet* tasks = nullptr;
+  };
+  std::map<uint64_t, G12CouplingKey> g12_coupling_tasks;
 
   DevBuf<double> d_D, d_G, d_Dother, d_R;
   TaskSet store_ts;                  // wavefront tasks of the integral store / transform
   uint64_t store_gen = ~0ull;        // sig_gen the store tasks were built from
+  TaskSet g12_ts;                    // wavefront tasks of the geminal build
+  uint64_t g12_gen = ~0ull;          // sig_gen they were built from
+  int g12_terms = -1;                // geminal terms they were cut for
   DevBuf<double> d_Dn1, d_cvec, d_store, d_Graw1, d_blk;
   lowdin_fock_stats stats{};
   int mixed = 0;            // mixed precision: FP32 quartets below tau
@@ -305,6 +314,7 @@ struct BuildPlan {
 
 Species::~Species() {
   for (auto& kv : coupling_tasks) delete kv.second.tasks;
+  for (auto& kv : g12_coupling_tasks) delete kv.second.tasks;
   delete own;
 }
 
@@ -508,6 +518,29 @@ static void emit_tasks(std::vector<Task>& out, int bra, int j0, int j1, const Pa
     out.push_back(Task{bra, j, k, flags});
     j = k;
   }
+}
+
+// The same with lanes sharing quartets: 64 >> split_units kets per task, a
+// quartet holding (primitive quartets x mult) independent terms.
+static void emit_split_tasks(std::vector<Task>& out, int bra, int nbp, int j0, int j1, const PairInfo* kets, int mult,
+                             int lmax) {
+  for (int j = j0; j < j1;) {
+    const int np = kets[j].nprim;
+    const int e = std::min(j + (64 >> split_units((long)nbp * np * mult, lmax)), j1);
+    int k = j + 1;
+    while (k < e && kets[k].nprim == np) ++k;
+    out.push_back(Task{bra, j, k, 0});
+    j = k;
+  }
+}
+
+// Terms a lane takes in a launch of `units` terms in all: even over about two
+// wavefronts per SIMD, no fewer than pay for a quartet's summation over the
+// lanes, which grows with the angular momentum's accumulators, and no more
+// than a lane's chain should last.
+static int unit_share(double units, int L) {
+  static const int least[9] = {16, 16, 8, 8, 4, 2, 1, 1, 1};
+  return (int)std::max((double)least[L], std::min(512.0, units / 131072.0));
 }
 
 static void sort_by_cost(std::vector<Task>& t, size_t from, const PairInfo* bras, const PairInfo* kets) {
@@ -1520,6 +1553,46 @@ static G12Params make_gem(const double* coefficients, const double* exponents, i
   return g;
 }
 
+// Wavefront tasks of the geminal builds over the quartets of the pair sets
+// A (bras where their class is the larger) and B (null: over A's own, ket <=
+// bra within a class), with lanes sharing quartets.
+static void build_g12_tasks(TaskSet& ts, const PairSet& A, const PairSet* B, int nterm, hipStream_t st) {
+  ts.tasks.clear();
+  ts.launches.clear();
+  for (int ca = 0; ca < kNumPairClasses; ++ca)
+    for (int cb = 0; cb < (B ? kNumPairClasses : ca + 1); ++cb) {
+      const bool a_bra = ca >= cb;
+      const PairSet& X = a_bra ? A : *B;
+      const PairSet& Y = a_bra ? (B ? *B : A) : A;
+      const int cx = a_bra ? ca : cb, cy = a_bra ? cb : ca;
+      const int nx = X.off[cx + 1] - X.off[cx], ny = Y.off[cy + 1] - Y.off[cy];
+      if (nx == 0 || ny == 0) continue;
+      const PairInfo* bras = X.pairs.data() + X.off[cx];
+      const PairInfo* kets = Y.pairs.data() + Y.off[cy];
+      const bool tri = !B && ca == cb;
+      double bp = 0.0, kp = 0.0;
+      for (int i = 0; i < nx; ++i) bp += bras[i].nprim;
+      for (int j = 0; j < ny; ++j) kp += kets[j].nprim;
+      const int L = kPairClassL[cx][0] + kPairClassL[cx][1] + kPairClassL[cy][0] + kPairClassL[cy][1];
+      const int lmax = unit_share((tri ? 0.5 : 1.0) * bp * kp * nterm, L);
+      const size_t from = ts.tasks.size();
+      const bool coop = L >= kCoopDefaultL;   // one wavefront per quartet: a task is a run of kets
+      const int run = (int)std::max(1.0, (tri ? 0.5 : 1.0) * nx * ny / kCoopDefaultWg);
+      for (int i = 0; i < nx; ++i) {
+        const int nk = tri ? i + 1 : ny;
+        if (!coop)
+          emit_split_tasks(ts.tasks, i, bras[i].nprim, 0, nk, kets, nterm, lmax);
+        else
+          for (int j = 0; j < nk; j += run) ts.tasks.push_back(Task{i, j, std::min(j + run, nk), 0});
+      }
+      sort_by_cost(ts.tasks, from, bras, kets);
+      ts.launches.push_back({kPairClassL[cx][0], kPairClassL[cx][1], kPairClassL[cy][0], kPairClassL[cy][1], cx, cy,
+                             a_bra ? 1 : 0, from, ts.tasks.size() - from, coop ? 4 : 0, lmax});
+    }
+  ts.d_tasks.upload(ts.tasks.data(), ts.tasks.size(), st);
+  ts.valid = true;
+}
+
 // dG (n x n) = 0.25 (Graw + Graw^T), Graw the six J/K updates of every
 // quartet of the pair list with the geminal operator (compute_g12_direct,
 // Libint2Iface.cpp:2193-2365: no density screen), enqueued on st.
@@ -1527,7 +1600,12 @@ static void enqueue_g12(Species& s, const double* dD, double* dG, double factor,
                         hipStream_t st, lowdin_fock_stats* stt) {
   Context& c = ctx();
   ensure_sig(s, st);
-  TaskSet& ts = store_taskset(s, st);
+  TaskSet& ts = s.g12_ts;
+  if (!ts.valid || s.g12_gen != s.sig_gen || s.g12_terms != gem.n) {
+    build_g12_tasks(ts, s.sig, nullptr, gem.n, st);
+    s.g12_gen = s.sig_gen;
+    s.g12_terms = gem.n;
+  }
   const int n = s.nbasis;
   double* graw = s.d_Graw1.ensure(std::max<size_t>((size_t)n * n, 1));
   launch_fill_zero(graw, (size_t)n * n, st);
@@ -1548,6 +1626,7 @@ static void enqueue_g12(Species& s, const double* dD, double* dG, double factor,
     g.D = dD;
     g.Graw = graw;
     g.same_class = L.cbra == L.cket ? 1 : 0;
+    g.lmax = L.lmax;
     g.half_factor = 0.5 * factor;
     g.gem = gem;
     if (!dispatch_g12(L.la, L.lb, L.lc, L.ld, g, hs)) throw std::runtime_error("no G12 kernel for class");
@@ -1559,6 +1638,20 @@ static void enqueue_g12(Species& s, const double* dD, double* dG, double factor,
   HIPCHK(hipGetLastError());
 }
 
+// The geminal coupling tasks of species a with b, kept with a like the
+// Coulomb coupling's.
+static TaskSet* g12_coupling_taskset(Species& a, Species& b, int nterm, hipStream_t st) {
+  Species::G12CouplingKey& k = a.g12_coupling_tasks[b.uid];
+  if (k.tasks && k.tasks->valid && k.gen_self == a.generation && k.gen_other == b.generation && k.nterm == nterm)
+    return k.tasks;
+  if (!k.tasks) k.tasks = new TaskSet();
+  build_g12_tasks(*k.tasks, a.all, &b.all, nterm, st);
+  k.gen_self = a.generation;
+  k.gen_other = b.generation;
+  k.nterm = nterm;
+  return k.tasks;
+}
+
 // dRa (n_a x n_a) = G12 coupling on species a from b's density dDb
 // (compute_g12inter_direct, Libint2Iface.cpp:2367-2550; the layout and
 // element sets of the Coulomb coupling), zeroed here, enqueued on st.
@@ -1567,7 +1660,7 @@ static void enqueue_g12_coupling(Species& a, Species& b, const double* dDb, doub
   Context& c = ctx();
   ensure_all(a, st);
   ensure_all(b, st);
-  TaskSet* ts = coupling_taskset(a, b, st);
+  TaskSet* ts = g12_coupling_taskset(a, b, gem.n, st);
   launch_fill_zero(dRa, (size_t)a.nbasis * a.nbasis, st);
   HIPCHK(hipEventRecord(c.fork, st));
   for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
@@ -1599,6 +1692,7 @@ static void enqueue_g12_coupling(Species& a, Species& b, const double* dDb, doub
       g.dbra = dDb;
     }
     ga.gem = gem;
+    ga.lmax = L.lmax;
     if (!dispatch_g12cp(L.la, L.lb, L.lc, L.ld, ga, hs)) throw std::runtime_error("no G12 coupling kernel for class");
     count_tasks(*ts, L, sb.all.pairs.data() + sb.all.off[L.cbra], sk.all.pairs.data() + sk.all.off[L.cket], stt);
   }

@@ -86,6 +86,16 @@ __host__ __device__ inline int split_shift(int nbp, int nkp, int lmax) {
   return ls;
 }
 
+// log2 of the lanes that share a quartet of `units` independent terms, so
+// that none takes more than lmax of them (at most one wavefront; lmax 0: one
+// lane each).  Host and device agree through it: a wavefront's task holds
+// 64 >> split_units kets.
+__host__ __device__ inline int split_units(long units, int lmax) {
+  int ls = 0;
+  while (lmax > 0 && ls < 6 && (units + (1 << ls) - 1) >> ls > lmax) ++ls;
+  return ls;
+}
+
 // Per molecule of a batched symmetrisation: the result of mols[m] of the
 // launch.
 struct SymDesc {
@@ -199,7 +209,7 @@ struct G12Args {
   const double* D;
   double* Graw;
   int same_class;
-  int pad;
+  int lmax;                // split_units: primitive quartets x geminal terms a lane takes
   double half_factor;
   G12Params gem;
 };
@@ -209,6 +219,8 @@ struct G12Args {
 struct G12CouplingArgs {
   CouplingArgs cp;
   G12Params gem;
+  int lmax;                // as G12Args::lmax
+  int pad;
 };
 
 // Raw overlap block <A|B> (row-major, A's components slowest) of two shells
