@@ -675,7 +675,7 @@ __device__ __forceinline__ void jk_strip_body(const JKArgs& a, const Task& t, un
   for (int jr = t.j0; jr < t.j1; jr += nround) {
     // lanes per quartet of this round of kets, from the primitive count of
     // its first ket (the kets come in descending order of it)
-    const int ls = a.lmax > 0 ? split_shift(P.nprim, pairs[M.off[a.cket] + jr].nprim, a.lmax) : 0;
+    const int ls = split_shift(P.nprim, pairs[M.off[a.cket] + jr].nprim, a.lmax);
     nround = (int)blockDim.x >> ls;
     const int j = jr + (tid >> ls), sub = tid & ((1 << ls) - 1);
     if (j >= t.j1) continue;

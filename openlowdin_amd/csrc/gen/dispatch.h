@@ -7,6 +7,7 @@ void launch_jks_0000(const JKArgs&, hipStream_t);
 void launch_cp_0000(const CouplingArgs&, hipStream_t);
 void launch_st_0000(const StoreArgs&, hipStream_t);
 void launch_cst_0000(const CouplingStoreArgs&, hipStream_t);
+void store_attr_0000();
 void launch_gjk_0000(const G12Args&, hipStream_t);
 void launch_gcp_0000(const G12CouplingArgs&, hipStream_t);
 void launch_jk_1000(const JKArgs&, hipStream_t);
@@ -14,6 +15,7 @@ void launch_jks_1000(const JKArgs&, hipStream_t);
 void launch_cp_1000(const CouplingArgs&, hipStream_t);
 void launch_st_1000(const StoreArgs&, hipStream_t);
 void launch_cst_1000(const CouplingStoreArgs&, hipStream_t);
+void store_attr_1000();
 void launch_gjk_1000(const G12Args&, hipStream_t);
 void launch_gcp_1000(const G12CouplingArgs&, hipStream_t);
 void launch_jk_1010(const JKArgs&, hipStream_t);
@@ -21,6 +23,7 @@ void launch_jks_1010(const JKArgs&, hipStream_t);
 void launch_cp_1010(const CouplingArgs&, hipStream_t);
 void launch_st_1010(const StoreArgs&, hipStream_t);
 void launch_cst_1010(const CouplingStoreArgs&, hipStream_t);
+void store_attr_1010();
 void launch_gjk_1010(const G12Args&, hipStream_t);
 void launch_gcp_1010(const G12CouplingArgs&, hipStream_t);
 void launch_jk_1100(const JKArgs&, hipStream_t);
@@ -28,6 +31,7 @@ void launch_jks_1100(const JKArgs&, hipStream_t);
 void launch_cp_1100(const CouplingArgs&, hipStream_t);
 void launch_st_1100(const StoreArgs&, hipStream_t);
 void launch_cst_1100(const CouplingStoreArgs&, hipStream_t);
+void store_attr_1100();
 void launch_gjk_1100(const G12Args&, hipStream_t);
 void launch_gcp_1100(const G12CouplingArgs&, hipStream_t);
 void launch_jk_1110(const JKArgs&, hipStream_t);
@@ -35,6 +39,7 @@ void launch_jks_1110(const JKArgs&, hipStream_t);
 void launch_cp_1110(const CouplingArgs&, hipStream_t);
 void launch_st_1110(const StoreArgs&, hipStream_t);
 void launch_cst_1110(const CouplingStoreArgs&, hipStream_t);
+void store_attr_1110();
 void launch_gjk_1110(const G12Args&, hipStream_t);
 void launch_gcp_1110(const G12CouplingArgs&, hipStream_t);
 void launch_jk_1111(const JKArgs&, hipStream_t);
@@ -42,6 +47,7 @@ void launch_jks_1111(const JKArgs&, hipStream_t);
 void launch_cp_1111(const CouplingArgs&, hipStream_t);
 void launch_st_1111(const StoreArgs&, hipStream_t);
 void launch_cst_1111(const CouplingStoreArgs&, hipStream_t);
+void store_attr_1111();
 void launch_gjk_1111(const G12Args&, hipStream_t);
 void launch_gcp_1111(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2000(const JKArgs&, hipStream_t);
@@ -49,6 +55,7 @@ void launch_jks_2000(const JKArgs&, hipStream_t);
 void launch_cp_2000(const CouplingArgs&, hipStream_t);
 void launch_st_2000(const StoreArgs&, hipStream_t);
 void launch_cst_2000(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2000();
 void launch_gjk_2000(const G12Args&, hipStream_t);
 void launch_gcp_2000(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2010(const JKArgs&, hipStream_t);
@@ -56,6 +63,7 @@ void launch_jks_2010(const JKArgs&, hipStream_t);
 void launch_cp_2010(const CouplingArgs&, hipStream_t);
 void launch_st_2010(const StoreArgs&, hipStream_t);
 void launch_cst_2010(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2010();
 void launch_gjk_2010(const G12Args&, hipStream_t);
 void launch_gcp_2010(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2011(const JKArgs&, hipStream_t);
@@ -63,6 +71,7 @@ void launch_jks_2011(const JKArgs&, hipStream_t);
 void launch_cp_2011(const CouplingArgs&, hipStream_t);
 void launch_st_2011(const StoreArgs&, hipStream_t);
 void launch_cst_2011(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2011();
 void launch_gjk_2011(const G12Args&, hipStream_t);
 void launch_gcp_2011(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2020(const JKArgs&, hipStream_t);
@@ -70,6 +79,7 @@ void launch_jks_2020(const JKArgs&, hipStream_t);
 void launch_cp_2020(const CouplingArgs&, hipStream_t);
 void launch_st_2020(const StoreArgs&, hipStream_t);
 void launch_cst_2020(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2020();
 void launch_gjk_2020(const G12Args&, hipStream_t);
 void launch_gcp_2020(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2100(const JKArgs&, hipStream_t);
@@ -77,6 +87,7 @@ void launch_jks_2100(const JKArgs&, hipStream_t);
 void launch_cp_2100(const CouplingArgs&, hipStream_t);
 void launch_st_2100(const StoreArgs&, hipStream_t);
 void launch_cst_2100(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2100();
 void launch_gjk_2100(const G12Args&, hipStream_t);
 void launch_gcp_2100(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2110(const JKArgs&, hipStream_t);
@@ -84,6 +95,7 @@ void launch_jks_2110(const JKArgs&, hipStream_t);
 void launch_cp_2110(const CouplingArgs&, hipStream_t);
 void launch_st_2110(const StoreArgs&, hipStream_t);
 void launch_cst_2110(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2110();
 void launch_gjk_2110(const G12Args&, hipStream_t);
 void launch_gcp_2110(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2111(const JKArgs&, hipStream_t);
@@ -91,6 +103,7 @@ void launch_jks_2111(const JKArgs&, hipStream_t);
 void launch_cp_2111(const CouplingArgs&, hipStream_t);
 void launch_st_2111(const StoreArgs&, hipStream_t);
 void launch_cst_2111(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2111();
 void launch_gjk_2111(const G12Args&, hipStream_t);
 void launch_gcp_2111(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2111(const JKArgs&, hipStream_t);
@@ -101,6 +114,7 @@ void launch_jks_2120(const JKArgs&, hipStream_t);
 void launch_cp_2120(const CouplingArgs&, hipStream_t);
 void launch_st_2120(const StoreArgs&, hipStream_t);
 void launch_cst_2120(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2120();
 void launch_gjk_2120(const G12Args&, hipStream_t);
 void launch_gcp_2120(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2120(const JKArgs&, hipStream_t);
@@ -108,6 +122,7 @@ bool launch_cpc_2120(const CouplingArgs&, hipStream_t);
 void coop_attr_2120();
 void launch_st_2121(const StoreArgs&, hipStream_t);
 void launch_cst_2121(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2121();
 void launch_gjk_2121(const G12Args&, hipStream_t);
 void launch_gcp_2121(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2121(const JKArgs&, hipStream_t);
@@ -118,6 +133,7 @@ void launch_jks_2200(const JKArgs&, hipStream_t);
 void launch_cp_2200(const CouplingArgs&, hipStream_t);
 void launch_st_2200(const StoreArgs&, hipStream_t);
 void launch_cst_2200(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2200();
 void launch_gjk_2200(const G12Args&, hipStream_t);
 void launch_gcp_2200(const G12CouplingArgs&, hipStream_t);
 void launch_jk_2210(const JKArgs&, hipStream_t);
@@ -125,6 +141,7 @@ void launch_jks_2210(const JKArgs&, hipStream_t);
 void launch_cp_2210(const CouplingArgs&, hipStream_t);
 void launch_st_2210(const StoreArgs&, hipStream_t);
 void launch_cst_2210(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2210();
 void launch_gjk_2210(const G12Args&, hipStream_t);
 void launch_gcp_2210(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2210(const JKArgs&, hipStream_t);
@@ -132,6 +149,7 @@ bool launch_cpc_2210(const CouplingArgs&, hipStream_t);
 void coop_attr_2210();
 void launch_st_2211(const StoreArgs&, hipStream_t);
 void launch_cst_2211(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2211();
 void launch_gjk_2211(const G12Args&, hipStream_t);
 void launch_gcp_2211(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2211(const JKArgs&, hipStream_t);
@@ -139,6 +157,7 @@ bool launch_cpc_2211(const CouplingArgs&, hipStream_t);
 void coop_attr_2211();
 void launch_st_2220(const StoreArgs&, hipStream_t);
 void launch_cst_2220(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2220();
 void launch_gjk_2220(const G12Args&, hipStream_t);
 void launch_gcp_2220(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2220(const JKArgs&, hipStream_t);
@@ -146,6 +165,7 @@ bool launch_cpc_2220(const CouplingArgs&, hipStream_t);
 void coop_attr_2220();
 void launch_st_2221(const StoreArgs&, hipStream_t);
 void launch_cst_2221(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2221();
 void launch_gjk_2221(const G12Args&, hipStream_t);
 void launch_gcp_2221(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2221(const JKArgs&, hipStream_t);
@@ -153,6 +173,7 @@ bool launch_cpc_2221(const CouplingArgs&, hipStream_t);
 void coop_attr_2221();
 void launch_st_2222(const StoreArgs&, hipStream_t);
 void launch_cst_2222(const CouplingStoreArgs&, hipStream_t);
+void store_attr_2222();
 void launch_gjk_2222(const G12Args&, hipStream_t);
 void launch_gcp_2222(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2222(const JKArgs&, hipStream_t);
@@ -222,15 +243,36 @@ inline bool dispatch_jk_coop(int la, int lb, int lc, int ld, const JKArgs& a, hi
   }
 }
 inline bool has_jk_coop(int la, int lb, int lc, int ld) { return la + lb + lc + ld >= 5; }
-// raise the dynamic LDS limit of every wave-cooperative kernel (once per process)
+// raise the dynamic LDS limit of the kernels that may use more (once per process)
 inline void coop_attr_all() {
+  store_attr_0000();
+  store_attr_1000();
+  store_attr_1010();
+  store_attr_1100();
+  store_attr_1110();
+  store_attr_1111();
+  store_attr_2000();
+  store_attr_2010();
+  store_attr_2011();
+  store_attr_2020();
+  store_attr_2100();
+  store_attr_2110();
+  store_attr_2111();
   coop_attr_2111();
+  store_attr_2120();
   coop_attr_2120();
+  store_attr_2121();
   coop_attr_2121();
+  store_attr_2200();
+  store_attr_2210();
   coop_attr_2210();
+  store_attr_2211();
   coop_attr_2211();
+  store_attr_2220();
   coop_attr_2220();
+  store_attr_2221();
   coop_attr_2221();
+  store_attr_2222();
   coop_attr_2222();
 }
 // wave-cooperative coupling kernel; false when the class has none

@@ -8,4 +8,5 @@ LOWDIN_ERI_CLASS(0, 0, 0, 0)
 
 void launch_st_0000(const StoreArgs& args, hipStream_t s) { launch_store_t<0, 0, 0, 0>(args, s); }
 void launch_cst_0000(const CouplingStoreArgs& args, hipStream_t s) { launch_cstore_t<0, 0, 0, 0>(args, s); }
+void store_attr_0000() { store_attr_t<0, 0, 0, 0>(); }
 }  // namespace lowdin

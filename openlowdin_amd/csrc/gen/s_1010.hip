@@ -8,4 +8,5 @@ LOWDIN_ERI_CLASS(1, 0, 1, 0)
 
 void launch_st_1010(const StoreArgs& args, hipStream_t s) { launch_store_t<1, 0, 1, 0>(args, s); }
 void launch_cst_1010(const CouplingStoreArgs& args, hipStream_t s) { launch_cstore_t<1, 0, 1, 0>(args, s); }
+void store_attr_1010() { store_attr_t<1, 0, 1, 0>(); }
 }  // namespace lowdin

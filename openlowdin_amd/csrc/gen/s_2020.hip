@@ -8,4 +8,5 @@ LOWDIN_ERI_CLASS(2, 0, 2, 0)
 
 void launch_st_2020(const StoreArgs& args, hipStream_t s) { launch_store_t<2, 0, 2, 0>(args, s); }
 void launch_cst_2020(const CouplingStoreArgs& args, hipStream_t s) { launch_cstore_t<2, 0, 2, 0>(args, s); }
+void store_attr_2020() { store_attr_t<2, 0, 2, 0>(); }
 }  // namespace lowdin

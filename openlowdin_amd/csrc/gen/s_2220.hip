@@ -5,7 +5,9 @@
 namespace lowdin {
 #include "eri_2220.inc"
 LOWDIN_ERI_CLASS(2, 2, 2, 0)
+#include "c_2220.inc"
 
 void launch_st_2220(const StoreArgs& args, hipStream_t s) { launch_store_t<2, 2, 2, 0>(args, s); }
 void launch_cst_2220(const CouplingStoreArgs& args, hipStream_t s) { launch_cstore_t<2, 2, 2, 0>(args, s); }
+void store_attr_2220() { store_attr_t<2, 2, 2, 0>(); }
 }  // namespace lowdin

@@ -5,7 +5,9 @@
 namespace lowdin {
 #include "eri_2221.inc"
 LOWDIN_ERI_CLASS(2, 2, 2, 1)
+#include "c_2221.inc"
 
 void launch_st_2221(const StoreArgs& args, hipStream_t s) { launch_store_t<2, 2, 2, 1>(args, s); }
 void launch_cst_2221(const CouplingStoreArgs& args, hipStream_t s) { launch_cstore_t<2, 2, 2, 1>(args, s); }
+void store_attr_2221() { store_attr_t<2, 2, 2, 1>(); }
 }  // namespace lowdin

@@ -696,9 +696,10 @@ STORE_TU = """// Generated by gen_eri.py -- do not edit.
 namespace lowdin {
 #include "eri_%(k)s.inc"
 LOWDIN_ERI_CLASS(%(a)d, %(b)d, %(c)d, %(d)d)
-
+%(coopinc)s
 void launch_st_%(k)s(const StoreArgs& args, hipStream_t s) { launch_store_t<%(a)d, %(b)d, %(c)d, %(d)d>(args, s); }
 void launch_cst_%(k)s(const CouplingStoreArgs& args, hipStream_t s) { launch_cstore_t<%(a)d, %(b)d, %(c)d, %(d)d>(args, s); }
+void store_attr_%(k)s() { store_attr_t<%(a)d, %(b)d, %(c)d, %(d)d>(); }
 }  // namespace lowdin
 """
 
@@ -792,7 +793,7 @@ def main(outdir):
         with open(os.path.join(gdir, "g_%s.hip" % k), "w") as fh:
             fh.write(G12_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k, "coopinc": coopinc})
         with open(os.path.join(gdir, "s_%s.hip" % k), "w") as fh:
-            fh.write(STORE_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k})
+            fh.write(STORE_TU % {"a": la, "b": lb, "c": lc, "d": ld, "k": k, "coopinc": coopinc})
         table[k] = {"L": L, "nacc": nacc, "vrr_flops": v.flops, "hrr_flops": h.flops}
     incs, cases, sizes = [], [], []
     for cl in classes:
@@ -820,6 +821,7 @@ def main(outdir):
             lines.append("void launch_cp_%s(const CouplingArgs&, hipStream_t);" % k)
         lines.append("void launch_st_%s(const StoreArgs&, hipStream_t);" % k)
         lines.append("void launch_cst_%s(const CouplingStoreArgs&, hipStream_t);" % k)
+        lines.append("void store_attr_%s();" % k)
         lines.append("void launch_gjk_%s(const G12Args&, hipStream_t);" % k)
         lines.append("void launch_gcp_%s(const G12CouplingArgs&, hipStream_t);" % k)
         if la + lb + lc + ld >= COOP_MIN_L:
@@ -849,9 +851,10 @@ def main(outdir):
             lines.append("    case %d: return launch_jkc_%d%d%d%d(a, s);" % (la * 1000 + lb * 100 + lc * 10 + ld, la, lb, lc, ld))
     lines.append("    default: return false;\n  }\n}")
     lines.append("inline bool has_jk_coop(int la, int lb, int lc, int ld) { return la + lb + lc + ld >= %d; }" % COOP_MIN_L)
-    lines.append("// raise the dynamic LDS limit of every wave-cooperative kernel (once per process)")
+    lines.append("// raise the dynamic LDS limit of the kernels that may use more (once per process)")
     lines.append("inline void coop_attr_all() {")
     for (la, lb, lc, ld) in classes:
+        lines.append("  store_attr_%d%d%d%d();" % (la, lb, lc, ld))
         if la + lb + lc + ld >= COOP_MIN_L:
             lines.append("  coop_attr_%d%d%d%d();" % (la, lb, lc, ld))
     lines.append("}")

@@ -177,7 +177,7 @@ struct PairSet {
   DevBuf<PairInfo> d_pairs;
   DevBuf<double> d_prims;
   DevBuf<float> d_primsf;           // the same records in FP32
-  DevBuf<int> d_pidx;               // nshell x nshell: pair of (sa, sb), -1 if none
+  DevBuf<int> d_pidx;               // nshell x nshell: pair of (sa, sb), -1 if none; then the shell of each function
   int jpoff[kNumPairClasses + 1] = {0};   // MolDesc::jpoff
   int maxprim = 0;                  // most primitive pairs of a pair
   bool q_ready = false;
@@ -219,7 +219,6 @@ struct Species {
   uint64_t dev_generation = ~0ull;
   DevBuf<ShellInfo> d_shells;
   DevBuf<double> d_pexp, d_pcoef, d_norma;
-  DevBuf<int> d_fsh;
 
   PairSet sig;        // significant pairs (intra builds), with Q
   PairSet all;        // every s1 <= s2 pair (coupling builds)
@@ -239,12 +238,16 @@ struct Species {
   std::map<uint64_t, G12CouplingKey> g12_coupling_tasks;
 
   DevBuf<double> d_D, d_G, d_Dother, d_R;
-  TaskSet store_ts;                  // wavefront tasks of the integral store / transform
+  TaskSet store_ts;                  // wavefront tasks of the integral store
   uint64_t store_gen = ~0ull;        // sig_gen the store tasks were built from
+  TaskSet it_ts;                     // workgroup tasks of the transform
+  uint64_t it_gen = ~0ull;
+  DevBuf<double> d_slab;             // transform: packed slabs on their way out
+  DevBuf<int> d_slot;                // where (k, l) lies in a packed slab
   TaskSet g12_ts;                    // wavefront tasks of the geminal build
   uint64_t g12_gen = ~0ull;          // sig_gen they were built from
   int g12_terms = -1;                // geminal terms they were cut for
-  DevBuf<double> d_Dn1, d_cvec, d_store, d_Graw1, d_blk;
+  DevBuf<double> d_Dn1, d_cvec, d_store, d_Graw1;
   lowdin_fock_stats stats{};
   int mixed = 0;            // mixed precision: FP32 quartets below tau
   int sig_mixed = 0;        // the precision mode the pair order of sig was chosen for
@@ -333,7 +336,6 @@ static void ensure_device_basis(Species& s, hipStream_t st) {
   s.d_pexp.upload(s.pexp.data(), s.pexp.size(), st);
   s.d_pcoef.upload(s.pcoef.data(), s.pcoef.size(), st);
   s.d_norma.upload(s.norma.data(), s.norma.size(), st);
-  s.d_fsh.upload(s.fsh.data(), s.fsh.size(), st);
   s.dev_generation = s.generation;
 }
 
@@ -436,7 +438,7 @@ static uint64_t morton_key(const double* P, const double* lo) {
 // Rewrites the primitive-pair records in that order.
 // Also lays out the packed density and J blocks of the pairs and the map from
 // shells to pairs (of this order).
-static void resort_by_q(PairSet& ps, int nshell, hipStream_t st, bool by_q) {
+static void resort_by_q(PairSet& ps, int nshell, const std::vector<int>& fsh, hipStream_t st, bool by_q) {
   std::vector<size_t> idx(ps.pairs.size());
   for (size_t k = 0; k < idx.size(); ++k) idx[k] = k;
   double lo[3] = {1e300, 1e300, 1e300};
@@ -480,6 +482,7 @@ static void resort_by_q(PairSet& ps, int nshell, hipStream_t st, bool by_q) {
   ps.maxprim = 0;
   for (const PairInfo& P : ps.pairs) ps.maxprim = std::max(ps.maxprim, P.nprim);
   for (size_t k = 0; k < ps.pairs.size(); ++k) pidx[(size_t)ps.pairs[k].sa * nshell + ps.pairs[k].sb] = (int)k;
+  pidx.insert(pidx.end(), fsh.begin(), fsh.end());
   ps.d_pidx.upload(pidx.data(), pidx.size(), st);
   for (int c = 0; c < kNumPairClasses; ++c)
     ps.jpoff[c + 1] = ps.jpoff[c] + (ps.off[c + 1] - ps.off[c]) * ncart_h(kPairClassL[c][0]) * ncart_h(kPairClassL[c][1]);
@@ -598,10 +601,84 @@ static void ensure_sig(Species& s, hipStream_t st) {
   if (!s.sig.valid) {
     build_pairset(s, s.pairlist, s.sig, st);
     compute_schwarz(s.sig, s.d_norma.p, st);
-    resort_by_q(s.sig, (int)s.shells.size(), st, s.mixed != 0);
+    resort_by_q(s.sig, (int)s.shells.size(), s.fsh, st, s.mixed != 0);
     s.sig_mixed = s.mixed;
     s.sig_gen++;
   }
+}
+
+// Cuts a bra's ket range into workgroup tasks of about equal estimated cost
+// (kets of one list, in runs of equal primitive counts).
+struct KetRun {
+  int j0, j1, np;
+};
+static std::vector<KetRun> ket_runs(const PairInfo* kets, int count) {
+  std::vector<KetRun> r;
+  for (int j = 0; j < count; ++j) {
+    if (r.empty() || r.back().np != kets[j].nprim) r.push_back(KetRun{j, j, kets[j].nprim});
+    r.back().j1 = j + 1;
+  }
+  return r;
+}
+class KetCutter {
+ public:
+  KetCutter(const std::vector<KetRun>& runs, int lmax, int block, double cap)
+      : kr(runs), lmax(lmax), block(block), cap(cap), unit(runs.size()), upto(runs.size()), round(runs.size()) {}
+  // the kets [0, nk) of bra i, which has nbp primitive pairs; nk > 0
+  void cut(std::vector<std::pair<double, Task>>& out, int i, int nbp, int nk, int flags) {
+    if (nbp != last) {   // per-run costs of this primitive count
+      double c = 0.0;
+      for (size_t r = 0; r < kr.size(); ++r) {
+        const int ls = split_shift(nbp, kr[r].np, lmax);
+        unit[r] = (double)nbp * kr[r].np + kQuartetIters * (double)(1 << ls);
+        round[r] = block >> ls;
+        upto[r] = c;
+        c += unit[r] * (kr[r].j1 - kr[r].j0);
+      }
+      last = nbp;
+    }
+    while (kr[rk].j1 < nk) ++rk;   // the run of the last ket
+    while (kr[rk].j0 >= nk) --rk;
+    const double all = upto[rk] + unit[rk] * (nk - kr[rk].j0);
+    if (all <= cap) {
+      out.push_back({all, Task{i, 0, nk, flags}});
+      return;
+    }
+    // pieces cut at whole rounds of the workgroup
+    const double share = all / std::ceil(all / cap) * (1.0 - 1e-9);
+    double acc = 0.0;
+    int j0 = 0;
+    for (size_t r = 0; r <= rk; ++r) {
+      const int end = std::min(kr[r].j1, nk);
+      for (int j = kr[r].j0; j < end;) {
+        const int want = (int)std::min(1e9, std::ceil((share - acc) / unit[r]));
+        const int take = std::min(end - j, std::max(1, (want + round[r] - 1) / round[r]) * round[r]);
+        acc += take * unit[r];
+        j += take;
+        if (acc >= share || j == nk) {
+          out.push_back({acc, Task{i, j0, j, flags}});
+          j0 = j;
+          acc = 0.0;
+        }
+      }
+    }
+  }
+
+ private:
+  const std::vector<KetRun>& kr;
+  int lmax, block;
+  double cap;
+  std::vector<double> unit, upto;   // per run: cost of a quartet, cost of the kets before it
+  std::vector<int> round;           // kets a workgroup takes at once
+  int last = -1;
+  size_t rk = 0;
+};
+
+// Appends the tasks made, most expensive first.
+static void append_by_cost(std::vector<Task>& tasks, std::vector<std::pair<double, Task>>& made) {
+  std::stable_sort(made.begin(), made.end(),
+                   [](const std::pair<double, Task>& x, const std::pair<double, Task>& y) { return x.first > y.first; });
+  for (const auto& t : made) tasks.push_back(t.second);
 }
 
 // Whether a plan runs as one launch over all quartet classes.
@@ -648,26 +725,15 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
   std::vector<std::pair<double, Task>> made;   // tasks of the launch at hand with their estimated costs
   // runs of kets with equal primitive counts and the primitive counts summed
   // up to each ket, per molecule and pair class
-  struct Run {
-    int j0, j1, np;
-  };
-  std::vector<std::array<std::vector<Run>, kNumPairClasses>> runs(nm);
+  std::vector<std::array<std::vector<KetRun>, kNumPairClasses>> runs(nm);
   std::vector<std::vector<double>> psum(nm);
   for (int m = 0; m < nm; ++m) {
     const PairSet& ps = p.mols[m]->sig;
     psum[m].assign(ps.pairs.size() + 1, 0.0);
-    for (int c = 0; c < kNumPairClasses; ++c)
-      for (int k = ps.off[c]; k < ps.off[c + 1]; ++k) {
-        std::vector<Run>& r = runs[m][c];
-        const int j = k - ps.off[c];
-        if (r.empty() || r.back().np != ps.pairs[k].nprim) r.push_back(Run{j, j, ps.pairs[k].nprim});
-        r.back().j1 = j + 1;
-        psum[m][k + 1] = psum[m][k] + ps.pairs[k].nprim;
-      }
+    for (size_t k = 0; k < ps.pairs.size(); ++k) psum[m][k + 1] = psum[m][k] + ps.pairs[k].nprim;
+    for (int c = 0; c < kNumPairClasses; ++c) runs[m][c] = ket_runs(ps.pairs.data() + ps.off[c], ps.off[c + 1] - ps.off[c]);
   }
   p.fused = want_fused(p);
-  std::vector<double> unit, upto;   // per run: cost of a quartet, cost of the kets before the run
-  std::vector<int> round;           // per run: kets a workgroup takes at once
   for (int id = 0; id < kNumClassPairs; ++id) {
     // one launch starts its workgroups in task order: the classes with the
     // longest chains (high angular momentum) first
@@ -731,12 +797,7 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
       const int nx = ps.off[cx + 1] - ps.off[cx], ny = ps.off[cy + 1] - ps.off[cy];
       if (nx == 0 || ny == 0) continue;
       const PairInfo* kets = ps.pairs.data() + ps.off[cy];
-      const std::vector<Run>& kr = runs[m][cy];
-      unit.resize(kr.size());
-      upto.resize(kr.size());
-      round.resize(kr.size());
-      int last = -1;   // primitive count of the bra the per-run costs are for
-      size_t rk = 0;
+      KetCutter cutter(runs[m][cy], lmax, block, cap);
       for (int i = 0; i < nx; ++i) {
         const int nk = (cx == cy) ? i + 1 : ny, nbp = ps.pairs[ps.off[cx] + i].nprim;
         if (coop) {
@@ -746,44 +807,7 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
             if (j1 > j0) made.push_back({(double)nbp * kets[j0].nprim * (j1 - j0), Task{i, j0, j1, m}});
           }
         } else if (strip) {
-          // pieces of about equal cost, cut at whole rounds of the workgroup
-          if (nbp != last) {
-            double c = 0.0;
-            for (size_t r = 0; r < kr.size(); ++r) {
-              const int ls = split_shift(nbp, kr[r].np, lmax);
-              unit[r] = (double)nbp * kr[r].np + kQuartetIters * (double)(1 << ls);
-              round[r] = block >> ls;
-              upto[r] = c;
-              c += unit[r] * (kr[r].j1 - kr[r].j0);
-            }
-            last = nbp;
-            rk = 0;
-          }
-          if (cx != cy) rk = kr.size() - 1;
-          while (kr[rk].j1 < nk) ++rk;   // the run of the last ket
-          while (kr[rk].j0 >= nk) --rk;
-          const double all = upto[rk] + unit[rk] * (nk - kr[rk].j0);
-          if (all <= cap) {
-            made.push_back({all, Task{i, 0, nk, m}});
-            continue;
-          }
-          const double share = all / std::ceil(all / cap) * (1.0 - 1e-9);
-          double acc = 0.0;
-          int j0 = 0;
-          for (size_t r = 0; r <= rk; ++r) {
-            const int end = std::min(kr[r].j1, nk);
-            for (int j = kr[r].j0; j < end;) {
-              const int want = (int)std::min(1e9, std::ceil((share - acc) / unit[r]));
-              const int take = std::min(end - j, std::max(1, (want + round[r] - 1) / round[r]) * round[r]);
-              acc += take * unit[r];
-              j += take;
-              if (acc >= share || j == nk) {
-                made.push_back({acc, Task{i, j0, j, m}});
-                j0 = j;
-                acc = 0.0;
-              }
-            }
-          }
+          cutter.cut(made, i, nbp, nk, m);
         } else {
           const size_t at = ts.tasks.size();
           emit_tasks(ts.tasks, i, 0, nk, kets, m);
@@ -795,9 +819,7 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
         }
       }
     }
-    std::stable_sort(made.begin(), made.end(),
-                     [](const std::pair<double, Task>& x, const std::pair<double, Task>& y) { return x.first > y.first; });
-    for (const auto& t : made) ts.tasks.push_back(t.second);
+    append_by_cost(ts.tasks, made);
     ts.launches.push_back({la, lb, lc, ld, cx, cy, 1, from, ts.tasks.size() - from,
                            coop ? coop : (strip ? (wave64 ? 2 : 1) : 0), lmax});
     // estimated cost of the launch: primitive quartets x class weight
@@ -1051,7 +1073,7 @@ static void fill_desc(MolDesc& M, const Species& s, double factor) {
   M.shells = s.d_shells.p;
   M.norma = s.d_norma.p;
   M.pidx = s.sig.d_pidx.p;
-  M.fsh = s.d_fsh.p;
+  M.fsh = s.sig.d_pidx.p + s.shells.size() * s.shells.size();
   for (int k = 0; k <= kNumPairClasses; ++k) {
     M.off[k] = s.sig.off[k];
     M.jpoff[k] = s.sig.jpoff[k];
@@ -1374,49 +1396,70 @@ static void compute_coupling(Species& a, Species* b, const double* db, double* r
 }
 
 // ------------------------------------------ integral store / first-quarter transform
-// Wavefront tasks over the significant pairs of one species: the quartet
-// set of the Fock build (bra class >= ket class, ket <= bra within a class).
-static TaskSet& store_taskset(Species& s, hipStream_t st) {
-  TaskSet& ts = s.store_ts;
-  if (ts.valid && s.store_gen == s.sig_gen) return ts;
+// Tasks over the significant pairs of one species: the quartet set of the
+// Fock build (bra class >= ket class, ket <= bra within a class).  Store
+// (mode 0): wavefronts of one bra and up to 64 kets, fewer where lanes share
+// quartets; transform (mode 1): workgroups of one bra and a run of kets, as
+// the Fock build's strips.  From L = kCoopDefaultL up one wavefront per
+// quartet, a task being a run of kets.
+static TaskSet& store_taskset(Species& s, int mode, hipStream_t st) {
+  TaskSet& ts = mode == 0 ? s.store_ts : s.it_ts;
+  uint64_t& gen = mode == 0 ? s.store_gen : s.it_gen;
+  if (ts.valid && gen == s.sig_gen) return ts;
   ts.tasks.clear();
   ts.launches.clear();
   const PairSet& ps = s.sig;
-  for (int cx = 0; cx < kNumPairClasses; ++cx)
-    for (int cy = 0; cy <= cx; ++cy) {
+  std::vector<std::pair<double, Task>> made;
+  for (int cx = kNumPairClasses - 1; cx >= 0; --cx)   // longest chains first
+    for (int cy = cx; cy >= 0; --cy) {
       const int nx = ps.off[cx + 1] - ps.off[cx], ny = ps.off[cy + 1] - ps.off[cy];
       if (nx == 0 || ny == 0) continue;
+      const PairInfo* bras = ps.pairs.data() + ps.off[cx];
       const PairInfo* kets = ps.pairs.data() + ps.off[cy];
+      const int la = kPairClassL[cx][0], lb = kPairClassL[cx][1], lc = kPairClassL[cy][0], ld = kPairClassL[cy][1];
+      const bool tri = cx == cy, coop = la + lb + lc + ld >= kCoopDefaultL;
+      const double total = tri ? 0.5 * nx * (nx + 1.0) : (double)nx * ny;
       const size_t from = ts.tasks.size();
-      for (int i = 0; i < nx; ++i) emit_tasks(ts.tasks, i, 0, cx == cy ? i + 1 : ny, kets, 0);
-      sort_by_cost(ts.tasks, from, ps.pairs.data() + ps.off[cx], kets);
-      ts.launches.push_back({kPairClassL[cx][0], kPairClassL[cx][1], kPairClassL[cy][0], kPairClassL[cy][1], cx, cy,
-                             1, from, ts.tasks.size() - from, 0});
+      const bool wave64 = total < 192.0 * nx;
+      const int block = wave64 ? 64 : 256;
+      const int lmax = (int)(mode == 0 ? kSplitMin : std::max(kSplitMin, std::min(kSplitMax, total / (kSplitKets * nx))));
+      const int run = (int)std::max(1.0, total / kCoopDefaultWg);
+      double bp = 0.0, kp = 0.0;
+      for (int i = 0; i < nx; ++i) bp += bras[i].nprim;
+      for (int j = 0; j < ny; ++j) kp += kets[j].nprim;
+      const double work = (tri ? 0.5 : 1.0) * bp * kp + kQuartetIters * total;
+      // rows of n summed in LDS and flushed by every workgroup
+      const double flush = 8.0 + (double)(ncart_h(la) * ncart_h(lb)) * s.nbasis / block;
+      const std::vector<KetRun> runs = ket_runs(kets, ny);
+      KetCutter cutter(runs, lmax, block, std::max(work / (wave64 ? 2048.0 : 512.0), 4.0 * block * flush));
+      made.clear();
+      for (int i = 0; i < nx; ++i) {
+        const int nk = tri ? i + 1 : ny, nbp = bras[i].nprim;
+        if (coop) {
+          for (int j = 0; j < nk; j += run) {
+            const int e = std::min(j + run, nk);
+            made.push_back({(double)nbp * kets[j].nprim * (e - j), Task{i, j, e, 0}});
+          }
+        } else if (mode == 1) {
+          cutter.cut(made, i, nbp, nk, 0);
+        } else {
+          for (int j = 0; j < nk;) {
+            const int np = kets[j].nprim, e = std::min(j + (64 >> split_shift(nbp, np, lmax)), nk);
+            int k = j + 1;
+            while (k < e && kets[k].nprim == np) ++k;
+            made.push_back({(double)nbp * np * (k - j), Task{i, j, k, 0}});
+            j = k;
+          }
+        }
+      }
+      append_by_cost(ts.tasks, made);
+      ts.launches.push_back({la, lb, lc, ld, cx, cy, 1, from, ts.tasks.size() - from,
+                             coop ? 4 : (mode == 1 ? (wave64 ? 2 : 1) : 0), lmax});
     }
   ts.d_tasks.upload(ts.tasks.data(), ts.tasks.size(), st);
   ts.valid = true;
-  s.store_gen = s.sig_gen;
+  gen = s.sig_gen;
   return ts;
-}
-
-// Launch one store class; the classes whose raw block is staged in HBM
-// (kStoreStagedNQ integrals per quartet) go in chunks of kStoreStagedTasks
-// tasks over the species' staging buffer, one after another on hs.
-template <typename Args, typename Dispatch>
-static void launch_store_class(const TaskSet::Launch& L, Args g, Species& s, hipStream_t hs, Dispatch dispatch) {
-  const int nq = ncart_h(L.la) * ncart_h(L.lb) * ncart_h(L.lc) * ncart_h(L.ld);
-  if (nq < kStoreStagedNQ) {
-    if (!dispatch(L.la, L.lb, L.lc, L.ld, g, hs)) throw std::runtime_error("no store kernel for class");
-    return;
-  }
-  const Task* tasks = g.tasks;
-  const int ntasks = g.ntasks;
-  g.blk = s.d_blk.ensure((size_t)kStoreStagedTasks * 64 * nq);
-  for (int t0 = 0; t0 < ntasks; t0 += kStoreStagedTasks) {
-    g.tasks = tasks + t0;
-    g.ntasks = std::min(kStoreStagedTasks, ntasks - t0);
-    if (!dispatch(L.la, L.lb, L.lc, L.ld, g, hs)) throw std::runtime_error("no store kernel for class");
-  }
 }
 
 // Candidate quartets / ERIs of a task range (before the density screen).
@@ -1433,25 +1476,31 @@ static void count_tasks(const TaskSet& ts, const TaskSet::Launch& L, const PairI
   }
 }
 
+constexpr size_t kSlabStage = 32u << 20;   // doubles (256 MB) of packed slabs unpacked at once
+
 // Intra-species integral store (mode 0: dOut = A, n^4, only kept elements
-// written) or first-quarter transform (mode 1: dOut = GG, n^3, zeroed,
-// accumulated and mirrored here; dC = row p of the coefficients), enqueued
+// written) or first-quarter transform (mode 1: dOut = GG, n^3, accumulated in
+// packed slabs and spread over both triangles here; dC = row p of the coefficients), enqueued
 // on st from the device density dD (its block norms drive the screen).
 static void enqueue_store(Species& s, const double* dD, const double* dC, double* dOut, int mode, hipStream_t st,
                           lowdin_fock_stats* stt) {
   Context& c = ctx();
   ensure_sig(s, st);
-  TaskSet& ts = store_taskset(s, st);
+  TaskSet& ts = store_taskset(s, mode, st);
   const int n = s.nbasis, ns = (int)s.shells.size();
+  const int np = s.sig.jpoff[kNumPairClasses];   // values of a packed slab
   const bool screen = s.is_electron;
   if (screen) launch_dnorm(dD, n, s.d_shells.p, ns, s.d_Dn1.ensure((size_t)ns * ns), st);
-  if (mode == 1) launch_fill_zero(dOut, (size_t)n * n * n, st);
+  if (mode == 1) {
+    launch_clear_slabs(dOut, n, np, st);
+    launch_slab_slots(s.d_slot.ensure((size_t)n * n), s.sig.d_pairs.p, s.sig.d_pidx.p,
+                      s.sig.d_pidx.p + (size_t)ns * ns, n, ns, s.sig.off, s.sig.jpoff, st);
+  }
   HIPCHK(hipEventRecord(c.fork, st));
   for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
-  size_t nlight = 0;
+  size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts.launches) {
-    // scratch-heavy classes on side stream 0, the others round robin over 1..3
-    hipStream_t hs = heavy_launch(L) ? c.side[0] : c.side[1 + nlight++ % (kSideStreams - 1)];
+    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
     StoreArgs g{};
     g.tasks = ts.d_tasks.p + L.off;
     g.ntasks = (int)L.count;
@@ -1468,14 +1517,27 @@ static void enqueue_store(Species& s, const double* dD, const double* dC, double
     g.same_class = L.cbra == L.cket ? 1 : 0;
     g.screen = screen ? 1 : 0;
     g.mode = mode;
+    g.lmax = L.lmax;
+    g.block = L.strip == 2 ? 64 : 256;
+    g.nbra = s.sig.off[L.cbra + 1] - s.sig.off[L.cbra];
+    g.nket = s.sig.off[L.cket + 1] - s.sig.off[L.cket];
+    g.bpk = s.sig.jpoff[L.cbra];
+    g.kpk = s.sig.jpoff[L.cket];
     g.eps = 2.220446049250313080847e-16;  // DBL_EPSILON, Libint2Iface.h:273-274, 316-317
     g.drop = 1.0e-10;                      // Libint2Iface.cpp:794, 2701
-    launch_store_class(L, g, s, hs, dispatch_store);
+    if (!dispatch_store(L.la, L.lb, L.lc, L.ld, g, hs)) throw std::runtime_error("no store kernel for class");
     count_tasks(ts, L, s.sig.pairs.data() + s.sig.off[L.cbra], s.sig.pairs.data() + s.sig.off[L.cket], stt);
   }
   HIPCHK(hipGetLastError());
   join_side_streams(st);
-  if (mode == 1) launch_mirror_upper(dOut, n, n, st);
+  if (mode == 1) {
+    // spread the slabs over both triangles, as many at a time as fit in the
+    // staging buffer
+    const int step = (int)std::max<size_t>(1, std::min<size_t>(n, kSlabStage / std::max(np, 1)));
+    double* tmp = s.d_slab.ensure(std::max<size_t>((size_t)step * np, 1));
+    for (int j0 = 0; j0 < n; j0 += step)
+      launch_unpack_slabs(dOut, tmp, s.d_slot.p, n, np, j0, std::min(step, n - j0), st);
+  }
   HIPCHK(hipGetLastError());
 }
 
@@ -1503,9 +1565,9 @@ static void enqueue_coupling_store(Species& a, Species& b, const double* dC, dou
   if (mode == 1) launch_fill_zero(dOut, na * nb * nb, st);
   HIPCHK(hipEventRecord(c.fork, st));
   for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
-  size_t nlight = 0;
+  size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts->launches) {
-    hipStream_t hs = heavy_launch(L) ? c.side[0] : c.side[1 + nlight++ % (kSideStreams - 1)];
+    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
     const bool a_bra = L.bra_is_a != 0;
     Species& sb = a_bra ? a : b;
     Species& sk = a_bra ? b : a;
@@ -1529,7 +1591,7 @@ static void enqueue_coupling_store(Species& a, Species& b, const double* dC, dou
     g.sx2 = nb * nb;
     g.sy1 = nb;
     g.drop = 1.0e-10;  // Libint2Iface.cpp:1456, 2865
-    launch_store_class(L, g, a, hs, dispatch_cstore);
+    if (!dispatch_cstore(L.la, L.lb, L.lc, L.ld, g, hs)) throw std::runtime_error("no store kernel for class");
     count_tasks(*ts, L, sb.all.pairs.data() + sb.all.off[L.cbra], sk.all.pairs.data() + sk.all.off[L.cket], stt);
   }
   HIPCHK(hipGetLastError());
@@ -1611,10 +1673,9 @@ static void enqueue_g12(Species& s, const double* dD, double* dG, double factor,
   launch_fill_zero(graw, (size_t)n * n, st);
   HIPCHK(hipEventRecord(c.fork, st));
   for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
-  size_t nlight = 0;
+  size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts.launches) {
-    // scratch-heavy classes on side stream 0, the others round robin over 1..3
-    hipStream_t hs = heavy_launch(L) ? c.side[0] : c.side[1 + nlight++ % (kSideStreams - 1)];
+    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
     G12Args g{};
     g.tasks = ts.d_tasks.p + L.off;
     g.ntasks = (int)L.count;
@@ -1664,9 +1725,9 @@ static void enqueue_g12_coupling(Species& a, Species& b, const double* dDb, doub
   launch_fill_zero(dRa, (size_t)a.nbasis * a.nbasis, st);
   HIPCHK(hipEventRecord(c.fork, st));
   for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
-  size_t nlight = 0;
+  size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts->launches) {
-    hipStream_t hs = heavy_launch(L) ? c.side[0] : c.side[1 + nlight++ % (kSideStreams - 1)];
+    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
     const bool a_bra = L.bra_is_a != 0;
     Species& sb = a_bra ? a : b;
     Species& sk = a_bra ? b : a;

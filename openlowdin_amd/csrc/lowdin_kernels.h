@@ -79,10 +79,10 @@ void launch_jk_fused(const FusedArgs& a, hipStream_t s);
 
 // log2 of the lanes that share a quartet of nbp x nkp primitive pairs: as few
 // as bring the serial loop of a lane down to lmax primitive quartets, at most
-// one wavefront and no more than the ket has primitive pairs.
+// one wavefront and no more than the ket has primitive pairs (lmax 0: one).
 __host__ __device__ inline int split_shift(int nbp, int nkp, int lmax) {
   int ls = 0;
-  while (ls < 6 && (1 << ls) < nkp && nbp * ((nkp + (1 << ls) - 1) >> ls) > lmax) ++ls;
+  while (lmax > 0 && ls < 6 && (1 << ls) < nkp && nbp * ((nkp + (1 << ls) - 1) >> ls) > lmax) ++ls;
   return ls;
 }
 
@@ -121,21 +121,12 @@ struct CouplingArgs {
   double drop;             // raw-integral drop (1e-10)
 };
 
-// Store kernels of classes with at least this many integrals per quartet
-// ((dd|dd)) keep the raw block in a buffer in HBM owned by the library (one
-// block per launched thread, StoreArgs::blk) instead of private memory, so
-// that their private segment stays within that of the Fock-build kernels;
-// launches of those classes are split into chunks of at most this many
-// tasks (256 tasks: 16384 threads, 170 MB of staging).
-constexpr int kStoreStagedNQ = 1296;
-constexpr int kStoreStagedTasks = 256;
-
 // Integral store (mode 0) or first-quarter transform (mode 1) over the
 // intra-species quartets of one species.
 //   mode 0: A[i][j][k][l] (n^4) = (ij|kl) * norma^4 for |raw| > drop, all
 //           eight index images; other elements are left as they are.
-//   mode 1: GG[j][k][l] (n^3) += sum_i c[i] (ij|kl), k <= l only (the other
-//           triangle is mirrored afterwards); GG must start at zero.
+//   mode 1: GG[j][k][l] (n^3) += sum_i c[i] (ij|kl), each slab j packed by
+//           shell pair (launch_clear_slabs before, launch_unpack_slabs after).
 struct StoreArgs {
   const Task* tasks;
   int ntasks;
@@ -147,12 +138,16 @@ struct StoreArgs {
   const double* c;         // mode 1: row p of the coefficient matrix (n)
   double* out;
   const double* boys;
-  double* blk;             // classes with kStoreStagedNQ integrals per block: one raw block per thread
   int n;
   int nshell;
   int same_class;          // bra and ket lists are the same class list
   int screen;              // Dnorm * Q * Q < eps screen (electrons)
   int mode;
+  int lmax;                // split_shift: primitive quartets a lane takes
+  int block;               // mode 1: threads per workgroup
+  int nbra, nket;          // mode 1: pairs of the bra and ket classes
+  int bpk, kpk;            // mode 1: their offsets in a packed slab
+  int row0, rows;          // mode 1: rows (a b) this pass sums in LDS (set by the launcher)
   int pad;
   double eps;
   double drop;             // kept if |raw| > drop
@@ -176,10 +171,10 @@ struct CouplingStoreArgs {
   const double* c;         // mode 1: row p of T's coefficient matrix
   double* out;
   const double* boys;
-  double* blk;             // as StoreArgs::blk
   int bra_is_x;            // mode 0: bra pair belongs to X
   int bra_is_t;            // mode 1: bra pair belongs to T
   int mode;
+  int lmax;                // as StoreArgs::lmax
   int n_o;                 // mode 1: basis size of O
   size_t sx1, sx2, sy1;    // mode 0 strides
   double drop;             // dropped if |raw| < drop
@@ -291,6 +286,14 @@ void launch_absmax(const double* x, size_t n, double* out, hipStream_t s);
 void launch_scale_cols(double* X, const double* U, const double* w, int n, int m, int col0, hipStream_t s);
 void launch_symmetrize_batch(const MolDesc* mols, const SymDesc* d, int nmol, int nmax, hipStream_t s);
 void launch_fill_zero(double* p, size_t count, hipStream_t s);
+// The packed slabs of an intra-species transform: clear their np values (of
+// n^2) each; spread slabs j0 .. j0 + count - 1 over both triangles through
+// tmp (count * np doubles) and slot (n^2: where (k, l) lies in a packed slab,
+// -1 nowhere), which launch_slab_slots fills.
+void launch_clear_slabs(double* GG, int n, int np, hipStream_t s);
+void launch_slab_slots(int* slot, const PairInfo* pairs, const int* pidx, const int* fsh, int n, int nshell,
+                       const int* off, const int* jpoff, hipStream_t s);
+void launch_unpack_slabs(double* GG, double* tmp, const int* slot, int n, int np, int j0, int count, hipStream_t s);
 // GG[i][k][j] = GG[i][j][k] for j < k, i < n1, j, k < n2.
 void launch_mirror_upper(double* GG, int n1, int n2, hipStream_t s);
 void launch_prologue_batch(const MolDesc* mols, int nmol, int nmax, hipStream_t s);

@@ -281,6 +281,52 @@ __global__ void fill_zero_kernel(double* p, size_t count) {
   for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < count; k += stride) p[k] = 0.0;
 }
 
+// Packed slabs of the intra-species transform (lowdin_kernels.h).
+__global__ void clear_slabs_kernel(double* GG, size_t n2, int np) {
+  double* slab = GG + (size_t)blockIdx.y * n2;
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < np; k += gridDim.x * blockDim.x) slab[k] = 0.0;
+}
+
+struct SlabOffsets {
+  int off[7], jpoff[7];
+};
+__global__ void slab_slots_kernel(int* slot, const PairInfo* pairs, const int* pidx, const int* fsh, int n, int nshell,
+                                  SlabOffsets o) {
+  const int i = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n || k >= n) return;
+  const int si = fsh[i], sk = fsh[k];
+  // the pair's orientation; within one shell the k <= l element holds the value
+  int x = i, y = k, q = pidx[si * nshell + sk];
+  if (q < 0 || (si == sk && i > k)) {
+    x = k;
+    y = i;
+    q = pidx[sk * nshell + si];
+  }
+  int at = -1;
+  if (q >= 0) {
+    const PairInfo* P = pairs + q;
+    const int c = P->la * (P->la + 1) / 2 + P->lb;
+    const int e = (x - P->bfa) * ncart_(P->lb) + (y - P->bfb);
+    at = o.jpoff[c] + e * (o.off[c + 1] - o.off[c]) + (q - o.off[c]);
+  }
+  slot[(size_t)i * n + k] = at;
+}
+
+__global__ void pack_slabs_kernel(const double* GG, double* tmp, size_t n2, int np, int j0) {
+  const double* slab = GG + (size_t)(j0 + blockIdx.y) * n2;
+  double* out = tmp + (size_t)blockIdx.y * np;
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < np; k += gridDim.x * blockDim.x) out[k] = slab[k];
+}
+
+__global__ void unpack_slabs_kernel(double* GG, const double* tmp, const int* slot, size_t n2, int np, int j0) {
+  double* slab = GG + (size_t)(j0 + blockIdx.y) * n2;
+  const double* in = tmp + (size_t)blockIdx.y * np;
+  for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n2; k += (size_t)gridDim.x * blockDim.x) {
+    const int at = slot[k];
+    slab[k] = at < 0 ? 0.0 : in[at];
+  }
+}
+
 // Lower triangle of every (k, l) slice from the upper one: the
 // first-quarter-transform kernels accumulate k <= l only.
 __global__ void mirror_upper_kernel(double* GG, int n1, int n2) {
@@ -442,6 +488,34 @@ void launch_fill_zero(double* p, size_t count, hipStream_t s) {
 }
 
 static unsigned grid_for(size_t count) { return (unsigned)std::min<size_t>((count + 255) / 256, 4096); }
+
+void launch_clear_slabs(double* GG, int n, int np, hipStream_t s) {
+  if (n <= 0 || np <= 0) return;
+  const unsigned bx = std::min((np + 255) / 256, 64);
+  hipLaunchKernelGGL(clear_slabs_kernel, dim3(bx, n), dim3(256), 0, s, GG, (size_t)n * n, np);
+}
+
+void launch_slab_slots(int* slot, const PairInfo* pairs, const int* pidx, const int* fsh, int n, int nshell,
+                       const int* off, const int* jpoff, hipStream_t s) {
+  if (n <= 0) return;
+  SlabOffsets o;
+  for (int c = 0; c < 7; ++c) {
+    o.off[c] = off[c];
+    o.jpoff[c] = jpoff[c];
+  }
+  const dim3 blk(32, 8), grd((n + 31) / 32, (n + 7) / 8);
+  hipLaunchKernelGGL(slab_slots_kernel, grd, blk, 0, s, slot, pairs, pidx, fsh, n, nshell, o);
+}
+
+void launch_unpack_slabs(double* GG, double* tmp, const int* slot, int n, int np, int j0, int count, hipStream_t s) {
+  if (n <= 0 || count <= 0) return;
+  const size_t n2 = (size_t)n * n;
+  if (np > 0)
+    hipLaunchKernelGGL(pack_slabs_kernel, dim3(std::min((np + 255) / 256, 64), count), dim3(256), 0, s, GG, tmp, n2, np,
+                       j0);
+  hipLaunchKernelGGL(unpack_slabs_kernel, dim3((unsigned)std::min<size_t>((n2 + 255) / 256, 64), count), dim3(256), 0, s,
+                     GG, tmp, slot, n2, np, j0);
+}
 
 void launch_mirror_upper(double* GG, int n1, int n2, hipStream_t s) {
   const size_t total = (size_t)n1 * n2 * n2;
