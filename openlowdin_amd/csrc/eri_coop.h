@@ -550,8 +550,8 @@ __device__ __forceinline__ void coop_coupling_update(double* R, const CouplingAr
 // (eri_core.h) split over the lanes -- lane k < NA NB sums result element
 // (a b) on the bra species over the ket density's element set, lane k <
 // NC ND element (c d) on the ket species over the bra density's.  A
-// workgroup owns one coupling task (a bra pair and up to 64 ket pairs);
-// its wavefronts take the kets in turn.  No private segment: the state of
+// workgroup, one wavefront, owns one coupling task (a bra pair and a run of
+// ket pairs).  No private segment: the state of
 // a quartet lives in the wavefront's LDS region.
 template <int LA, int LB, int LC, int LD>
 __global__ __launch_bounds__(256, 2) void coupling_coop_kernel(CouplingArgs a) {
@@ -584,19 +584,14 @@ template <int LA, int LB, int LC, int LD>
 static void coop_attr_t() {
   (void)hipFuncSetAttribute((const void*)jk_coop_kernel<LA, LB, LC, LD>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)kCoopLdsMax);
-  (void)hipFuncSetAttribute((const void*)coupling_coop_kernel<LA, LB, LC, LD>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCoopLdsMax);
 }
 
-// One workgroup of up to four wavefronts per coupling task.
+// One wavefront per coupling task.
 template <int LA, int LB, int LC, int LD>
 static bool launch_cp_coop_t(const CouplingArgs& a, hipStream_t s) {
   if (a.ntasks <= 0) return true;
   constexpr size_t wave = (size_t)coop_wave_doubles<LA, LB, LC, LD>() * sizeof(double);
-  int W = 4;
-  while (W > 1 && W * wave > kCoopLdsMax) --W;
-  if (W * wave > kCoopLdsMax) return false;
-  hipLaunchKernelGGL((coupling_coop_kernel<LA, LB, LC, LD>), dim3(a.ntasks), dim3(64 * W), W * wave, s, a);
+  hipLaunchKernelGGL((coupling_coop_kernel<LA, LB, LC, LD>), dim3(a.ntasks), dim3(64), wave, s, a);
   return true;
 }
 

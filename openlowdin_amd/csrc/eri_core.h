@@ -835,8 +835,9 @@ __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_s
 }
 
 // ------------------------------------------------------- coupling kernel
-// Quartets (bra pair of species X | ket pair of species Y) over ALL pairs
-// s1 <= s2 of both species.  Computes the result on the bra species from the
+// Quartets (bra pair of species X | ket pair of species Y) over all pairs
+// s1 <= s2 of both species, less those whose Schwarz bound lies below the
+// drop of raw integrals (they hold nothing that is kept).  Computes the result on the bra species from the
 // ket species' density (rbra) and/or on the ket species from the bra
 // species' density (rket), each with the reference's element sets and drop.
 // Drop, density weights and scatter of one coupling quartet's raw block
@@ -920,40 +921,46 @@ __global__ __launch_bounds__(256) void coupling_kernel(CouplingArgs a) {
   if (wid >= a.ntasks) return;
   const Task t = a.tasks[wid];
   const int lane = threadIdx.x & 63;
-  const int j = t.j0 + lane;
+  const PairInfo P = load_pair((gcptr<PairInfo>)a.bra + t.bra);
+  const int ls = split_shift(P.nprim, a.ket[t.j0].nprim, a.lmax);
+  const int j = t.j0 + (lane >> ls), sub = lane & ((1 << ls) - 1);
   // every lane stays for the wavefront's bra-side reduction; lanes without
-  // a ket contribute a zero block and no ket-side update
+  // a ket, and all but the first that share one, contribute a zero block and
+  // no ket-side update
   const bool active = j < t.j1;
-  const PairInfo& P = a.bra[t.bra];
-  const PairInfo K = a.ket[active ? j : t.j0];
+  const PairInfo K = load_pair((gcptr<PairInfo>)a.ket + (active ? j : t.j0));
   double out[NA * NB * NC * ND];
-  if (active) {
-    contracted_quartet<LA, LB, LC, LD>(a.bprim + (size_t)P.poff * kPrimPairStride, P.nprim,
-                                       a.kprim + (size_t)K.poff * kPrimPairStride, K.nprim, a.boys,
-                                       P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
-  } else {
+  if (active)
+    contracted_quartet<LA, LB, LC, LD>((gcptr<double>)a.bprim + (size_t)P.poff * kPrimPairStride, P.nprim,
+                                       (gcptr<double>)a.kprim + (size_t)K.poff * kPrimPairStride, K.nprim, a.boys,
+                                       P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out, sub, 1 << ls);
+  if (!active || sub != 0) {
 #pragma unroll
     for (int k = 0; k < NA * NB * NC * ND; ++k) out[k] = 0.0;
   }
   CouplingArgs b = a;
-  if (!active) b.rket = nullptr;
+  if (!active || sub != 0) b.rket = nullptr;
   coupling_scatter<LA, LB, LC, LD, true>(b, P, K, out);
 }
 
 // --------------------------------------------------- Schwarz (a11) kernel
 // Q(pair) = sqrt(max_i |(ij|ij)_raw|) over the diagonal of the pair's
 // (ab|ab) block, no primitive screening (Libint2Iface.cpp:3361-3404).
+// 2^ls lanes share a pair: its (8 x 8)^2 primitive quartets (cc-pVDZ carbon
+// s shells) in one lane were 1.6 ms of a first build, the longest part.
 template <int LA, int LB>
-__global__ __launch_bounds__(256) void schwarz_kernel(PairInfo* pairs, int npairs, const double* prim,
+__global__ __launch_bounds__(256) void schwarz_kernel(PairInfo* pairs, int npairs, int ls, const double* prim,
                                                       const double* boys, const double* norma) {
   constexpr int NA = ncart(LA), NB = ncart(LB), N2 = NA * NB;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = (int)(idx >> ls), sub = (int)(idx & ((1 << ls) - 1));
   if (i >= npairs) return;
   PairInfo P = pairs[i];
   double out[N2 * N2];
   const double* pp = prim + (size_t)P.poff * kPrimPairStride;
   contracted_quartet<LA, LB, LA, LB>(pp, P.nprim, pp, P.nprim, boys, P.ABx, P.ABy, P.ABz, P.ABx,
-                                     P.ABy, P.ABz, out);
+                                     P.ABy, P.ABz, out, sub, 1 << ls);
+  if (sub != 0) return;
   double mx = 0.0, mxn = 0.0;
 #pragma unroll
   for (int ia = 0; ia < NA; ++ia)
@@ -994,11 +1001,11 @@ static void launch_cp_t(const CouplingArgs& a, hipStream_t s) {
 }
 
 template <int LA, int LB>
-static void launch_schwarz_t(PairInfo* pairs, int npairs, const double* prim, const double* boys, const double* norma,
-                             hipStream_t s) {
+static void launch_schwarz_t(PairInfo* pairs, int npairs, int ls, const double* prim, const double* boys,
+                             const double* norma, hipStream_t s) {
   if (npairs <= 0) return;
-  hipLaunchKernelGGL((schwarz_kernel<LA, LB>), dim3((npairs + 255) / 256), dim3(256), 0, s, pairs, npairs, prim, boys,
-                     norma);
+  const unsigned blocks = (unsigned)((((long)npairs << ls) + 255) / 256);
+  hipLaunchKernelGGL((schwarz_kernel<LA, LB>), dim3(blocks), dim3(256), 0, s, pairs, npairs, ls, prim, boys, norma);
 }
 
 }  // namespace lowdin

@@ -179,12 +179,12 @@ void launch_gcp_2222(const G12CouplingArgs&, hipStream_t);
 bool launch_jkc_2222(const JKArgs&, hipStream_t);
 bool launch_cpc_2222(const CouplingArgs&, hipStream_t);
 void coop_attr_2222();
-void launch_schwarz_00(PairInfo*, int, const double*, const double*, const double*, hipStream_t);
-void launch_schwarz_10(PairInfo*, int, const double*, const double*, const double*, hipStream_t);
-void launch_schwarz_11(PairInfo*, int, const double*, const double*, const double*, hipStream_t);
-void launch_schwarz_20(PairInfo*, int, const double*, const double*, const double*, hipStream_t);
-void launch_schwarz_21(PairInfo*, int, const double*, const double*, const double*, hipStream_t);
-void launch_schwarz_22(PairInfo*, int, const double*, const double*, const double*, hipStream_t);
+void launch_schwarz_00(PairInfo*, int, int, const double*, const double*, const double*, hipStream_t);
+void launch_schwarz_10(PairInfo*, int, int, const double*, const double*, const double*, hipStream_t);
+void launch_schwarz_11(PairInfo*, int, int, const double*, const double*, const double*, hipStream_t);
+void launch_schwarz_20(PairInfo*, int, int, const double*, const double*, const double*, hipStream_t);
+void launch_schwarz_21(PairInfo*, int, int, const double*, const double*, const double*, hipStream_t);
+void launch_schwarz_22(PairInfo*, int, int, const double*, const double*, const double*, hipStream_t);
 inline bool dispatch_jk(int la, int lb, int lc, int ld, const JKArgs& a, hipStream_t s) {
   switch (la * 1000 + lb * 100 + lc * 10 + ld) {
     case 0: launch_jk_0000(a, s); return true;
@@ -414,14 +414,14 @@ inline bool dispatch_g12cp(int la, int lb, int lc, int ld, const G12CouplingArgs
     default: return false;
   }
 }
-inline bool dispatch_schwarz(int la, int lb, PairInfo* p, int np, const double* prim, const double* boys, const double* norma, hipStream_t s) {
+inline bool dispatch_schwarz(int la, int lb, PairInfo* p, int np, int ls, const double* prim, const double* boys, const double* norma, hipStream_t s) {
   switch (la * 10 + lb) {
-    case 0: launch_schwarz_00(p, np, prim, boys, norma, s); return true;
-    case 10: launch_schwarz_10(p, np, prim, boys, norma, s); return true;
-    case 11: launch_schwarz_11(p, np, prim, boys, norma, s); return true;
-    case 20: launch_schwarz_20(p, np, prim, boys, norma, s); return true;
-    case 21: launch_schwarz_21(p, np, prim, boys, norma, s); return true;
-    case 22: launch_schwarz_22(p, np, prim, boys, norma, s); return true;
+    case 0: launch_schwarz_00(p, np, ls, prim, boys, norma, s); return true;
+    case 10: launch_schwarz_10(p, np, ls, prim, boys, norma, s); return true;
+    case 11: launch_schwarz_11(p, np, ls, prim, boys, norma, s); return true;
+    case 20: launch_schwarz_20(p, np, ls, prim, boys, norma, s); return true;
+    case 21: launch_schwarz_21(p, np, ls, prim, boys, norma, s); return true;
+    case 22: launch_schwarz_22(p, np, ls, prim, boys, norma, s); return true;
     default: return false;
   }
 }

@@ -770,8 +770,8 @@ def main(outdir):
         with open(os.path.join(gdir, "eri_%s.inc" % k), "w") as fh:
             fh.write("\n".join(inc))
         diag = (la, lb) == (lc, ld)
-        schwfn = ("void launch_schwarz_%d%d(PairInfo* pairs, int npairs, const double* prim, const double* boys, "
-                  "const double* norma, hipStream_t s) { launch_schwarz_t<%d, %d>(pairs, npairs, prim, boys, norma, s); }\n"
+        schwfn = ("void launch_schwarz_%d%d(PairInfo* pairs, int npairs, int ls, const double* prim, const double* boys, "
+                  "const double* norma, hipStream_t s) { launch_schwarz_t<%d, %d>(pairs, npairs, ls, prim, boys, norma, s); }\n"
                   % (la, lb, la, lb)
                   if diag else "")
         coop = la + lb + lc + ld >= COOP_MIN_L
@@ -829,7 +829,7 @@ def main(outdir):
             lines.append("bool launch_cpc_%s(const CouplingArgs&, hipStream_t);" % k)
             lines.append("void coop_attr_%s();" % k)
     for (la, lb) in pcs:
-        lines.append("void launch_schwarz_%d%d(PairInfo*, int, const double*, const double*, const double*, hipStream_t);"
+        lines.append("void launch_schwarz_%d%d(PairInfo*, int, int, const double*, const double*, const double*, hipStream_t);"
                      % (la, lb))
     lane_classes = [c for c in classes if sum(c) < COOP_ONLY_L]
     lines.append("inline bool dispatch_jk(int la, int lb, int lc, int ld, const JKArgs& a, hipStream_t s) {")
@@ -890,11 +890,11 @@ def main(outdir):
     for (la, lb, lc, ld) in classes:
         lines.append("    case %d: launch_gcp_%d%d%d%d(a, s); return true;" % (la * 1000 + lb * 100 + lc * 10 + ld, la, lb, lc, ld))
     lines.append("    default: return false;\n  }\n}")
-    lines.append("inline bool dispatch_schwarz(int la, int lb, PairInfo* p, int np, const double* prim, const double* boys, "
+    lines.append("inline bool dispatch_schwarz(int la, int lb, PairInfo* p, int np, int ls, const double* prim, const double* boys, "
                  "const double* norma, hipStream_t s) {")
     lines.append("  switch (la * 10 + lb) {")
     for (la, lb) in pcs:
-        lines.append("    case %d: launch_schwarz_%d%d(p, np, prim, boys, norma, s); return true;" % (la * 10 + lb, la, lb))
+        lines.append("    case %d: launch_schwarz_%d%d(p, np, ls, prim, boys, norma, s); return true;" % (la * 10 + lb, la, lb))
     lines.append("    default: return false;\n  }\n}")
     lines.append("}  // namespace lowdin")
     with open(os.path.join(gdir, "dispatch.h"), "w") as fh:

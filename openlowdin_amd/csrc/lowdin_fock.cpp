@@ -180,6 +180,7 @@ struct PairSet {
   DevBuf<int> d_pidx;               // nshell x nshell: pair of (sa, sb), -1 if none; then the shell of each function
   int jpoff[kNumPairClasses + 1] = {0};   // MolDesc::jpoff
   int maxprim = 0;                  // most primitive pairs of a pair
+  uint64_t listed[kNumPairClasses] = {0}, listed_prims[kNumPairClasses] = {0};   // pairs asked for, their primitive pairs
   bool q_ready = false;
 };
 
@@ -342,8 +343,10 @@ static void ensure_device_basis(Species& s, hipStream_t st) {
 // Canonical pair records (higher-l shell first) grouped by pair class,
 // sorted within a class by surviving primitive-pair count (descending) so
 // that neighbouring lanes run equal primitive loops.
-static void build_pairset(const Species& s, const std::vector<std::pair<int, int>>& list, PairSet& ps,
-                          hipStream_t st) {
+// Pairs without a surviving primitive pair are kept only on request: every
+// integral over them is zero.
+static void build_pairset(const Species& s, const std::vector<std::pair<int, int>>& list, PairSet& ps, hipStream_t st,
+                          bool keep_empty) {
   struct Tmp {
     PairInfo info;
     std::vector<double> prim;
@@ -351,6 +354,8 @@ static void build_pairset(const Species& s, const std::vector<std::pair<int, int
   };
   std::vector<Tmp> tmp;
   tmp.reserve(list.size());
+  std::fill(std::begin(ps.listed), std::end(ps.listed), 0);
+  std::fill(std::begin(ps.listed_prims), std::end(ps.listed_prims), 0);
   const double kfac = std::sqrt(2.0) * std::pow(M_PI, 1.25);
   for (size_t k = 0; k < list.size(); ++k) {
     int sa = list[k].first, sb = list[k].second;
@@ -385,7 +390,10 @@ static void build_pairset(const Species& s, const std::vector<std::pair<int, int
       }
     }
     P.nprim = (int)(t.prim.size() / kPrimPairStride);
-    tmp.push_back(std::move(t));
+    const int pc = pair_class(P.la, P.lb);
+    ps.listed[pc]++;
+    ps.listed_prims[pc] += (uint64_t)P.nprim;
+    if (P.nprim > 0 || keep_empty) tmp.push_back(std::move(t));
   }
   std::stable_sort(tmp.begin(), tmp.end(), [](const Tmp& x, const Tmp& y) {
     const int cx = pair_class(x.info.la, x.info.lb), cy = pair_class(y.info.la, y.info.lb);
@@ -489,6 +497,17 @@ static void resort_by_q(PairSet& ps, int nshell, const std::vector<int>& fsh, hi
   HIPCHK(hipStreamSynchronize(st));
 }
 
+// Lanes share a quartet when one lane would take more than lmax primitive
+// quartets one after another: that serial loop (up to 8^4 for cc-pVDZ carbon)
+// is what a small build waits for, and what leaves the lanes of a wavefront
+// and the waves of a workgroup uneven in a large one.  Long ket rows fill the
+// lanes by themselves, so lmax grows with the kets per bra.  Measured, lmax
+// 5000 (never shared) / 64 / 16: water 6-31G** 1066 / 782 / 569 us,
+// (H2O)10 3.51 / 3.31 / 3.22 ms, C20H42 21.1 / 20.7 / 22.0 ms (its (ss|ss)
+// alone 2.99 / 1.76 / 2.23 ms), 72 clusters in a batch 26.6 / 25.1 / 23.7 ms.
+constexpr double kSplitMin = 16.0, kSplitMax = 64.0;
+constexpr double kSplitKets = 32.0;   // kets per bra for each unit of lmax
+
 // Runs on the heavy-kernel stream (the (dd|dd) diagonal spills); the pair
 // records were uploaded and their stream drained by build_pairset.
 static void compute_schwarz(PairSet& ps, const double* d_norma, hipStream_t st) {
@@ -498,7 +517,10 @@ static void compute_schwarz(PairSet& ps, const double* d_norma, hipStream_t st) 
   for (int pc = 0; pc < kNumPairClasses; ++pc) {
     const int n = ps.off[pc + 1] - ps.off[pc];
     if (n == 0) continue;
-    if (!dispatch_schwarz(kPairClassL[pc][0], kPairClassL[pc][1], ps.d_pairs.p + ps.off[pc], n, ps.d_prims.p,
+    // lanes per pair for the longest primitive loop of the class (the pairs
+    // come in descending order of primitive count)
+    const int ls = split_shift(ps.pairs[ps.off[pc]].nprim, ps.pairs[ps.off[pc]].nprim, (int)kSplitMin);
+    if (!dispatch_schwarz(kPairClassL[pc][0], kPairClassL[pc][1], ps.d_pairs.p + ps.off[pc], n, ls, ps.d_prims.p,
                           c.boys.p, d_norma, hs))
       throw std::runtime_error("no Schwarz kernel for pair class");
   }
@@ -573,17 +595,6 @@ constexpr long kCoopMinRun = 4;
 // more in zeroed, filled and flushed LDS than the even load gains (C20H42:
 // 512 -> 4096 workgroups 20.9 -> 22.5 ms).
 constexpr double kQuartetIters = 12.0;
-// Lanes share a quartet when one lane would take more than lmax primitive
-// quartets one after another: that serial loop (up to 8^4 for cc-pVDZ carbon)
-// is what a small build waits for, and what leaves the lanes of a wavefront
-// and the waves of a workgroup uneven in a large one.  Long ket rows fill the
-// lanes by themselves, so lmax grows with the kets per bra.  Measured, lmax
-// 5000 (never shared) / 64 / 16: water 6-31G** 1066 / 782 / 569 us,
-// (H2O)10 3.51 / 3.31 / 3.22 ms, C20H42 21.1 / 20.7 / 22.0 ms (its (ss|ss)
-// alone 2.99 / 1.76 / 2.23 ms), 72 clusters in a batch 26.6 / 25.1 / 23.7 ms.
-constexpr double kSplitMin = 16.0, kSplitMax = 64.0;
-constexpr double kSplitKets = 32.0;   // kets per bra for each unit of lmax
-
 // A plan runs as one launch over all classes (jk_fused_kernel) up to this
 // many candidate quartets and tasks (one per bra and ket class).  Above, its
 // one wavefront per SIMD costs more than the side-by-side classes gain: class
@@ -599,7 +610,7 @@ static inline int class_pair_id(int cx, int cy) { return cx * (cx + 1) / 2 + cy;
 static void ensure_sig(Species& s, hipStream_t st) {
   ensure_device_basis(s, st);
   if (!s.sig.valid) {
-    build_pairset(s, s.pairlist, s.sig, st);
+    build_pairset(s, s.pairlist, s.sig, st, true);
     compute_schwarz(s.sig, s.d_norma.p, st);
     resort_by_q(s.sig, (int)s.shells.size(), s.fsh, st, s.mixed != 0);
     s.sig_mixed = s.mixed;
@@ -878,12 +889,44 @@ static void ensure_all(Species& s, hipStream_t st) {
     const int ns = (int)s.shells.size();
     for (int s1 = 0; s1 < ns; ++s1)
       for (int s2 = s1; s2 < ns; ++s2) list.push_back({s1, s2});
-    build_pairset(s, list, s.all, st);
+    build_pairset(s, list, s.all, st, false);
+    // Schwarz bounds; within a class and primitive count the largest first,
+    // so that a bra's kets above a bound are the first ones of each run (the
+    // primitive records stay where they are)
+    compute_schwarz(s.all, s.d_norma.p, st);
+    std::stable_sort(s.all.pairs.begin(), s.all.pairs.end(), [](const PairInfo& x, const PairInfo& y) {
+      const int cx = pair_class(x.la, x.lb), cy = pair_class(y.la, y.lb);
+      if (cx != cy) return cx < cy;
+      if (x.nprim != y.nprim) return x.nprim > y.nprim;
+      return x.Q > y.Q;
+    });
+    s.all.d_pairs.upload(s.all.pairs.data(), s.all.pairs.size(), st);
+  }
+}
+
+// Raw coupling integrals below this are dropped (Libint2Iface.cpp:1226-1228,
+// 1456, 2496-2497, 2865).
+constexpr double kCouplingDrop = 1.0e-10;
+
+// Kets that, with a bra of bound q, may hold a raw integral of at least
+// kCouplingDrop, as runs of equal primitive counts.  |(ab|cd)| <= Q_ab Q_cd;
+// the factor of ten covers the rounding of bounds that are themselves small
+// differences.
+template <typename F>
+static void kets_above(const PairInfo* kets, const std::vector<KetRun>& runs, double q, F&& f) {
+  for (const KetRun& r : runs) {
+    const PairInfo* e = std::partition_point(kets + r.j0, kets + r.j1,
+                                             [&](const PairInfo& k) { return !(q * k.Q < 0.1 * kCouplingDrop); });
+    if (e > kets + r.j0) f(r.j0, (int)(e - kets), r.np);
   }
 }
 
 // Coupling quartets between species a and b: for every pair of pair
 // classes the larger class is the bra (the kernels' VRR builds on the bra).
+// Quartets whose Schwarz bound lies below the drop are left out, lanes share
+// those that are left and the high classes go out in short runs: C20H42 with
+// a quantum proton (510 and 23 functions) 2.21 -> 1.20 ms, FHF- with its
+// proton 0.87 -> 0.66 ms for its two builds and the coupling.
 static TaskSet* coupling_taskset(Species& a, Species& b, hipStream_t st) {
   auto it = a.coupling_tasks.find(b.uid);
   if (it != a.coupling_tasks.end() && it->second.gen_self == a.generation && it->second.gen_other == b.generation &&
@@ -894,6 +937,7 @@ static TaskSet* coupling_taskset(Species& a, Species& b, hipStream_t st) {
   ts->tasks.clear();
   ts->launches.clear();
   std::vector<double> cost;
+  std::vector<std::pair<double, Task>> made;
   for (int ca = 0; ca < kNumPairClasses; ++ca)
     for (int cb = 0; cb < kNumPairClasses; ++cb) {
       const int na = a.all.off[ca + 1] - a.all.off[ca], nb = b.all.off[cb + 1] - b.all.off[cb];
@@ -905,19 +949,34 @@ static TaskSet* coupling_taskset(Species& a, Species& b, hipStream_t st) {
       const int nbra = a_bra ? na : nb, nket = a_bra ? nb : na;
       const PairInfo* bras = B.pairs.data() + B.off[cbra];
       const PairInfo* kets = K.pairs.data() + K.off[cket];
+      const int la = kPairClassL[cbra][0], lb = kPairClassL[cbra][1];
+      const int lc = kPairClassL[cket][0], ld = kPairClassL[cket][1];
+      const std::vector<KetRun> runs = ket_runs(kets, nket);
+      double work = 0.0, total = 0.0;   // primitive quartets, quartets that may hold a kept integral
+      for (int i = 0; i < nbra; ++i)
+        kets_above(kets, runs, bras[i].Q, [&](int j0, int j1, int np) {
+          work += (double)bras[i].nprim * np * (j1 - j0);
+          total += j1 - j0;
+        });
+      if (total == 0.0) continue;
+      const bool coop = la + lb + lc + ld >= kCoopDefaultL;   // one wavefront per quartet
+      const int lmax = unit_share(work, la + lb + lc + ld);
+      const int run = (int)std::max(1.0, total / kCoopDefaultWg);
       const size_t from = ts->tasks.size();
-      for (int i = 0; i < nbra; ++i) emit_tasks(ts->tasks, i, 0, nket, kets, 0);
-      sort_by_cost(ts->tasks, from, bras, kets);
-      ts->launches.push_back({kPairClassL[cbra][0], kPairClassL[cbra][1], kPairClassL[cket][0],
-                              kPairClassL[cket][1], cbra, cket, a_bra ? 1 : 0, from, ts->tasks.size() - from, 0});
+      made.clear();
+      for (int i = 0; i < nbra; ++i)
+        kets_above(kets, runs, bras[i].Q, [&](int j0, int j1, int np) {
+          const int step = coop ? run : 64 >> split_shift(bras[i].nprim, np, lmax);
+          for (int j = j0; j < j1; j += step) {
+            const int e = std::min(j + step, j1);
+            made.push_back({(double)bras[i].nprim * np * (e - j), Task{i, j, e, 0}});
+          }
+        });
+      append_by_cost(ts->tasks, made);
+      ts->launches.push_back({la, lb, lc, ld, cbra, cket, a_bra ? 1 : 0, from, ts->tasks.size() - from, coop ? 4 : 0,
+                              lmax});
       // estimated cost: primitive quartets x class weight, as for the J/K launches
-      const int lt = kPairClassL[cbra][0] + kPairClassL[cbra][1] + kPairClassL[cket][0] + kPairClassL[cket][1];
-      double c = 0.0;
-      for (size_t t = from; t < ts->tasks.size(); ++t) {
-        const Task& k = ts->tasks[t];
-        c += (double)bras[k.bra].nprim * kets[k.j0].nprim * (k.j1 - k.j0);
-      }
-      cost.push_back(c * (1.0 + lt * lt));
+      cost.push_back(work * (1.0 + (la + lb + lc + ld) * (la + lb + lc + ld)));
     }
   ts->order.resize(ts->launches.size());
   for (size_t k = 0; k < ts->order.size(); ++k) ts->order[k] = k;
@@ -1288,6 +1347,20 @@ static void compute_2body(Species& s, const double* dens, double* result, double
   s.stats = p.stats;
 }
 
+// Quartets, ERIs and primitive quartets of all pairs of both species (the
+// reference's loop, before any bound).
+static void count_coupling(const Species& a, const Species& b, lowdin_fock_stats* stt) {
+  if (!stt) return;
+  for (int ca = 0; ca < kNumPairClasses; ++ca)
+    for (int cb = 0; cb < kNumPairClasses; ++cb) {
+      const uint64_t q = a.all.listed[ca] * b.all.listed[cb];
+      stt->quartets += q;
+      stt->eris += q * (uint64_t)(ncart_h(kPairClassL[ca][0]) * ncart_h(kPairClassL[ca][1]) *
+                                  ncart_h(kPairClassL[cb][0]) * ncart_h(kPairClassL[cb][1]));
+      stt->prim_quartets += a.all.listed_prims[ca] * b.all.listed_prims[cb];
+    }
+}
+
 // Enqueue the coupling quartets of species a and b on st: dRa (n_a^2) =
 // coupling on a from dDb and/or dRb (n_b^2) = coupling on b from dDa (device
 // pointers; either result may be null).  Results are zeroed here by a fill
@@ -1307,7 +1380,6 @@ static void enqueue_coupling(Species& a, Species& b, const double* dDb, double* 
     HIPCHK(hipEventRecord(c.fork, st));
     for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
   }
-  uint64_t quartets = 0, eris = 0, prims = 0;
   for (size_t r = 0; r < ts->launches.size(); ++r) {
     const TaskSet::Launch& L = ts->launches[ts->order[r]];
     hipStream_t hs = inline_launch ? st : c.side[r % kSideStreams];
@@ -1326,7 +1398,8 @@ static void enqueue_coupling(Species& a, Species& b, const double* dDb, double* 
     g.nbra = sb.nbasis;
     g.nket = sk.nbasis;
     g.boys = c.boys.p;
-    g.drop = 1.0e-10;  // Libint2Iface.cpp:1226-1228
+    g.drop = kCouplingDrop;
+    g.lmax = L.lmax;
     if (a_bra) {
       g.rbra = dRa;  g.dket = dDb;
       g.rket = dRb;  g.dbra = dDa;
@@ -1339,24 +1412,11 @@ static void enqueue_coupling(Species& a, Species& b, const double* dDb, double* 
     const bool coop = L.la + L.lb + L.lc + L.ld >= kCoopDefaultL && has_jk_coop(L.la, L.lb, L.lc, L.ld);
     if (!(coop ? dispatch_cp_coop(L.la, L.lb, L.lc, L.ld, g, hs) : dispatch_cp(L.la, L.lb, L.lc, L.ld, g, hs)))
       throw std::runtime_error("no coupling kernel for class");
-    if (stt) {
-      for (size_t k = L.off; k < L.off + L.count; ++k) {
-        const Task& t = ts->tasks[k];
-        const int nq = t.j1 - t.j0;
-        quartets += nq;
-        eris += (uint64_t)nq * ncart_h(L.la) * ncart_h(L.lb) * ncart_h(L.lc) * ncart_h(L.ld);
-        prims += (uint64_t)nq * sb.all.pairs[sb.all.off[L.cbra] + t.bra].nprim *
-                 sk.all.pairs[sk.all.off[L.cket] + t.j0].nprim;
-      }
-    }
   }
   HIPCHK(hipGetLastError());
   if (!inline_launch) join_side_streams(st);
-  if (stt) {
-    stt->quartets = quartets;
-    stt->eris = eris;
-    stt->prim_quartets = prims;
-  }
+  if (stt) stt->quartets = stt->eris = stt->prim_quartets = 0;
+  count_coupling(a, b, stt);
 }
 
 static void compute_coupling(Species& a, Species* b, const double* db, double* ra, const double* da, double* rb) {
@@ -1590,12 +1650,13 @@ static void enqueue_coupling_store(Species& a, Species& b, const double* dC, dou
     g.sx1 = na * nb * nb;
     g.sx2 = nb * nb;
     g.sy1 = nb;
-    g.drop = 1.0e-10;  // Libint2Iface.cpp:1456, 2865
+    g.drop = kCouplingDrop;
+    g.lmax = L.lmax;
     if (!dispatch_cstore(L.la, L.lb, L.lc, L.ld, g, hs)) throw std::runtime_error("no store kernel for class");
-    count_tasks(*ts, L, sb.all.pairs.data() + sb.all.off[L.cbra], sk.all.pairs.data() + sk.all.off[L.cket], stt);
   }
   HIPCHK(hipGetLastError());
   join_side_streams(st);
+  count_coupling(a, b, stt);
   if (mode == 1) launch_mirror_upper(dOut, (int)na, (int)nb, st);
   HIPCHK(hipGetLastError());
 }
@@ -1744,7 +1805,7 @@ static void enqueue_g12_coupling(Species& a, Species& b, const double* dDb, doub
     g.nbra = sb.nbasis;
     g.nket = sk.nbasis;
     g.boys = c.boys.p;
-    g.drop = 1.0e-10;  // Libint2Iface.cpp:2496-2497
+    g.drop = kCouplingDrop;
     if (a_bra) {
       g.rbra = dRa;
       g.dket = dDb;
@@ -1755,10 +1816,10 @@ static void enqueue_g12_coupling(Species& a, Species& b, const double* dDb, doub
     ga.gem = gem;
     ga.lmax = L.lmax;
     if (!dispatch_g12cp(L.la, L.lb, L.lc, L.ld, ga, hs)) throw std::runtime_error("no G12 coupling kernel for class");
-    count_tasks(*ts, L, sb.all.pairs.data() + sb.all.off[L.cbra], sk.all.pairs.data() + sk.all.off[L.cket], stt);
   }
   HIPCHK(hipGetLastError());
   join_side_streams(st);
+  count_coupling(a, b, stt);
 }
 
 // Host-pointer G12 build (b null: intra-species on a with a's density;

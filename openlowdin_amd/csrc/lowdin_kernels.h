@@ -119,6 +119,8 @@ struct CouplingArgs {
   int nbra;
   int nket;
   double drop;             // raw-integral drop (1e-10)
+  int lmax;                // split_shift: primitive quartets a lane takes
+  int pad;
 };
 
 // Integral store (mode 0) or first-quarter transform (mode 1) over the
