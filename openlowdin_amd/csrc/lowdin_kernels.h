@@ -285,6 +285,10 @@ void launch_antisym(double* E, const double* T, int n, hipStream_t s);
 void launch_sym_add(double* Acc, const double* R, int n, double scale, hipStream_t s);
 void launch_lincomb(double* out, const double* hist, size_t nn, const LinComb& lc, hipStream_t s);
 void launch_absmax(const double* x, size_t n, double* out, hipStream_t s);
+// count symmetric n x n matrices (upper triangles, stride_a apart) to
+// eigenvectors in place and ascending eigenvalues (stride_w apart); info[k]
+// nonzero where it did not converge.  False: n too large for it.
+bool launch_syev(double* a, int n, size_t stride_a, double* w, size_t stride_w, int* info, int count, hipStream_t s);
 void launch_scale_cols(double* X, const double* U, const double* w, int n, int m, int col0, hipStream_t s);
 void launch_symmetrize_batch(const MolDesc* mols, const SymDesc* d, int nmol, int nmax, hipStream_t s);
 void launch_fill_zero(double* p, size_t count, hipStream_t s);

@@ -12,8 +12,8 @@
 //     sum_j q_i q_j J_{i<-j}[D_j], symmetrised from the upper triangle;
 //     F = H + q^2 G + C; E = E_pc + sum_s Tr(D_s (H_s + G_s/2 + C_s/2));
 //   * DIIS on the orthogonalised commutator X^T (F D S - S D F) X, history 8,
-//     over all species at once; diagonalisation of X^T F X (rocSOLVER
-//     dsyevd), C = X C', D = eta C_occ C_occ^T.
+//     over all species at once; diagonalisation of X^T F X (one compute
+//     unit up to 64 functions, rocSOLVER dsyevd above), C = X C', D = eta C_occ C_occ^T.
 // Every matrix stays in HBM; the host sees only scalars (traces, the DIIS
 // B-matrix row, the error maximum) and solves the (k+1) x (k+1) DIIS system.
 // Matrices are column-major n x n (all symmetric except X and C).
@@ -135,13 +135,19 @@ double dot(Scf& s, size_t nn, const double* x, const double* y) {
   return r;
 }
 
-// Symmetric eigenproblem in place: A (n x n) -> eigenvectors, W ascending.
+// Symmetric eigenproblem in place: A (n x n) -> eigenvectors, W ascending,
+// on the stream.  The library takes over for large n.
+void syevd_async(Scf& s, ScfSpecies& p, int n, double* A, double* W) {
+  if (!lowdin::launch_syev(A, n, (size_t)n * n, W, n, s.d_info, 1, s.stream))
+    BLASCHK(rocsolver_dsyevd(s.blas, rocblas_evect_original, rocblas_fill_upper, n, A, n, W, p.Ework.p, s.d_info));
+}
+
 void syevd(Scf& s, ScfSpecies& p, int n, double* A, double* W) {
-  BLASCHK(rocsolver_dsyevd(s.blas, rocblas_evect_original, rocblas_fill_upper, n, A, n, W, p.Ework.p, s.d_info));
+  syevd_async(s, p, n, A, W);
   int info = 0;
   SCFCHK(hipMemcpyAsync(&info, s.d_info, sizeof(int), hipMemcpyDeviceToHost, s.stream));
   SCFCHK(hipStreamSynchronize(s.stream));
-  if (info != 0) throw std::runtime_error("rocsolver_dsyevd did not converge (info " + std::to_string(info) + ")");
+  if (info != 0) throw std::runtime_error("diagonalisation did not converge (info " + std::to_string(info) + ")");
 }
 
 // F' = X^T F X into Fp (m x m, leading dimension m).
@@ -163,13 +169,12 @@ void density_from_vectors(Scf& s, ScfSpecies& p, const double* Cp) {
     lowdin::launch_fill_zero(p.D.p, (size_t)n * n, s.stream);
 }
 
-// D from F: orthogonal F', rocSOLVER dsyevd (its info lands in the species'
+// D from F: orthogonal F', its eigenvectors (the info lands in the species'
 // scalar slot and is checked with the next Fock step), C, D.  No host wait.
 void density_from_fock(Scf& s, size_t k, const double* F) {
   ScfSpecies& p = s.sp[k];
   orthogonal_fock(s, p, F, p.Fp.p);
-  BLASCHK(rocsolver_dsyevd(s.blas, rocblas_evect_original, rocblas_fill_upper, p.m, p.Fp.p, p.m, p.W.p, p.Ework.p,
-                           s.d_info));
+  syevd_async(s, p, p.m, p.Fp.p, p.W.p);
   SCFCHK(hipMemcpyAsync(s.d_sc + k * kScal + 4, s.d_info, sizeof(int), hipMemcpyDeviceToDevice, s.stream));
   density_from_vectors(s, p, p.Fp.p);
 }
@@ -288,7 +293,7 @@ void fock_end(Scf& s) {
     int info = 0;
     std::memcpy(&info, sc + 4, sizeof(int));
     if (info != 0)
-      throw std::runtime_error("rocsolver_dsyevd did not converge (info " + std::to_string(info) + ")");
+      throw std::runtime_error("diagonalisation did not converge (info " + std::to_string(info) + ")");
     for (int i = 0; i < nstored; ++i) row[i] += sc[5 + i];
   }
   for (int i = 0; i < nstored; ++i) {
@@ -373,7 +378,7 @@ void update(Scf& s) {
 
 // Grouped diagonalisation for many SCF objects on one stream: the
 // orthogonalised Fock matrices of equal dimension m are packed into one
-// strided array and diagonalised by one rocsolver_dsyevd_strided_batched.
+// strided array and diagonalised by one batched call.
 struct GroupWork {
   Buf A, W, E;
   int* info = nullptr;
@@ -417,8 +422,9 @@ void update_many(const std::vector<Scf*>& scfs) {
       ScfSpecies& p = s.sp[g.second[i].second];
       orthogonal_fock(s, p, p.F.p, w.A.p + (size_t)i * mm);
     }
-    BLASCHK(rocsolver_dsyevd_strided_batched(s0.blas, rocblas_evect_original, rocblas_fill_upper, m, w.A.p, m,
-                                             (rocblas_stride)mm, w.W.p, m, w.E.p, m, w.info, cnt));
+    if (!lowdin::launch_syev(w.A.p, m, mm, w.W.p, m, w.info, cnt, st))
+      BLASCHK(rocsolver_dsyevd_strided_batched(s0.blas, rocblas_evect_original, rocblas_fill_upper, m, w.A.p, m,
+                                               (rocblas_stride)mm, w.W.p, m, w.E.p, m, w.info, cnt));
     for (int i = 0; i < cnt; ++i) {
       Scf& s = *g.second[i].first;
       const size_t k = g.second[i].second;

@@ -12,7 +12,7 @@
 // Species of equal basis size n (and orthogonal dimension m) share a bucket:
 // strided arrays with one slot per species, so that every matrix product of
 // the iteration is one rocblas strided-batched GEMM per bucket, the
-// diagonalisation one rocsolver dsyevd_strided_batched per bucket, and the
+// diagonalisation one batched launch per bucket (rocsolver's for large ones), and the
 // small steps (Fock assembly, traces, error maxima, the DIIS history, its
 // B matrix, the solve of the DIIS equations and the extrapolation) are
 // batched kernels of this file.  The DIIS state lives on the device.  The
@@ -594,8 +594,9 @@ void enqueue_syevd(Engine& e) {
     Bucket& b = *bp;
     const int u = b.used();
     if (!u) continue;
-    BLCHK(rocsolver_dsyevd_strided_batched(e.blas, rocblas_evect_original, rocblas_fill_upper, b.m, b.Fp.p, b.m,
-                                           (rocblas_stride)b.mm(), b.W.p, b.m, b.E.p, b.m, b.info.p, u));
+    if (!lowdin::launch_syev(b.Fp.p, b.m, b.mm(), b.W.p, b.m, b.info.p, u, e.stream))
+      BLCHK(rocsolver_dsyevd_strided_batched(e.blas, rocblas_evect_original, rocblas_fill_upper, b.m, b.Fp.p, b.m,
+                                             (rocblas_stride)b.mm(), b.W.p, b.m, b.E.p, b.m, b.info.p, u));
   }
 }
 
@@ -713,7 +714,7 @@ void step_end(Engine& e) {
                   sizeof(int));
       if (info != 0 && J.status == 0) {
         J.status = 1;
-        J.message = "rocsolver_dsyevd did not converge (info " + std::to_string(info) + ")";
+        J.message = "diagonalisation did not converge (info " + std::to_string(info) + ")";
       }
     }
     J.energy = E;
@@ -731,8 +732,9 @@ void setup_species(Engine& e, const double* H, const double* S, int n, std::vect
   e.tmpE.grow(n, 0, st);
   e.tmpInfo.grow(1, 0, st);
   BCHK(hipMemcpyAsync(e.tmpA.p, S, nn * sizeof(double), hipMemcpyHostToDevice, st));
-  BLCHK(rocsolver_dsyevd(e.blas, rocblas_evect_original, rocblas_fill_upper, n, e.tmpA.p, n, e.tmpW.p, e.tmpE.p,
-                         e.tmpInfo.p));
+  if (!lowdin::launch_syev(e.tmpA.p, n, nn, e.tmpW.p, n, e.tmpInfo.p, 1, st))
+    BLCHK(rocsolver_dsyevd(e.blas, rocblas_evect_original, rocblas_fill_upper, n, e.tmpA.p, n, e.tmpW.p, e.tmpE.p,
+                           e.tmpInfo.p));
   std::vector<double> w(n), U(nn);
   int info = 0;
   BCHK(hipMemcpyAsync(w.data(), e.tmpW.p, n * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -765,8 +767,9 @@ void density_one(Engine& e, Bucket& b, int k) {
   gemm_sb(e, T, N, m, m, n, X, n, nn, Tm, n, nn, 0.0, Fp, m, mm, 1);
   e.tmpE.grow(m, 0, st);
   e.tmpInfo.grow(1, 0, st);
-  BLCHK(rocsolver_dsyevd(e.blas, rocblas_evect_original, rocblas_fill_upper, m, Fp, m, b.W.p + (size_t)k * m,
-                         e.tmpE.p, e.tmpInfo.p));
+  if (!lowdin::launch_syev(Fp, m, mm, b.W.p + (size_t)k * m, m, e.tmpInfo.p, 1, st))
+    BLCHK(rocsolver_dsyevd(e.blas, rocblas_evect_original, rocblas_fill_upper, m, Fp, m, b.W.p + (size_t)k * m,
+                           e.tmpE.p, e.tmpInfo.p));
   double* C = b.C.p + (size_t)k * nn;
   gemm_sb(e, N, N, n, m, m, X, n, nn, Fp, m, mm, 0.0, C, n, nn, 1);
   hipLaunchKernelGGL(b_scale_cols_kernel, dim3((n + 255) / 256, m, 1), dim3(256), 0, st, Tm, C, b.occ.p + (size_t)k * m,
