@@ -67,13 +67,12 @@ struct DevBuf {
 };
 
 // ------------------------------------------------------------ process state
-constexpr int kSideStreams = 4;  // class launches overlap on these (default priority)
-// Kernels of the classes with total angular momentum >= 6 spill to a large
-// private (scratch) segment (up to ~15 KB per lane for (dd|dd)).  The
-// runtime provisions scratch per hardware queue for the device-wide wave
-// count, so such kernels run on one stream only (side stream 0): J/K class
-// launches, the Schwarz kernels and the coupling kernels alike.
-constexpr int kHeavyL = 6;
+// Class launches overlap on these and on the caller's stream (default
+// priority): four streams for the four hardware queues of a process.  A fifth
+// shares a queue with another, so that its launches come after that one's
+// (four side streams beside an idle caller's stream: (H2O)10 2.68 ms against
+// 2.25, C20H42 + proton coupling 1.20 against 0.98, FHF- 0.66 against 0.49).
+constexpr int kSideStreams = 3;
 
 struct Context {
   bool ready = false;
@@ -508,8 +507,8 @@ static void resort_by_q(PairSet& ps, int nshell, const std::vector<int>& fsh, hi
 constexpr double kSplitMin = 16.0, kSplitMax = 64.0;
 constexpr double kSplitKets = 32.0;   // kets per bra for each unit of lmax
 
-// Runs on the heavy-kernel stream (the (dd|dd) diagonal spills); the pair
-// records were uploaded and their stream drained by build_pairset.
+// On one side stream (the (dd|dd) diagonal spills); the pair records were
+// uploaded and their stream drained by build_pairset.
 static void compute_schwarz(PairSet& ps, const double* d_norma, hipStream_t st) {
   Context& c = ctx();
   HIPCHK(hipStreamSynchronize(st));
@@ -1017,19 +1016,19 @@ static void ensure_launch_events(BuildPlan& p) {
   }
 }
 
-// Per-lane kernels of the high-L classes spill to a large private segment;
-// the wave-cooperative kernels keep their state in LDS.
-static inline bool heavy_launch(const TaskSet::Launch& L) {
-  return L.strip < 3 && L.la + L.lb + L.lc + L.ld >= kHeavyL;
+// Streams of the class launches between fork_side_streams and
+// join_side_streams: launch k goes to class_stream(k, st).
+static void fork_side_streams(hipStream_t st) {
+  Context& c = ctx();
+  HIPCHK(hipEventRecord(c.fork, st));
+  for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
 }
 
-// Class launches of one build on the side streams, forked from and joined
-// back to st.  The scratch-heavy classes (few quartets, long per-lane
-// latency) go first, all on side stream 0, so that they run beside the
-// large classes instead of after them; the other classes follow largest
-// first, round robin over the remaining side streams (all four when the
-// plan has no heavy class).  which: 0 all, 1 all but the scratch-heavy
-// ones, 2 only the scratch-heavy ones.
+static hipStream_t class_stream(size_t k, hipStream_t st) {
+  const size_t q = k % (kSideStreams + 1);
+  return q < kSideStreams ? ctx().side[q] : st;
+}
+
 static void join_side_streams(hipStream_t st) {
   Context& c = ctx();
   for (int q = 0; q < kSideStreams; ++q) {
@@ -1038,13 +1037,14 @@ static void join_side_streams(hipStream_t st) {
   }
 }
 
+// Class launches of one build, forked from and joined back to st.
 // mols / counts: descriptor array and per-task counter array the kernels
 // use (null: the plan's own; counts_off: no counters).
-static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, int which, bool join = true,
-                            const MolDesc* mols = nullptr, bool counts_off = false) {
+static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, const MolDesc* mols = nullptr,
+                            bool counts_off = false) {
   Context& c = ctx();
   const size_t nl = p.ts.launches.size();
-  if (p.fused && which != 2) {
+  if (p.fused) {
     FusedArgs f{};
     f.tasks = p.ts.d_tasks.p;
     f.mols = mols ? mols : p.d_desc.p;
@@ -1061,31 +1061,16 @@ static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, int which,
     launch_jk_fused(f, st);
     return;
   }
-  bool any = false, any_heavy = false;
-  for (size_t k = 0; k < nl; ++k) {
-    any = any || which == 0 || (which == 1) != heavy_launch(p.ts.launches[k]);
-    any_heavy = any_heavy || heavy_launch(p.ts.launches[k]);
-  }
-  if (!any) return;
+  if (nl == 0) return;
   // inline plans launch on the caller's stream itself (several batched
   // SCF lanes then overlap without sharing the library's side streams)
   const bool fork = !p.inline_launch;
-  if (fork) {
-    HIPCHK(hipEventRecord(c.fork, st));
-    for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
-  }
-  const int first_light = (any_heavy && which == 0) ? 1 : 0;
-  size_t nlight = 0;
-  for (size_t pass = 0; pass < 2 * nl; ++pass) {
-    const size_t r = pass % nl;
+  if (fork) fork_side_streams(st);
+  // largest first
+  for (size_t r = 0; r < nl; ++r) {
     const size_t k = p.ts.order[r];
     const TaskSet::Launch& L = p.ts.launches[k];
-    const bool heavy = heavy_launch(L);
-    if ((pass < nl) != heavy) continue;   // first pass: heavy classes, second: the rest
-    if ((which == 1 && heavy) || (which == 2 && !heavy)) continue;
-    int q = 0;
-    if (!p.serialize && !heavy) q = first_light + (int)(nlight++ % (size_t)(kSideStreams - first_light));
-    hipStream_t ls = fork ? c.side[q] : st;
+    hipStream_t ls = fork ? class_stream(p.serialize ? 0 : r, st) : st;
     JKArgs a{};
     a.tasks = p.ts.d_tasks.p + L.off;
     a.ntasks = (int)L.count;
@@ -1109,7 +1094,7 @@ static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, int which,
     if (!ok) throw std::runtime_error("no J/K kernel for class");
     if (timed) HIPCHK(hipEventRecord(p.launch_ev[2 * k + 1], ls));
   }
-  if (join && fork) join_side_streams(st);
+  if (fork) join_side_streams(st);
 }
 
 // Dnorm, packed densities and zeroed accumulators (no memset: capturable).
@@ -1184,11 +1169,6 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
   if (timed) ensure_launch_events(p);
   if (record) HIPCHK(hipEventRecord(c.ev0, st));
   if (p.use_graph && !p.fused) {
-    // The graph holds the classes without a large private segment.  Kernels
-    // in a graph run on the runtime's own streams (one per branch), so the
-    // scratch-heavy classes stay outside it, on side stream 0: they are
-    // enqueued after the prologue and before the graph launch, and joined
-    // with it before the epilogue, so that they run beside the graph.
     if (!p.graph || p.graph_layout != p.layout || p.graph_stream != st || p.graph_any_mixed != p.any_mixed ||
         p.graph_eps != p.eps) {
       if (p.graph) HIPCHK(hipGraphExecDestroy(p.graph));
@@ -1196,7 +1176,7 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
       hipGraph_t g = nullptr;
       HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
       try {
-        enqueue_classes(p, st, false, 1);
+        enqueue_classes(p, st, false);
       } catch (...) {
         (void)hipStreamEndCapture(st, &g);
         if (g) (void)hipGraphDestroy(g);
@@ -1212,13 +1192,11 @@ static void enqueue_plan(BuildPlan& p, const double* dD, double* dG, const doubl
       p.graph_eps = p.eps;
     }
     enqueue_prologue(p, st);
-    enqueue_classes(p, st, false, 2, false);
     HIPCHK(hipGraphLaunch(p.graph, st));
-    join_side_streams(st);
     enqueue_epilogue(p, st);
   } else {
     enqueue_prologue(p, st);
-    enqueue_classes(p, st, timed, 0);
+    enqueue_classes(p, st, timed);
     enqueue_epilogue(p, st);
   }
   if (record) HIPCHK(hipEventRecord(c.ev1, st));
@@ -1295,7 +1273,7 @@ static void enqueue_noalloc(BuildPlan& p, Species& s, const double* dD, double* 
   p.eps = s.screen_eps;
   hipLaunchKernelGGL(store_desc_kernel, dim3(1), dim3(1), 0, st, md, M, sd, Y);
   launch_prologue_batch(md, 1, M.n, st);
-  enqueue_classes(p, st, false, 0, true, md, true);
+  enqueue_classes(p, st, false, md, true);
   launch_symmetrize_batch(md, sd, 1, M.n, st);
   HIPCHK(hipGetLastError());
 }
@@ -1364,7 +1342,7 @@ static void count_coupling(const Species& a, const Species& b, lowdin_fock_stats
 // Enqueue the coupling quartets of species a and b on st: dRa (n_a^2) =
 // coupling on a from dDb and/or dRb (n_b^2) = coupling on b from dDa (device
 // pointers; either result may be null).  Results are zeroed here by a fill
-// kernel; the classes run on the heavy-kernel stream, joined back to st.
+// kernel; the classes run on the side streams and st, joined back to st.
 static void enqueue_coupling(Species& a, Species& b, const double* dDb, double* dRa, const double* dDa, double* dRb,
                              hipStream_t st, lowdin_fock_stats* stt, bool inline_launch = false) {
   Context& c = ctx();
@@ -1373,16 +1351,11 @@ static void enqueue_coupling(Species& a, Species& b, const double* dDb, double* 
   TaskSet* ts = coupling_taskset(a, b, st);
   if (dRa) launch_fill_zero(dRa, (size_t)a.nbasis * a.nbasis, st);
   if (dRb) launch_fill_zero(dRb, (size_t)b.nbasis * b.nbasis, st);
-  // class launches largest first, round robin over the side streams (the
-  // cooperative kernels have no private segment, the per-lane ones at most
-  // a few hundred bytes per lane); inline: all on the caller's stream
-  if (!inline_launch) {
-    HIPCHK(hipEventRecord(c.fork, st));
-    for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
-  }
+  // class launches largest first; inline: all on the caller's stream
+  if (!inline_launch) fork_side_streams(st);
   for (size_t r = 0; r < ts->launches.size(); ++r) {
     const TaskSet::Launch& L = ts->launches[ts->order[r]];
-    hipStream_t hs = inline_launch ? st : c.side[r % kSideStreams];
+    hipStream_t hs = inline_launch ? st : class_stream(r, st);
     const bool a_bra = L.bra_is_a != 0;
     Species& sb = a_bra ? a : b;
     Species& sk = a_bra ? b : a;
@@ -1556,11 +1529,10 @@ static void enqueue_store(Species& s, const double* dD, const double* dC, double
     launch_slab_slots(s.d_slot.ensure((size_t)n * n), s.sig.d_pairs.p, s.sig.d_pidx.p,
                       s.sig.d_pidx.p + (size_t)ns * ns, n, ns, s.sig.off, s.sig.jpoff, st);
   }
-  HIPCHK(hipEventRecord(c.fork, st));
-  for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
+  fork_side_streams(st);
   size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts.launches) {
-    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
+    hipStream_t hs = class_stream(nlaunch++, st);
     StoreArgs g{};
     g.tasks = ts.d_tasks.p + L.off;
     g.ntasks = (int)L.count;
@@ -1623,11 +1595,10 @@ static void enqueue_coupling_store(Species& a, Species& b, const double* dC, dou
   TaskSet* ts = coupling_taskset(a, b, st);
   const size_t na = a.nbasis, nb = b.nbasis;
   if (mode == 1) launch_fill_zero(dOut, na * nb * nb, st);
-  HIPCHK(hipEventRecord(c.fork, st));
-  for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
+  fork_side_streams(st);
   size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts->launches) {
-    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
+    hipStream_t hs = class_stream(nlaunch++, st);
     const bool a_bra = L.bra_is_a != 0;
     Species& sb = a_bra ? a : b;
     Species& sk = a_bra ? b : a;
@@ -1732,11 +1703,10 @@ static void enqueue_g12(Species& s, const double* dD, double* dG, double factor,
   const int n = s.nbasis;
   double* graw = s.d_Graw1.ensure(std::max<size_t>((size_t)n * n, 1));
   launch_fill_zero(graw, (size_t)n * n, st);
-  HIPCHK(hipEventRecord(c.fork, st));
-  for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
+  fork_side_streams(st);
   size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts.launches) {
-    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
+    hipStream_t hs = class_stream(nlaunch++, st);
     G12Args g{};
     g.tasks = ts.d_tasks.p + L.off;
     g.ntasks = (int)L.count;
@@ -1784,11 +1754,10 @@ static void enqueue_g12_coupling(Species& a, Species& b, const double* dDb, doub
   ensure_all(b, st);
   TaskSet* ts = g12_coupling_taskset(a, b, gem.n, st);
   launch_fill_zero(dRa, (size_t)a.nbasis * a.nbasis, st);
-  HIPCHK(hipEventRecord(c.fork, st));
-  for (int q = 0; q < kSideStreams; ++q) HIPCHK(hipStreamWaitEvent(c.side[q], c.fork, 0));
+  fork_side_streams(st);
   size_t nlaunch = 0;
   for (const TaskSet::Launch& L : ts->launches) {
-    hipStream_t hs = c.side[nlaunch++ % kSideStreams];
+    hipStream_t hs = class_stream(nlaunch++, st);
     const bool a_bra = L.bra_is_a != 0;
     Species& sb = a_bra ? a : b;
     Species& sk = a_bra ? b : a;
