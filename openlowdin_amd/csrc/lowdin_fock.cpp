@@ -594,6 +594,13 @@ constexpr long kCoopMinRun = 4;
 // more in zeroed, filled and flushed LDS than the even load gains (C20H42:
 // 512 -> 4096 workgroups 20.9 -> 22.5 ms).
 constexpr double kQuartetIters = 12.0;
+// A strip task is no shorter than this many times its own share of filling
+// and flushing the row strips (a few dozen atomics to scattered lines for each
+// thread).  4 / 8 / 16 / 32: (H2O)10 2.26 / 2.13 / 2.10 / 2.10 ms, (H2O)6 0.84 /
+// 0.82 / 0.79 / 0.84, mixed C13H28 6.94 / 6.90 / 6.83 / 6.80, 4 clusters in a
+// batch 0.166 / 0.165 / 0.165 / 0.175.  Shorter tasks for the high classes,
+// whose quartets cost more, lose as well: 2.64 ms for (H2O)10.
+constexpr double kFlushShare = 16.0;
 // A plan runs as one launch over all classes (jk_fused_kernel) up to this
 // many candidate quartets and tasks (one per bra and ket class).  Above, its
 // one wavefront per SIMD costs more than the side-by-side classes gain: class
@@ -799,7 +806,7 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
     }
     const double flush = 8.0 + (double)(ncart_h(la) + ncart_h(lb)) * p.nmax / block;
     const double goal = (wave64 ? 4.0 : 1.0) * (double)tgt;
-    const double cap = std::max((work + kQuartetIters * (double)total) / goal, 4.0 * block * flush);
+    const double cap = std::max((work + kQuartetIters * (double)total) / goal, kFlushShare * block * flush);
     const long even = (total + tgt - 1) / tgt;   // kets of a cooperative task
     const long chunk = p.fused ? even : std::max(kCoopMinRun, std::min(32768L, (even + 3) / 4 * 4));
     for (int m = 0; m < nm; ++m) {
@@ -832,8 +839,8 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
     append_by_cost(ts.tasks, made);
     ts.launches.push_back({la, lb, lc, ld, cx, cy, 1, from, ts.tasks.size() - from,
                            coop ? coop : (strip ? (wave64 ? 2 : 1) : 0), lmax});
-    // estimated cost of the launch: primitive quartets x class weight
-    cost.push_back(work * (1.0 + (la + lb + lc + ld) * (la + lb + lc + ld)));
+    // estimated cost of the launch: (primitive) quartets x class weight
+    cost.push_back((work + kQuartetIters * (double)total) * (1.0 + (la + lb + lc + ld) * (la + lb + lc + ld)));
   }
   ts.order.resize(ts.launches.size());
   for (size_t k = 0; k < ts.order.size(); ++k) ts.order[k] = k;
