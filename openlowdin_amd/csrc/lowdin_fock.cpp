@@ -194,6 +194,7 @@ struct TaskSet {
     int strip;        // intra: one workgroup per task with LDS row strips (1: 256 threads, 2: 64);
                       // 3: wave-cooperative kernel with row strips, 4: the same without strips
     int lmax = 0;         // intra strips: JKArgs::lmax
+    int block = 256;      // intra strips: threads of a workgroup
   };
   std::vector<Launch> launches;
   std::vector<size_t> order;   // launch order: estimated cost, largest first
@@ -601,6 +602,20 @@ constexpr double kQuartetIters = 12.0;
 // batch 0.166 / 0.165 / 0.165 / 0.175.  Shorter tasks for the high classes,
 // whose quartets cost more, lose as well: 2.64 ms for (H2O)10.
 constexpr double kFlushShare = 16.0;
+// Strip workgroups of two wavefronts instead of four: the kets of a bra fill
+// whole rounds of a workgroup but for the last, in which the first wavefronts
+// work alone, and the quartets above the screen come first.  Four / two by the
+// rule below: (H2O)10 2.06 / 1.91 ms, 72 clusters in a batch 22.7 / 18.1, C20H42
+// 18.6 / 18.2; eight or sixteen add 12 and 40 % to the batch.  High classes,
+// whose quartets are long and few, gain at every size (one wavefront: another
+// -7 % for the batch, +14 and +8 % for (H2O)10 and C20H42); lighter ones only
+// with few kets per bra, otherwise the strips' filling and flushing weighs
+// more (two everywhere for L = 3 below 2000: (H2O)10 +8 %; for L <= 2 below 8000:
+// C20H42 +4 %, (H2O)20 +7 %).
+static bool narrow_strips(int L, double kets_per_bra) {
+  return L >= 4 || kets_per_bra < (L == 3 ? 1000.0 : 2000.0);
+}
+
 // A plan runs as one launch over all classes (jk_fused_kernel) up to this
 // many candidate quartets and tasks (one per bra and ket class).  Above, its
 // one wavefront per SIMD costs more than the side-by-side classes gain: class
@@ -783,13 +798,13 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
     if (kd >= 4) kd = 0;
     const bool strip_ok = (size_t)(ncart_h(la) + ncart_h(lb)) * p.nmax * sizeof(double) <= kStripLdsMax &&
                           maxbra <= kMaxStripPrims;
-    // untuned: strips wherever they fit, of 256 threads when a bra has on
-    // average >= 192 kets, else of one wavefront (short ket runs of small
+    // untuned: strips wherever they fit, of 128 or 256 threads when a bra has
+    // on average >= 192 kets, else of one wavefront (short ket runs of small
     // molecules would leave most of a 256-thread workgroup idle)
     const bool strip = coop || (strip_ok && (kd == 1 || kd == 3 || kd == 0));
     const bool wave64 = kd == 3 || (kd == 0 && total < 192 * nbras);
     const size_t from = ts.tasks.size();
-    const int block = wave64 ? 64 : 256;
+    const int block = wave64 ? 64 : kd == 0 && !coop && narrow_strips(la + lb + lc + ld, (double)total / nbras) ? 128 : 256;
     const long tgt = coop_default ? kCoopDefaultWg : p.fused ? kFusedWg : p.target_wg[class_pair_id(cx, cy)];
     made.clear();
     double work = 0.0;   // primitive quartets of the launch
@@ -838,8 +853,10 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
     }
     append_by_cost(ts.tasks, made);
     ts.launches.push_back({la, lb, lc, ld, cx, cy, 1, from, ts.tasks.size() - from,
-                           coop ? coop : (strip ? (wave64 ? 2 : 1) : 0), lmax});
-    // estimated cost of the launch: (primitive) quartets x class weight
+                           coop ? coop : (strip ? (wave64 ? 2 : 1) : 0), lmax, coop ? 256 : block});
+    // estimated cost of the launch: (primitive) quartets x class weight (by
+    // the longest workgroup instead: C20H42 18.2 -> 17.8 ms, but (H2O)10 1.91
+    // -> 1.98 and 64 clusters in a batch 0.81 -> 0.97)
     cost.push_back((work + kQuartetIters * (double)total) * (1.0 + (la + lb + lc + ld) * (la + lb + lc + ld)));
   }
   ts.order.resize(ts.launches.size());
@@ -1089,7 +1106,7 @@ static void enqueue_classes(BuildPlan& p, hipStream_t st, bool timed, const MolD
     a.cket = L.cket;
     a.same_class = L.cbra == L.cket ? 1 : 0;
     a.lds_n = p.nmax;
-    a.block = L.strip == 2 ? 64 : 256;
+    a.block = L.block;
     if (L.strip == 4) a.lds_n = 0;
     a.eps = p.eps;  // DBL_EPSILON by default (Libint2Iface.h:269-271)
     a.any_mixed = p.any_mixed ? 1 : 0;
