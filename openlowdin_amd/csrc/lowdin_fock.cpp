@@ -74,6 +74,13 @@ struct DevBuf {
 // 2.25, C20H42 + proton coupling 1.20 against 0.98, FHF- 0.66 against 0.49).
 constexpr int kSideStreams = 3;
 
+// Host matrices up to this size pass through pinned memory: the copies of a
+// pageable array wait for the device on their own, 40 us after a small build.
+// Larger ones are copied from and to the caller's array.
+constexpr size_t kPinned = 1 << 20;
+
+constexpr int kNumClassPairs = 21;
+
 struct Context {
   bool ready = false;
   hipStream_t stream = nullptr;
@@ -82,6 +89,9 @@ struct Context {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   DevBuf<double> boys;    // full table (one-body integrals)
   DevBuf<float> boysf;    // FP32 table of its own grid (mixed precision)
+  DevBuf<double> norms;   // overlap norms of the shell pairs of a pair list
+  char* pinned = nullptr;            // kPinned bytes a host call's matrices pass through
+  unsigned long long* hcnt = nullptr;   // pinned: counts of a build
   std::mutex mu;  // one process stream: calls are serialised
 };
 
@@ -145,6 +155,8 @@ static void ensure_context() {
     HIPCHK(hipEventCreateWithFlags(&c.join[k], hipEventDisableTiming));
   }
   HIPCHK(hipEventCreateWithFlags(&c.fork, hipEventDisableTiming));
+  HIPCHK(hipHostMalloc((void**)&c.pinned, kPinned, hipHostMallocDefault));
+  HIPCHK(hipHostMalloc((void**)&c.hcnt, 3 * kNumClassPairs * sizeof(unsigned long long), hipHostMallocDefault));
   HIPCHK(hipEventCreate(&c.ev0));
   HIPCHK(hipEventCreate(&c.ev1));
   std::vector<double> tab = make_boys_table();
@@ -264,7 +276,6 @@ struct Species {
 // the index of their molecule (Task.flags) into a device array of MolDesc.
 // Densities and results are packed: molecule m's n_m x n_m block starts at
 // off[m] elements.
-constexpr int kNumClassPairs = 21;
 struct BuildPlan {
   std::vector<Species*> mols;
   std::vector<uint64_t> sig_gen;        // each molecule's sig_gen when the tasks were built
@@ -1309,8 +1320,9 @@ static void collect_plan_stats(BuildPlan& p, hipStream_t st, double t0) {
   std::vector<unsigned long long> cnt(3 * std::max<size_t>(nl, 1));
   launch_reduce_counts_multi(p.d_task_counts.p, p.d_ranges.p, (int)nl, p.d_cnt.p, st);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(cnt.data(), p.d_cnt.p, cnt.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipMemcpyAsync(c.hcnt, p.d_cnt.p, cnt.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  std::copy(c.hcnt, c.hcnt + cnt.size(), cnt.begin());
   float kms = 0.f;
   HIPCHK(hipEventElapsedTime(&kms, c.ev0, c.ev1));
   lowdin_fock_stats stt{};
@@ -1341,11 +1353,16 @@ static void compute_2body(Species& s, const double* dens, double* result, double
   const size_t nn = (size_t)s.nbasis * s.nbasis;
   if (s.setup_each_build) s.sig.valid = false;
   BuildPlan& p = own_plan(s);
-  s.d_D.upload(dens, nn, st);
+  const size_t bytes = nn * sizeof(double);
+  const bool pin = bytes <= kPinned;
+  // the copy back into the staging memory follows the one out of it
+  if (pin) std::memcpy(c.pinned, dens, bytes);
+  s.d_D.upload(pin ? reinterpret_cast<const double*>(c.pinned) : dens, nn, st);
   s.d_G.ensure(nn);
   enqueue_plan(p, s.d_D.p, s.d_G.p, &factor, st);
-  HIPCHK(hipMemcpyAsync(result, s.d_G.p, nn * sizeof(double), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipMemcpyAsync(pin ? (void*)c.pinned : result, s.d_G.p, bytes, hipMemcpyDeviceToHost, st));
   collect_plan_stats(p, st, t0);
+  if (pin) std::memcpy(result, c.pinned, bytes);
   s.stats = p.stats;
 }
 
@@ -1980,13 +1997,14 @@ void LibintInterface_init_2body_ints(void* lint) {
     lowdin::ensure_device_basis(*s, st);
     const int ns = (int)s->shells.size();
     const size_t npair = (size_t)ns * (ns + 1) / 2;
-    lowdin::DevBuf<double> d_norms;
-    d_norms.ensure(npair);
-    lowdin::launch_pair_norms(s->d_shells.p, s->d_pexp.p, s->d_pcoef.p, ns, d_norms.p, st);
+    const size_t bytes = npair * sizeof(double);
+    const bool pin = bytes <= lowdin::kPinned;
+    c.norms.ensure(npair);
+    lowdin::launch_pair_norms(s->d_shells.p, s->d_pexp.p, s->d_pcoef.p, ns, c.norms.p, st);
     HIPCHK(hipGetLastError());
-    std::vector<double> norms(npair);
-    if (npair)
-      HIPCHK(hipMemcpyAsync(norms.data(), d_norms.p, npair * sizeof(double), hipMemcpyDeviceToHost, st));
+    std::vector<double> far(pin ? 0 : npair);
+    double* norms = pin ? reinterpret_cast<double*>(c.pinned) : far.data();
+    if (npair) HIPCHK(hipMemcpyAsync(norms, c.norms.p, bytes, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     std::vector<std::pair<int, int>> list;
     size_t k = 0;

@@ -224,7 +224,7 @@ struct G12CouplingArgs {
 // with l <= 2, from primitives whose coefficients already carry N(alpha,l).
 // Obara-Saika 1-D recursion S(i+1,j) = PA S(i,j) + (i S(i-1,j) + j S(i,j-1))/(2p).
 __host__ __device__ inline void overlap_block(const ShellInfo& A, const ShellInfo& B, const double* pexp,
-                                              const double* pcoef, double* blk) {
+                                              const double* pcoef, double* blk, int first = 0, int step = 1) {
   const int la = A.l, lb = B.l;
   const int na = (la + 1) * (la + 2) / 2, nb = (lb + 1) * (lb + 2) / 2;
   int ca[6][3], cb[6][3];
@@ -240,28 +240,27 @@ __host__ __device__ inline void overlap_block(const ShellInfo& A, const ShellInf
   const double Ax[3] = {A.x, A.y, A.z}, Bx[3] = {B.x, B.y, B.z};
   double ab2 = 0.0;
   for (int d = 0; d < 3; ++d) ab2 += (Ax[d] - Bx[d]) * (Ax[d] - Bx[d]);
-  for (int i = 0; i < A.nprim; ++i) {
+  for (int ij = first; ij < A.nprim * B.nprim; ij += step) {
+    const int i = ij / B.nprim, j = ij % B.nprim;
     const double a = pexp[A.poff + i], ca_ = pcoef[A.poff + i];
-    for (int j = 0; j < B.nprim; ++j) {
-      const double b = pexp[B.poff + j], cb_ = pcoef[B.poff + j];
-      const double p = a + b, o2p = 0.5 / p;
-      const double pre = ca_ * cb_ * exp(-a * b / p * ab2) * pow(3.14159265358979323846 / p, 1.5);
-      double S[3][3][3];  // [axis][i][j], i, j <= 2
-      for (int d = 0; d < 3; ++d) {
-        const double P = (a * Ax[d] + b * Bx[d]) / p;
-        const double PA = P - Ax[d], PB = P - Bx[d];
-        S[d][0][0] = 1.0;
-        for (int ii = 0; ii < la; ++ii)
-          S[d][ii + 1][0] = PA * S[d][ii][0] + (ii > 0 ? ii * o2p * S[d][ii - 1][0] : 0.0);
-        for (int jj = 0; jj < lb; ++jj)
-          for (int ii = 0; ii <= la; ++ii)
-            S[d][ii][jj + 1] = PB * S[d][ii][jj] + (ii > 0 ? ii * o2p * S[d][ii - 1][jj] : 0.0) +
-                               (jj > 0 ? jj * o2p * S[d][ii][jj - 1] : 0.0);
-      }
-      for (int x = 0; x < na; ++x)
-        for (int y = 0; y < nb; ++y)
-          blk[x * nb + y] += pre * S[0][ca[x][0]][cb[y][0]] * S[1][ca[x][1]][cb[y][1]] * S[2][ca[x][2]][cb[y][2]];
+    const double b = pexp[B.poff + j], cb_ = pcoef[B.poff + j];
+    const double p = a + b, o2p = 0.5 / p;
+    const double pre = ca_ * cb_ * exp(-a * b / p * ab2) * pow(3.14159265358979323846 / p, 1.5);
+    double S[3][3][3];  // [axis][i][j], i, j <= 2
+    for (int d = 0; d < 3; ++d) {
+      const double P = (a * Ax[d] + b * Bx[d]) / p;
+      const double PA = P - Ax[d], PB = P - Bx[d];
+      S[d][0][0] = 1.0;
+      for (int ii = 0; ii < la; ++ii)
+        S[d][ii + 1][0] = PA * S[d][ii][0] + (ii > 0 ? ii * o2p * S[d][ii - 1][0] : 0.0);
+      for (int jj = 0; jj < lb; ++jj)
+        for (int ii = 0; ii <= la; ++ii)
+          S[d][ii][jj + 1] = PB * S[d][ii][jj] + (ii > 0 ? ii * o2p * S[d][ii - 1][jj] : 0.0) +
+                             (jj > 0 ? jj * o2p * S[d][ii][jj - 1] : 0.0);
     }
+    for (int x = 0; x < na; ++x)
+      for (int y = 0; y < nb; ++y)
+        blk[x * nb + y] += pre * S[0][ca[x][0]][cb[y][0]] * S[1][ca[x][1]][cb[y][1]] * S[2][ca[x][2]][cb[y][2]];
   }
 }
 
