@@ -316,7 +316,8 @@ int lowdin_fock_batch_launch_profile(void* batch, int cap, int* classes, float* 
 
 /* Autotuner: for each class launch, the kernel shape is chosen among the
  * wavefront kernel (one bra x 64 kets per wave), the LDS-strip kernel cut
- * into about {512, 2048, 8192} workgroups of 256 threads, the LDS-strip
+ * into about {512, 2048, 8192} workgroups of two or four wavefronts (by the
+ * class and its kets per bra, as untuned), the LDS-strip
  * kernel with one-wavefront workgroups (about 512) and, for total angular
  * momentum >= 5, the wave-cooperative kernel (one quartet per wavefront,
  * with row strips at about {2048, 8192} workgroups or without at about
@@ -351,7 +352,7 @@ int lowdin_fock_targets(void* lint, int* targets);
  * >= OVERLAP_EIGEN_THRESHOLD, 1e-8 unless set), G = q^2 (J + f K) through this library's direct build (skipped
  * when build_two = 0), couplings q_i q_j J_{i<-j} through the device coupling
  * build, F = H + G + C, DIIS (8) on X^T (F D S - S D F) X over all species,
- * rocSOLVER diagonalisation, D = eta C_occ C_occ^T.  E = e_pc +
+ * diagonalisation (one workgroup up to 64 functions, rocSOLVER above), D = eta C_occ C_occ^T.  E = e_pc +
  * sum_s Tr(D_s (H_s + G_s / 2 + C_s / 2)).  No reference counterpart as a C
  * entry point: openLOWDIN runs this loop in Fortran with LAPACK on the host. */
 typedef struct {
@@ -388,7 +389,7 @@ int lowdin_scf_fock_end(void* scf, double* energy, double* error);
 /* DIIS extrapolation and new densities. */
 int lowdin_scf_update(void* scf);
 /* lowdin_scf_update for many SCF objects on one stream: their orthogonalised
- * Fock matrices of equal dimension are diagonalised by one batched rocSOLVER
+ * Fock matrices of equal dimension are diagonalised by one batched
  * call per dimension. */
 int lowdin_scf_update_many(void* const* scfs, int count);
 /* Iterate fock/update until |dE| < e_tol and error < d_tol.  Returns 0 when
@@ -410,7 +411,7 @@ void* lowdin_scf_stream(void* scf);
  * over all jobs: the direct builds of every species in one class launch per
  * quartet class, couplings per species pair, and -- per group of species of
  * equal basis size -- strided-batched GEMMs (error, X^T F X, C, D), one
- * rocsolver dsyevd_strided_batched, and batched kernels for the Fock
+ * batched diagonalisation, and batched kernels for the Fock
  * assembly, traces, error maxima and the DIIS history, B matrix, solve and
  * extrapolation (the DIIS state stays on the device).  While the jobs are
  * unchanged an iteration replays two captured HIP graphs around the

@@ -630,10 +630,10 @@ static bool narrow_strips(int L, double kets_per_bra) {
 // A plan runs as one launch over all classes (jk_fused_kernel) up to this
 // many candidate quartets and tasks (one per bra and ket class).  Above, its
 // one wavefront per SIMD costs more than the side-by-side classes gain: class
-// launches against one launch, us: water 6-31G** 557 / 122, (H2O)3 887 / 219,
-// (H2O)6 1297 / 848, (H2O)10 2665 / 2833, C4H10 cc-pVDZ 1107 / 754, C7H16
-// 2442 / 3106; batches of 4 clusters 718 / 568, of 64 monomers and dimers
-// (1.5e6 quartets, 26000 tasks) 924 / 1352.
+// launches against one launch, us: (H2O)3 6-31G** 545 / 219, (H2O)5 671 / 495,
+// (H2O)6 814 / 784, (H2O)8 1296 / 1720, C4H10 cc-pVDZ 847 / 693, C7H16 2070 /
+// 3060; batches of 4 clusters 461 / 165, of 64 monomers (7e5 quartets, 18000
+// tasks) 401 / 387, of 64 monomers and dimers (1.5e6, 26000) 924 / 1352.
 constexpr double kFusedQuartets = 4.0e6, kFusedTasks = 8.0e3;
 constexpr long kFusedWg = 128;   // strip workgroups a class is cut into at least
 
@@ -815,7 +815,7 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
     const bool strip = coop || (strip_ok && (kd == 1 || kd == 3 || kd == 0));
     const bool wave64 = kd == 3 || (kd == 0 && total < 192 * nbras);
     const size_t from = ts.tasks.size();
-    const int block = wave64 ? 64 : kd == 0 && !coop && narrow_strips(la + lb + lc + ld, (double)total / nbras) ? 128 : 256;
+    const int block = wave64 ? 64 : !coop && narrow_strips(la + lb + lc + ld, (double)total / nbras) ? 128 : 256;
     const long tgt = coop_default ? kCoopDefaultWg : p.fused ? kFusedWg : p.target_wg[class_pair_id(cx, cy)];
     made.clear();
     double work = 0.0;   // primitive quartets of the launch
@@ -2546,7 +2546,7 @@ static int plan_autotune(lowdin::BuildPlan& p, const double* d_dens, double* d_r
   lowdin::ensure_context();
   hipStream_t st = stream ? stream : c.stream;
   // candidates: the wavefront kernel, LDS strips aiming at that many
-  // workgroups per launch, and LDS strips with one-wavefront workgroups
+  // workgroups per launch (of the default width), and LDS strips with one-wavefront workgroups
   static const int cand[][2] = {{2, 2048}, {1, 512}, {1, 2048}, {1, 8192}, {3, 512}, {4, 2048},
                                 {4, 8192}, {5, 2048}, {5, 8192}, {5, 32768}};   // {kind, workgroups}
   const bool tl = p.time_launches, se = p.serialize, ug = p.use_graph;

@@ -22,8 +22,8 @@
 // graphs around the diagonalisation: (build, couplings, assembly, traces,
 // error, DIIS, X^T F X) and (C = X C', D = C diag(occ) C^T, scalar copy).
 // The first iteration after a change runs eagerly (it also prepares the
-// build's task lists); the next one captures.  rocsolver runs outside the
-// graphs.
+// build's task lists); the next one captures.  The diagonalisation
+// runs outside the graphs.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>

@@ -1,8 +1,8 @@
 """Device-resident SCF: the multi-species Hartree-Fock iteration of
 openLOWDIN (src/scf/MultiSCF.f90:276-440, 730-1002; WaveFunction.f90:394-467,
 817-1535, 1768-2003) with every matrix in HBM (``lowdin_scf_*`` in
-liblowdin_fock.so: rocBLAS/rocSOLVER for the dense algebra, this library's
-direct Fock and coupling builds for G and C).  Same iteration, DIIS and
+liblowdin_fock.so: rocBLAS products, this library's diagonalisation (rocSOLVER
+above 64 functions) and direct Fock and coupling builds).  Same iteration, DIIS and
 convergence test as :func:`openlowdin_amd.wavefunction.run_scf`, which keeps
 the dense algebra on the host.
 """
