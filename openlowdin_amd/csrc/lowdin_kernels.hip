@@ -230,33 +230,36 @@ __global__ void symmetrize_kernel(const double* Graw, int n, double scale, doubl
 // (blockIdx.y): G_raw and Jp cleared, the normalised density blocks of the
 // pairs packed into Dp, and (where the build screens or runs mixed precision)
 // the shell-block norms of D.  One launch: each part is far shorter than a
-// launch, so a small build pays for launches alone.
+// launch, so a small build pays for launches alone.  8 lanes take the rows of
+// a shell block, one lane each matrix element: a lane per pair and per block
+// ran through up to 36 loads one after another (water 11 us,
+// so 5.6; C20H42 13, 7.5).
 __global__ void prologue_batch_kernel(const MolDesc* mols) {
   const MolDesc& M = mols[blockIdx.y];
-  const int nsh = M.nshell, n = M.n, npairs = M.off[6], njp = M.jpoff[6];
-  const int first = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
-  double* G = M.Graw;
-  double* Jp = M.Jp;
-  for (int k = first; k < n * n; k += stride) G[k] = 0.0;
-  for (int k = first; k < njp; k += stride) Jp[k] = 0.0;
-  for (int k = first; k < npairs; k += stride) {
-    const PairInfo* P = M.pairs + k;
-    const int la = P->la, lb = P->lb, c = la * (la + 1) / 2 + lb;
-    const int na = ncart_(la), nb = ncart_(lb), ncls = M.off[c + 1] - M.off[c];
-    const int bfa = P->bfa, bfb = P->bfb;
-    double* out = M.Dp + M.jpoff[c] + (k - M.off[c]);
-    for (int i = 0; i < na; ++i)
-      for (int j = 0; j < nb; ++j)
-        out[(size_t)(i * nb + j) * ncls] =
-            M.D[(size_t)(bfa + i) * n + bfb + j] * M.norma[bfa + i] * M.norma[bfb + j];
-  }
-  if (!(M.screen || M.mixed)) return;
-  for (int k = first; k < nsh * nsh; k += stride) {
-    const ShellInfo A = M.shells[k / nsh], B = M.shells[k % nsh];
-    double m = 0.0;
-    for (int i = 0; i < ncart_(A.l); ++i)
-      for (int j = 0; j < ncart_(B.l); ++j) m = fmax(m, fabs(M.D[(size_t)(A.bf + i) * n + B.bf + j]));
-    M.Dn[k] = m;
+  const int nsh = M.nshell, n = M.n;
+  const int nblk = M.screen || M.mixed ? 8 * nsh * nsh : 0;
+  for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < nblk + n * n; w += gridDim.x * blockDim.x) {
+    if (w < nblk) {
+      const int k = w >> 3, r = w & 7;
+      const ShellInfo A = M.shells[k / nsh], B = M.shells[k % nsh];
+      const int na = ncart_(A.l), nb = ncart_(B.l);
+      const double* row = M.D + (size_t)(A.bf + min(r, na - 1)) * n + B.bf;
+      double m = 0.0;
+#pragma unroll
+      for (int j = 0; j < 6; ++j) m = fmax(m, fabs(row[min(j, nb - 1)]));
+      for (int o = 4; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+      if (r == 0) M.Dn[k] = m;
+    } else {
+      const int e = w - nblk, i = e / n, k = e % n;
+      M.Graw[e] = 0.0;
+      const int q = M.pidx[M.fsh[i] * nsh + M.fsh[k]];
+      if (q < 0) continue;   // no pair, or the pair of (k, i)
+      const PairInfo* P = M.pairs + q;
+      const int la = P->la, lb = P->lb, c = la * (la + 1) / 2 + lb, ncls = M.off[c + 1] - M.off[c];
+      const size_t slot = M.jpoff[c] + (size_t)((i - P->bfa) * ncart_(lb) + (k - P->bfb)) * ncls + (q - M.off[c]);
+      M.Dp[slot] = M.D[e] * M.norma[i] * M.norma[k];
+      M.Jp[slot] = 0.0;
+    }
   }
 }
 
@@ -479,7 +482,7 @@ void launch_symmetrize(const double* Graw, int n, double scale, double* G, hipSt
 
 void launch_prologue_batch(const MolDesc* mols, int nmol, int nmax, hipStream_t s) {
   if (nmol <= 0 || nmax <= 0) return;
-  const int blocks = std::min((nmax * nmax + 255) / 256, 1024);
+  const int blocks = std::min((3 * nmax * nmax + 255) / 256, 2048);
   hipLaunchKernelGGL(prologue_batch_kernel, dim3(blocks, nmol), dim3(256), 0, s, mols);
 }
 
