@@ -631,10 +631,15 @@ static bool narrow_strips(int L, double kets_per_bra) {
 // many candidate quartets and tasks (one per bra and ket class).  Above, its
 // one wavefront per SIMD costs more than the side-by-side classes gain: class
 // launches against one launch, us: (H2O)3 6-31G** 545 / 219, (H2O)5 671 / 495,
-// (H2O)6 814 / 784, (H2O)8 1296 / 1720, C4H10 cc-pVDZ 847 / 693, C7H16 2070 /
+// (H2O)6 814 / 766, (H2O)8 1296 / 1720, C4H10 cc-pVDZ 847 / 646, C7H16 2070 /
 // 3060; batches of 4 clusters 461 / 165, of 64 monomers (7e5 quartets, 18000
 // tasks) 401 / 387, of 64 monomers and dimers (1.5e6, 26000) 924 / 1352.
 constexpr double kFusedQuartets = 4.0e6, kFusedTasks = 8.0e3;
+// split_shift's lmax of such a plan by total angular momentum: the light
+// classes fill its wavefronts by their number, the high ones are its longest
+// chains.  16 for all / this: C4H10 684 / 646 us, (H2O)6 780 / 765, water 117 /
+// 116; 32 for all: C4H10 641, water 162; 8 for the high ones: (H2O)4 365 / 381.
+constexpr int kFusedSplit[6] = {32, 32, 24, 24, 16, 16};
 constexpr long kFusedWg = 128;   // strip workgroups a class is cut into at least
 
 static inline int class_pair_id(int cx, int cy) { return cx * (cx + 1) / 2 + cy; }
@@ -829,6 +834,7 @@ static void build_plan_tasks(BuildPlan& p, hipStream_t st) {
     int lmax = 0;
     if (strip && !coop) {
       lmax = (int)std::max(kSplitMin, std::min(kSplitMax, (double)total / (kSplitKets * (double)nbras)));
+      if (p.fused) lmax = kFusedSplit[la + lb + lc + ld];
     }
     const double flush = 8.0 + (double)(ncart_h(la) + ncart_h(lb)) * p.nmax / block;
     const double goal = (wave64 ? 4.0 : 1.0) * (double)tgt;
