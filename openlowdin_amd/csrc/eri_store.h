@@ -27,9 +27,71 @@ namespace lowdin {
 // Blocks up to this many integrals get fully unrolled element loops.
 constexpr int kStoreFullUnroll = 216;
 
+// Elements of one block have the same eight index images where the shells of
+// a pair are the same, or bra and ket are the same pair: ((a b) and (b a), (c d)
+// and (d c), (ab|cd) and (cd|ab)).  Their recursions round differently, and
+// lanes that share a block store them side by side, so they get one value (the
+// later element's, or the other's where that one was dropped) before any is
+// stored: all images of an integral hold the same bits, whatever the timing.
+// w: the raw block, in registers or (kShared) in LDS, where lane takes every 64th
+// element.  The norms of the four functions are multiplied in pairs, (a b) by
+// (c d), which rounds alike for all of them.
+__device__ __forceinline__ void join_elements(double& later, double& other, double drop) {
+  const double v = fabs(later) > drop ? later : other;
+  later = v;
+  other = v;
+}
+
+template <bool kShared>
+__device__ __forceinline__ void join_fence() {
+  if constexpr (kShared) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <bool kShared, int NA, int NB, int NC, int ND>
+__device__ __forceinline__ void join_images(double* w, bool bdiag, bool kdiag, bool same, double drop, int lane) {
+  constexpr int N = NA * NB * NC * ND, kTurns = kShared ? (N + 63) / 64 : N, U = kShared ? 1 : N;
+  if constexpr (NC == ND) {
+    if (kdiag) {
+      join_fence<kShared>();
+#pragma unroll U
+      for (int t = 0; t < kTurns; ++t) {
+        const int e = kShared ? 64 * t + lane : t;
+        const int id = e % ND, ic = e / ND % NC, ab = e / (NC * ND);
+        if (e < N && ic > id) join_elements(w[e], w[(ab * NC + id) * ND + ic], drop);
+      }
+    }
+  }
+  if constexpr (NA == NB) {
+    if (bdiag) {
+      join_fence<kShared>();
+#pragma unroll U
+      for (int t = 0; t < kTurns; ++t) {
+        const int e = kShared ? 64 * t + lane : t;
+        const int cd = e % (NC * ND), ib = e / (NC * ND) % NB, ia = e / (NC * ND * NB);
+        if (e < N && ia > ib) join_elements(w[e], w[(ib * NB + ia) * NC * ND + cd], drop);
+      }
+    }
+  }
+  if constexpr (NA == NC && NB == ND) {
+    if (same) {
+      join_fence<kShared>();
+#pragma unroll U
+      for (int t = 0; t < kTurns; ++t) {
+        const int e = kShared ? 64 * t + lane : t;
+        const int id = e % ND, ic = e / ND % NC, ib = e / (NC * ND) % NB, ia = e / (NC * ND * NB);
+        // an order of the pairs that (a b) and (b a) agree on
+        const int ab = (max(ia, ib) * 8 + min(ia, ib)) * 8 + ia, cd = (max(ic, id) * 8 + min(ic, id)) * 8 + ic;
+        if (e < N && ab > cd) join_elements(w[e], w[((ic * ND + id) * NA + ia) * NB + ib], drop);
+      }
+    }
+  }
+  join_fence<kShared>();
+}
+
 // The eight index images of one kept integral of an intra-species quartet.
-// Images that coincide are written by this lane only, so the result does not
-// depend on timing.
 __device__ __forceinline__ void store_images(double* A, size_t n, size_t i, size_t j, size_t k, size_t l, double v) {
   const size_t n2 = n * n, n3 = n2 * n;
   A[i * n3 + j * n2 + k * n + l] = v;
@@ -75,6 +137,7 @@ __global__ __launch_bounds__(256) void store_kernel(StoreArgs a) {
   for (int i = 0; i < NC; ++i) nc[i] = nrm[K.bfa + i];
 #pragma unroll
   for (int i = 0; i < ND; ++i) nd[i] = nrm[K.bfb + i];
+  join_images<false, NA, NB, NC, ND>(out, P.sa == P.sb, K.sa == K.sb, a.same_class && j == t.bra, a.drop, 0);
   int turn = 0;
 #pragma unroll U1
   for (int ia = 0; ia < NA; ++ia)
@@ -88,7 +151,7 @@ __global__ __launch_bounds__(256) void store_kernel(StoreArgs a) {
           const bool mine = (turn++ & ((1 << ls) - 1)) == sub;
           if (mine && fabs(v) > a.drop)
             store_images(a.out, a.n, P.bfa + ia, P.bfb + ib, K.bfa + ic, K.bfb + id,
-                         v * na[ia] * nb[ib] * nc[ic] * nd[id]);
+                         v * ((na[ia] * nb[ib]) * (nc[ic] * nd[id])));
         }
 }
 
@@ -255,14 +318,16 @@ __global__ __launch_bounds__(64) void store_coop_kernel(StoreArgs a) {
     coop_quartet<LA, LB, LC, LD>(R, Pg::prog() + lane, prim + (size_t)P.poff * kPrimPairStride, P.nprim,
                                  prim + (size_t)K.poff * kPrimPairStride, K.nprim, a.boys, P, K, lane);
     double* out = R + Pg::kOut;
+    if constexpr (MODE == 0)
+      join_images<true, NA, NB, NC, ND>(out, P.sa == P.sb, K.sa == K.sb, a.same_class && j == t.bra, a.drop, lane);
     for (int e = lane; e < NA * NB * NC * ND; e += 64) {
       const int id = e % ND, ic = e / ND % NC, ib = e / (ND * NC) % NB, ia = e / (ND * NC * NB);
       const double v = out[e];
-      const double w = fabs(v) > a.drop ? v * nrm[P.bfa + ia] * nrm[P.bfb + ib] * nrm[K.bfa + ic] * nrm[K.bfb + id] : 0.0;
+      const double nn = (nrm[P.bfa + ia] * nrm[P.bfb + ib]) * (nrm[K.bfa + ic] * nrm[K.bfb + id]);
       if constexpr (MODE == 0) {
-        if (w != 0.0) store_images(a.out, a.n, P.bfa + ia, P.bfb + ib, K.bfa + ic, K.bfb + id, w);
+        if (fabs(v) > a.drop) store_images(a.out, a.n, P.bfa + ia, P.bfb + ib, K.bfa + ic, K.bfb + id, v * nn);
       } else {
-        out[e] = w;
+        out[e] = fabs(v) > a.drop ? v * nn : 0.0;
       }
     }
     if constexpr (MODE == 1) {
