@@ -212,8 +212,9 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
     if (w == 0) {
       const double dr = lane < n ? d[lane] : 0.0, er = lane < n - 1 ? e[lane] : 0.0;
       // [l, hi]: first block without a negligible e
-      const unsigned long long small = __ballot(
-          lane >= n - 1 || fabs(er) <= fmax(2.220446049250313e-16 * (fabs(dr) + fabs(__shfl_down(dr, 1))), 1e-18));
+      const double dn = __shfl_down(dr, 1);   // of all lanes: it reads the neighbour's register
+      const unsigned long long small =
+          __ballot(lane >= n - 1 || fabs(er) <= fmax(2.220446049250313e-16 * (fabs(dr) + fabs(dn)), 1e-18));
       int hi = l;
       for (; l < n - 1; ++l, iter = 0) {
         const unsigned long long from = small >> l << l;
