@@ -4,8 +4,8 @@
 //
 // The orthogonalised Fock matrix of an iteration is small (two water
 // molecules in 6-31G**: 50), and a library call takes some hundred dependent
-// launches over it.  Measured, library / here: n = 25 0.63 / 0.18, 50 1.25 /
-// 0.53, 64 1.70 / 0.84 ms; 72 matrices at once take as long as one.  Past 64
+// launches over it.  Measured, library / here: n = 25 0.64 / 0.17, 50 1.30 /
+// 0.57, 64 1.69 / 0.90 ms; 72 matrices at once take as long as one.  Past 64
 // a row no longer fits a lane and the library changes its method: with two
 // rows per lane 75 1.16 / 1.32, 100 1.63 / 2.14 ms.  (Parallel Jacobi over the
 // same LDS: 50 0.49, 75 1.13 ms, with twice to four times the loss of
@@ -17,7 +17,12 @@
 //     a barrier;
 //   * QL, the longest: one lane chases the bulge of the next sweep (a chain of
 //     some 14 dependent operations for each of the n^2 rotations, 0.14 us)
-//     while a second wavefront applies the last sweep's, one row per lane.
+//     while a second wavefront applies the last sweep's, one row per lane;
+//   * one step of refinement against the matrix itself, five products on the
+//     matrix unit (10 us at n = 64): rotations alone leave residuals up to twice
+//     the library's.  Worst of 6 matrices of 4 kinds each at n = 64, library /
+//     rotations / refined: |AV - VW| / |A| 2.0e-15 / 2.7e-15 / 1.0e-15,
+//     |V^T V - 1| 1.4e-14 / 1.8e-14 / 0.5e-14.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -75,13 +80,48 @@ __device__ __forceinline__ double rsqrt_cubic(double x) {
   return fma(y * h, fma(0.375, h, 0.5), y);
 }
 
+// 16 x 16 tile (I, J) of c + X Y of n x n matrices on the matrix unit, x(i, k)
+// and y(k, j) their elements: a lane's four are rows 16 I + lane / 16 + 4 r,
+// column 16 J + lane % 16.
+typedef double double4v __attribute__((ext_vector_type(4)));
+
+template <typename X, typename Y>
+__device__ __forceinline__ double4v tile_product(double4v c, int n, int I, int J, int lane, X x, Y y) {
+  const int i = 16 * I + (lane & 15), j = 16 * J + (lane & 15);
+  for (int k0 = 0; k0 < n; k0 += 4) {
+    const int k = k0 + (lane >> 4);
+    const double a = i < n && k < n ? x(i, k) : 0.0, b = k < n && j < n ? y(k, j) : 0.0;
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  return c;
+}
+
+template <typename F>
+__device__ __forceinline__ void tile_each(int n, int I, int J, int lane, F f) {
+  const int j = 16 * J + (lane & 15);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = 16 * I + (lane >> 4) + 4 * r;
+    if (i < n && j < n) f(i, j, r);
+  }
+}
+
+// Tile t of those on and above the diagonal, by columns.
+__device__ __forceinline__ int2 upper_tile(int t) {
+  int J = 0;
+  while ((J + 1) * (J + 2) / 2 <= t) ++J;
+  return make_int2(t - J * (J + 1) / 2, J);
+}
+
 __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
   extern __shared__ double lds[];
   const int n = g.n, tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  double* A = lds;                          // A[c n + i]: row i of column c
-  double* part = A + n * n;                 // kSyevWaves x n partial products
-  double* d = part + kSyevWaves * n;
+  const int ld = n | 1;                     // odd: columns side by side use different banks
+  double* A = lds;                          // A[c ld + i]: row i of column c
+  double* B = A + n * ld;                   // second matrix of the last step
+  double* part = B;                         // kSyevWaves x n partial products
+  double* d = B + max(n * ld, kSyevWaves * n);
   double* e = d + n;
   double* tau = e + n;
   double* rot = tau + n;                    // two sweeps of (c, s)
@@ -95,7 +135,7 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
   for (int k = tid; k < n * n; k += kSyevThreads) {
     const int c = k / n, i = k % n;
     const double v = G[(size_t)max(i, c) * n + min(i, c)];
-    A[k] = v;
+    A[c * ld + i] = v;
     mx = fabs(v) < INFINITY ? fmax(mx, fabs(v)) : INFINITY;
   }
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
@@ -109,19 +149,19 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
   }
   int ex = 0;
   if (mx > 0.0) (void)frexp(mx, &ex);
-  for (int k = tid; k < n * n; k += kSyevThreads) A[k] = ldexp(A[k], -ex);
+  for (int k = tid; k < n * ld; k += kSyevThreads) A[k] = ldexp(A[k], -ex);
   __syncthreads();
 
   // Step j: reflector H = 1 - tau v v^T (v[j+1] = 1) of column j below the
   // diagonal, A22 -= v u^T + u v^T.
   for (int j = 0; j < n - 2; ++j) {
     const bool below = lane > j && lane < n;
-    double v = below ? A[j * n + lane] : 0.0;
+    double v = below ? A[j * ld + lane] : 0.0;
     const double x0 = lane_value(v, j + 1);
     const double s2 = wave_total(lane > j + 1 ? v * v : 0.0);
     if (s2 < 1e-290) {   // nothing to eliminate (to 1e-145 of the largest element)
       if (tid == 0) {
-        d[j] = A[j * n + j];
+        d[j] = A[j * ld + j];
         e[j] = x0;
         tau[j] = 0.0;
       }
@@ -134,7 +174,7 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
     double y = 0.0;
     const int c0 = j + 1 + ((w - j - 1) & (kSyevWaves - 1));   // first own column
     for (int c = c0; c < n; c += kSyevWaves)
-      if (lane < n) y = fma(A[c * n + lane], lane_value(v, c), y);
+      if (lane < n) y = fma(A[c * ld + lane], lane_value(v, c), y);
     if (lane < n) part[w * n + lane] = y;
     __syncthreads();
     y = 0.0;
@@ -144,9 +184,9 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
     }
     y = t * fma(-0.5 * t * wave_total(y * v), v, y);
     if (w == 0) {
-      if (below) A[j * n + lane] = v;
+      if (below) A[j * ld + lane] = v;
       if (lane == 0) {
-        d[j] = A[j * n + j];
+        d[j] = A[j * ld + j];
         e[j] = beta;
         tau[j] = t;
       }
@@ -154,13 +194,13 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
     for (int c = c0; c < n; c += kSyevWaves) {
       const double vc = lane_value(v, c), yc = lane_value(y, c);
       // products rounded one by one: both triangles get the same bits
-      if (below) A[c * n + lane] -= __dadd_rn(__dmul_rn(v, yc), __dmul_rn(y, vc));
+      if (below) A[c * ld + lane] -= __dadd_rn(__dmul_rn(v, yc), __dmul_rn(y, vc));
     }
     __syncthreads();
   }
   if (tid == 0) {
-    for (int j = n > 2 ? n - 2 : 0; j < n; ++j) d[j] = A[j * n + j];
-    if (n > 1) e[n - 2] = A[(n - 2) * n + n - 1];
+    for (int j = n > 2 ? n - 2 : 0; j < n; ++j) d[j] = A[j * ld + j];
+    if (n > 1) e[n - 2] = A[(n - 2) * ld + n - 1];
   }
   __syncthreads();
 
@@ -180,7 +220,7 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int i = sub + 16 * k;
-        v[k] = i > j && i < n ? A[j * n + i] : 0.0;
+        v[k] = i > j && i < n ? A[j * ld + i] : 0.0;
       }
 #pragma unroll
       for (int b = 0; b < kSyevPasses; ++b) {
@@ -198,7 +238,7 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int c = col + kCols * b, i = sub + 16 * k;
-        if (c < n && i < n) A[c * n + i] = q[b][k];
+        if (c < n && i < n) A[c * ld + i] = q[b][k];
       }
   }
   __syncthreads();
@@ -268,7 +308,7 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
     }
     const int r = tid - 64;
     if (r >= 0 && r < n) {
-      double f = A[hi * n + r];
+      double f = A[hi * ld + r];
       int k = hi - 1;
       for (; k >= lo + 3; k -= 4) {
         double c[4], s[4], zk[4];
@@ -276,22 +316,75 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
         for (int u = 0; u < 4; ++u) {
           c[u] = cs[2 * (k - u)];
           s[u] = cs[2 * (k - u) + 1];
-          zk[u] = A[(k - u) * n + r];
+          zk[u] = A[(k - u) * ld + r];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          A[(k - u + 1) * n + r] = fma(c[u], f, s[u] * zk[u]);
+          A[(k - u + 1) * ld + r] = fma(c[u], f, s[u] * zk[u]);
           f = fma(c[u], zk[u], -s[u] * f);
         }
       }
       for (; k >= lo; --k) {
-        const double c = cs[2 * k], s = cs[2 * k + 1], zk = A[k * n + r];
-        A[(k + 1) * n + r] = fma(c, f, s * zk);
+        const double c = cs[2 * k], s = cs[2 * k + 1], zk = A[k * ld + r];
+        A[(k + 1) * ld + r] = fma(c, f, s * zk);
         f = fma(c, zk, -s * f);
       }
-      A[lo * n + r] = f;
+      A[lo * ld + r] = f;
     }
   }
+
+  // One step of refinement: with S = V^T A V and R = 1 - V^T V of the vectors
+  // found, w = S_ii / (1 - R_ii) and V += V E, E_ij = R_ij / 2 + X_ij, X_ij =
+  // (S_ij + (w_i + w_j) R_ij / 2) / (w_j - w_i) = -X_ji where that is small
+  // enough for its square to vanish, else 0 (levels as close as that rotate
+  // into each other by rounding alone).
+  const int nt = (n + 15) >> 4;             // tiles of 16 x 16
+  __syncthreads();
+  for (int k = tid; k < n * n; k += kSyevThreads) {
+    const int c = k / n, i = k % n;
+    B[c * ld + i] = ldexp(G[(size_t)max(i, c) * n + min(i, c)], -ex);
+  }
+  __syncthreads();
+  double4v acc[2];
+  for (int u = 0, t = w; t < nt * nt; ++u, t += kSyevWaves)
+    acc[u] = tile_product(double4v{}, n, t / nt, t % nt, lane, [&](int i, int k) { return B[k * ld + i]; },
+                          [&](int k, int j) { return A[j * ld + k]; });
+  __syncthreads();
+  for (int u = 0, t = w; t < nt * nt; ++u, t += kSyevWaves)
+    tile_each(n, t / nt, t % nt, lane, [&](int i, int j, int r) { B[j * ld + i] = acc[u][r]; });   // A V
+  __syncthreads();
+  double4v S[2], N[2];                      // V^T A V, V^T V: tiles I <= J
+  for (int u = 0, t = w; t < nt * (nt + 1) / 2; ++u, t += kSyevWaves) {
+    const int2 b = upper_tile(t);
+    const auto row = [&](int i, int k) { return A[i * ld + k]; };
+    S[u] = tile_product(double4v{}, n, b.x, b.y, lane, row, [&](int k, int j) { return B[j * ld + k]; });
+    N[u] = tile_product(double4v{}, n, b.x, b.y, lane, row, [&](int k, int j) { return A[j * ld + k]; });
+    tile_each(n, b.x, b.y, lane, [&](int i, int j, int r) {
+      if (i == j) d[i] = S[u][r] / N[u][r];
+    });
+  }
+  __syncthreads();
+  for (int u = 0, t = w; t < nt * (nt + 1) / 2; ++u, t += kSyevWaves) {
+    const int2 b = upper_tile(t);
+    tile_each(n, b.x, b.y, lane, [&](int i, int j, int r) {
+      if (i > j) return;
+      const double half = 0.5 * (i == j ? 1.0 - N[u][r] : -N[u][r]);
+      const double num = fma(d[i] + d[j], half, S[u][r]), gap = d[j] - d[i];
+      const double x = i != j && fabs(num) < 1e-9 * fabs(gap) ? num / gap : 0.0;
+      B[j * ld + i] = half + x;
+      if (i != j) B[i * ld + j] = half - x;
+    });
+  }
+  __syncthreads();
+  for (int u = 0, t = w; t < nt * nt; ++u, t += kSyevWaves) {
+    double4v v{};
+    tile_each(n, t / nt, t % nt, lane, [&](int i, int j, int r) { v[r] = A[j * ld + i]; });
+    acc[u] = tile_product(v, n, t / nt, t % nt, lane, [&](int i, int k) { return A[k * ld + i]; },
+                          [&](int k, int j) { return B[j * ld + k]; });
+  }
+  __syncthreads();
+  for (int u = 0, t = w; t < nt * nt; ++u, t += kSyevWaves)
+    tile_each(n, t / nt, t % nt, lane, [&](int i, int j, int r) { A[j * ld + i] = acc[u][r]; });
 
   // ascending order (equal values keep theirs)
   int* rank = (int*)rot;
@@ -306,12 +399,13 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
   __syncthreads();
   for (int k = tid; k < n * n; k += kSyevThreads) {
     const int c = k / n, i = k % n;
-    G[(size_t)rank[c] * n + i] = A[k];
+    G[(size_t)rank[c] * n + i] = A[c * ld + i];
   }
 }
 
 size_t syev_lds(int n) {
-  return sizeof(double) * ((size_t)n * n + (size_t)(kSyevWaves + 7) * n + kSyevWaves) + 8 * sizeof(int);
+  const int nld = n * (n | 1), second = nld > kSyevWaves * n ? nld : kSyevWaves * n;
+  return sizeof(double) * (size_t)(nld + second + 7 * n + kSyevWaves) + 8 * sizeof(int);
 }
 
 }  // namespace
@@ -319,6 +413,10 @@ size_t syev_lds(int n) {
 bool launch_syev(double* a, int n, size_t stride_a, double* w, size_t stride_w, int* info, int count, hipStream_t s) {
   if (n < 1 || n > kSyevMax) return false;
   if (count <= 0) return true;
+  // above 64 KB from n = 62
+  static const hipError_t attr = hipFuncSetAttribute(
+      (const void*)syev_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)syev_lds(kSyevMax));
+  (void)attr;
   const SyevArgs g{a, w, info, stride_a, stride_w, n};
   hipLaunchKernelGGL(syev_kernel, dim3(count), dim3(kSyevThreads), syev_lds(n), s, g);
   return true;
