@@ -324,8 +324,9 @@ int lowdin_fock_batch_launch_profile(void* batch, int cap, int* classes, float* 
  * {2048, 8192, 32768}), by timing `reps` serialised builds per candidate on
  * the given inputs.  Classes of total angular momentum >= 6 run only the
  * wave-cooperative kernel (the per-lane kernels would spill to scratch).
- * Small FP64 builds (up to about 4e6 candidate quartets) run as one launch over
- * all classes whatever the choices.
+ * Small FP64 builds (up to about 4e6 candidate quartets, fewer above 360
+ * functions) run as one launch over all classes whatever the choices; a build or
+ * batch with any mixed-precision species has one launch per class.
  * Results are unchanged by the choice up to FP64 summation order. */
 int lowdin_fock_batch_autotune(void* batch, const double* d_dens, double* d_result, const double* factors,
                                void* stream, int reps);

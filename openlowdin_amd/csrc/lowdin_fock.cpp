@@ -634,6 +634,13 @@ static bool narrow_strips(int L, double kets_per_bra) {
 // (H2O)6 814 / 766, (H2O)8 1296 / 1720, C4H10 cc-pVDZ 847 / 646, C7H16 2070 /
 // 3060; batches of 4 clusters 461 / 165, of 64 monomers (7e5 quartets, 18000
 // tasks) 401 / 387, of 64 monomers and dimers (1.5e6, 26000) 924 / 1352.
+// Its workgroups hold row strips for the largest class, 12 n doubles of LDS:
+// where fewer than four fit in a CU (n above 360; 514: three to two) the
+// quartets allowed fall with the square of the wavefronts in flight.  Waters
+// 14 A apart, class launches against one launch, us: n = 400 (0.8e6 quartets)
+// 819 / 615, 500 (1.2e6) 937 / 888, 525 (1.3e6) 946 / 1364, 675 (2.2e6) 1124 /
+// 2089; 12 and 14 methanes cc-pVDZ (n = 420, 490; 2.2e6, 3.0e6) 1054 / 1093 and
+// 1146 / 1418; 136 sites of two s and a p shell (n = 680, 0.3e6) 255 / 180.
 constexpr double kFusedQuartets = 4.0e6, kFusedTasks = 8.0e3;
 // split_shift's lmax of such a plan by total angular momentum: the light
 // classes fill its wavefronts by their number, the high ones are its longest
@@ -641,6 +648,8 @@ constexpr double kFusedQuartets = 4.0e6, kFusedTasks = 8.0e3;
 // 116; 32 for all: C4H10 641, water 162; 8 for the high ones: (H2O)4 365 / 381.
 constexpr int kFusedSplit[6] = {32, 32, 24, 24, 16, 16};
 constexpr long kFusedWg = 128;   // strip workgroups a class is cut into at least
+constexpr size_t kLdsPerCu = 163840;
+constexpr size_t kFusedStaticLds = kMaxStripPrims * kPrimPairStride * sizeof(double) + 16;   // beside jk_fused_lds
 
 static inline int class_pair_id(int cx, int cy) { return cx * (cx + 1) / 2 + cy; }
 
@@ -732,6 +741,9 @@ static void append_by_cost(std::vector<Task>& tasks, std::vector<std::pair<doubl
 // Whether a plan runs as one launch over all quartet classes.
 static bool want_fused(const BuildPlan& p) {
   if (p.time_launches || p.serialize) return false;   // per-class times are wanted
+  int nmax = 0;
+  for (const Species* s : p.mols) nmax = std::max(nmax, s->nbasis);
+  const double fit = std::min<size_t>(4, kLdsPerCu / (jk_fused_lds(nmax) + kFusedStaticLds));
   double quartets = 0.0, tasks = 0.0;   // tasks: one per bra and ket class
   for (const Species* s : p.mols) {
     const PairSet& ps = s->sig;
@@ -740,7 +752,7 @@ static bool want_fused(const BuildPlan& p) {
       return false;
     quartets += 0.5 * (double)ps.pairs.size() * (double)ps.pairs.size();
     for (int c = 0; c < kNumPairClasses; ++c) tasks += (double)(ps.off[c + 1] - ps.off[c]) * (c + 1);
-    if (quartets > kFusedQuartets || tasks > kFusedTasks) return false;
+    if (quartets > kFusedQuartets * fit * fit / 16.0 || tasks > kFusedTasks) return false;
   }
   return true;
 }
