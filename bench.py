@@ -56,10 +56,10 @@ def cpu_baseline(sp, D, stride, eris_full):
 
 def kernel_name(code, target, tuned):
     """Kernel template that ran class `code` (e.g. "2121") under the
-    autotuner choice `target` (lowdin_fock_targets encoding).  Untuned plans
-    run the wave-cooperative kernel from total L = 6 and LDS strips below."""
+    autotuner choice `target` (lowdin_fock_targets encoding).  From total
+    L = 6 only the wave-cooperative kernel runs, below LDS strips by default."""
     args = ", ".join(code)
-    if target >= 1000000 or (not tuned and sum(int(c) for c in code) >= 6):
+    if target >= 1000000 or sum(int(c) for c in code) >= 6:
         return "jk_coop_kernel<%s>" % args
     if tuned and target == 0:
         return "jk_kernel<%s>" % args

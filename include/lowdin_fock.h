@@ -315,14 +315,16 @@ int lowdin_fock_batch_launch_profile(void* batch, int cap, int* classes, float* 
                                      uint64_t* prim_quartets);
 
 /* Autotuner: for each class launch, the kernel shape is chosen among the
- * wavefront kernel (one bra x 64 kets per wave), the LDS-strip kernel cut
- * into about {512, 2048, 8192} workgroups of two or four wavefronts (by the
- * class and its kets per bra, as untuned), the LDS-strip
+ * default one, the wavefront kernel (one bra x 64 kets per wave), the LDS-strip
+ * kernel cut into about {512, 2048, 8192} workgroups of two or four wavefronts
+ * (by the class and its kets per bra, as untuned), the LDS-strip
  * kernel with one-wavefront workgroups (about 512) and, for total angular
  * momentum >= 5, the wave-cooperative kernel (one quartet per wavefront,
  * with row strips at about {2048, 8192} workgroups or without at about
  * {2048, 8192, 32768}), by timing `reps` serialised builds per candidate on
- * the given inputs.  Classes of total angular momentum >= 6 run only the
+ * the given inputs.  The choices are kept if the whole build, its launches side
+ * by side, is faster with them than with the default shapes and with those it
+ * had.  Classes of total angular momentum >= 6 run only the
  * wave-cooperative kernel (the per-lane kernels would spill to scratch).
  * Small FP64 builds (up to about 4e6 candidate quartets, fewer above 360
  * functions) run as one launch over all classes whatever the choices; a build or

@@ -2554,8 +2554,13 @@ int lowdin_fock_batch_launch_profile(void* batch, int cap, int* classes, float* 
   return plan_profile(static_cast<lowdin_fock_batch_t*>(batch)->plan, cap, classes, ms, quartets, prim_quartets);
 }
 
-// Per class launch: try each candidate workgroup target on serialised,
-// event-timed builds and keep the fastest (ties to the smaller target).
+// Per class launch: try each candidate on serialised, event-timed builds and
+// keep the fastest; ties go to the default shapes, which come first.  The
+// classes of a build run side by side, where a launch that is faster alone may
+// take more from the others than it gains, so the choices are kept only if
+// the whole build is faster with them than with the defaults and with what the
+// plan had (C13H28 7.00 ms by default, 7.40-7.50 with the fastest launch of
+// each class; 72 water clusters in a batch 18.1 and 16.4).
 static int plan_autotune(lowdin::BuildPlan& p, const double* d_dens, double* d_result, const double* factors,
                          hipStream_t stream, int reps, const double* const* dD_each = nullptr,
                          double* const* dG_each = nullptr) {
@@ -2563,33 +2568,60 @@ static int plan_autotune(lowdin::BuildPlan& p, const double* d_dens, double* d_r
   std::lock_guard<std::mutex> lk(c.mu);
   lowdin::ensure_context();
   hipStream_t st = stream ? stream : c.stream;
-  // candidates: the wavefront kernel, LDS strips aiming at that many
-  // workgroups per launch (of the default width), and LDS strips with one-wavefront workgroups
-  static const int cand[][2] = {{2, 2048}, {1, 512}, {1, 2048}, {1, 8192}, {3, 512}, {4, 2048},
+  // candidates: the default shape, the wavefront kernel, LDS strips aiming at that many
+  // workgroups per launch (of the default width), LDS strips with one-wavefront workgroups and
+  // the cooperative kernel
+  static const int cand[][2] = {{0, 512}, {2, 2048}, {1, 512}, {1, 2048}, {1, 8192}, {3, 512}, {4, 2048},
                                 {4, 8192}, {5, 2048}, {5, 8192}, {5, 32768}};   // {kind, workgroups}
+  constexpr int K = lowdin::kNumClassPairs;
+  struct Choice {
+    int kind[K], wg[K];
+  } before, standard, pick;
+  double best[K];
+  for (int k = 0; k < K; ++k) {
+    best[k] = 1e300;
+    before.kind[k] = pick.kind[k] = p.kind[k];
+    before.wg[k] = pick.wg[k] = p.target_wg[k];
+    standard.kind[k] = cand[0][0];
+    standard.wg[k] = cand[0][1];
+  }
+  const auto use = [&](const Choice& x) {
+    std::copy(x.kind, x.kind + K, p.kind);
+    std::copy(x.wg, x.wg + K, p.target_wg);
+    p.valid = false;
+  };
+  const auto build = [&] {
+    lowdin::enqueue_plan(p, d_dens, d_result, factors, st, dD_each, dG_each);
+    lowdin::collect_plan_stats(p, st, lowdin::now_ms());
+  };
+  const auto overlapped = [&](const Choice& x) {   // least device time of a build
+    use(x);
+    double ms = 1e300;
+    for (int r = 0; r < reps + 3; ++r) {
+      build();
+      if (r > 0) ms = std::min(ms, p.stats.kernel_ms);
+    }
+    return ms;
+  };
   const bool tl = p.time_launches, se = p.serialize, ug = p.use_graph;
+  const auto restore = [&] {
+    p.time_launches = tl;
+    p.serialize = se;
+    p.use_graph = ug;
+  };
   p.time_launches = true;
   p.serialize = true;
   p.use_graph = false;
-  double best[lowdin::kNumClassPairs];
-  int pick[lowdin::kNumClassPairs], pick_kind[lowdin::kNumClassPairs];
-  for (int k = 0; k < lowdin::kNumClassPairs; ++k) {
-    best[k] = 1e300;
-    pick[k] = p.target_wg[k];
-    pick_kind[k] = p.kind[k];
-  }
   try {
     for (const auto& cd : cand) {
       const int kind = cd[0], wg = cd[1];
-      for (int k = 0; k < lowdin::kNumClassPairs; ++k) {
-        p.kind[k] = kind;
-        p.target_wg[k] = wg;
-      }
-      p.valid = false;
+      Choice all;
+      std::fill(all.kind, all.kind + K, kind);
+      std::fill(all.wg, all.wg + K, wg);
+      use(all);
       std::vector<double> ms;
       for (int r = 0; r < reps + 1; ++r) {
-        lowdin::enqueue_plan(p, d_dens, d_result, factors, st, dD_each, dG_each);
-        lowdin::collect_plan_stats(p, st, lowdin::now_ms());
+        build();
         if (r == 0) {
           ms.assign(p.ts.launches.size(), 0.0);
           continue;  // warm-up
@@ -2599,34 +2631,31 @@ static int plan_autotune(lowdin::BuildPlan& p, const double* d_dens, double* d_r
       for (size_t k = 0; k < p.ts.launches.size(); ++k) {
         const lowdin::TaskSet::Launch& L = p.ts.launches[k];
         const int id = lowdin::class_pair_id(L.cbra, L.cket);
-        if (kind != 2 && !L.strip) continue;   // strips impossible for this class: candidate ran as waves
-        if ((kind >= 4) != (L.strip >= 3)) continue;   // no cooperative kernel, or a default one ran
+        if (kind != 0 && kind != 2 && !L.strip) continue;   // strips impossible for this class: candidate ran as waves
+        if (kind != 0 && (kind >= 4) != (L.strip >= 3)) continue;   // no cooperative kernel, or a default one ran
         if (ms[k] < 0.97 * best[id]) {
           best[id] = ms[k];
-          pick[id] = wg;
-          pick_kind[id] = kind;
+          pick.wg[id] = wg;
+          pick.kind[id] = kind;
         }
       }
     }
-  } catch (...) {
-    for (int k = 0; k < lowdin::kNumClassPairs; ++k) {
-      p.target_wg[k] = pick[k];
-      p.kind[k] = pick_kind[k];
+    p.time_launches = false;
+    p.serialize = false;
+    // small plans run as one launch whatever the choices: those stay for when
+    // the plan's molecules grow
+    if (!lowdin::want_fused(p)) {
+      const double with = overlapped(pick), without = overlapped(standard), was = overlapped(before);
+      if (!(with < 0.99 * without)) pick = standard;
+      if (!(std::min(with, without) < 0.99 * was)) pick = before;
     }
-    p.valid = false;
-    p.time_launches = tl;
-    p.serialize = se;
-    p.use_graph = ug;
+  } catch (...) {
+    use(before);
+    restore();
     throw;
   }
-  for (int k = 0; k < lowdin::kNumClassPairs; ++k) {
-    p.target_wg[k] = pick[k];
-    p.kind[k] = pick_kind[k];
-  }
-  p.valid = false;
-  p.time_launches = tl;
-  p.serialize = se;
-  p.use_graph = ug;
+  use(pick);
+  restore();
   return 0;
 }
 

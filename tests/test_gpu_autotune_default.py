@@ -1,0 +1,39 @@
+"""The autotuner keeps its choices only where the whole build gains: a tuned
+build is not slower than the untuned one, and gives the same result."""
+import time
+
+import numpy as np
+import pytest
+
+from openlowdin_amd import hip as H
+from openlowdin_amd import libint2_interface as LI
+from openlowdin_amd import system as S
+
+pytestmark = pytest.mark.gpu
+
+
+def test_tuned_build_is_not_slower_than_the_default():
+    sp = S.alkane(13).species[0]
+    n = sp.nbasis
+    X = np.random.default_rng(17).normal(size=(n, sp.n_occupied)) / np.sqrt(n)
+    dD, dG = H.DeviceArray.from_host(2.0 * X @ X.T), H.DeviceArray((n, n))
+
+    def least(h):
+        t = []
+        for _ in range(12):
+            t0 = time.perf_counter()
+            h.compute_2body_device(dD.ptr, dG.ptr, -0.5)
+            t.append(time.perf_counter() - t0)
+        return min(t), dG.download()
+
+    h, g = LI.Libint2Interface(sp, 1), LI.Libint2Interface(sp, 1)
+    for x in (h, g):
+        x.init_2body_ints()
+    g.compute_2body_device(dD.ptr, dG.ptr, -0.5)
+    g.autotune(dD.ptr, dG.ptr, -0.5, reps=1)
+    untuned, Gu = least(h)
+    tuned, Gt = least(g)
+    h.close()
+    g.close()
+    assert np.max(np.abs(Gt - Gu)) < 1e-12 * max(1.0, np.max(np.abs(Gu)))
+    assert tuned < 1.03 * untuned, (tuned, untuned)
