@@ -165,10 +165,16 @@ const char* lowdin_fock_last_error(void);
  * with norma.  Returns 0 on success. */
 int lowdin_fock_1body(void* lint, int kind, int ncharge, const double* Z, const double* xyz, double* result);
 
+/* Fock builds count what was evaluated, after the density screen.  Couplings
+ * (Coulomb and geminal) and stores count the reference's loops: every pair of
+ * one species with every pair of the other (stores of one species: before the
+ * density screen).  Of a coupling's quartets the library evaluates those whose
+ * Schwarz bound reaches a tenth of the 1e-10 drop; the others hold no integral
+ * that is kept. */
 typedef struct {
-  uint64_t quartets;        /* shell quartets evaluated by the last build */
-  uint64_t eris;            /* contracted ERIs (the reference's num_ints_computed) */
-  uint64_t prim_quartets;   /* primitive quartets evaluated */
+  uint64_t quartets;        /* shell quartets of the last build */
+  uint64_t eris;            /* their contracted ERIs (the reference's num_ints_computed) */
+  uint64_t prim_quartets;   /* their primitive quartets */
   double kernel_ms;         /* device time of the integral kernels (HIP events) */
   double total_ms;          /* wall time of the call */
   uint64_t quartets_fp32;   /* of `quartets`, evaluated in FP32 (mixed precision) */
