@@ -554,21 +554,17 @@ __device__ __forceinline__ void coop_coupling_update(double* R, const CouplingAr
 // ket pairs).  No private segment: the state of
 // a quartet lives in the wavefront's LDS region.
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(256, 2) void coupling_coop_kernel(CouplingArgs a) {
+__global__ __launch_bounds__(64, 2) void coupling_coop_kernel(CouplingArgs a) {
   using Pg = CoopProgram<LA, LB, LC, LD>;
-  constexpr int kWave = coop_wave_doubles<LA, LB, LC, LD>();
-  extern __shared__ double lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nw = blockDim.x >> 6;
+  extern __shared__ double R[];
+  const int lane = threadIdx.x;
   const Task t = a.tasks[blockIdx.x];
   const PairInfo P = load_pair((gcptr<PairInfo>)a.bra + t.bra);
-  double* R = lds + w * kWave;
   if (lane < 2) R[kCoopZero + lane] = 0.0;
   coop_coupling_weights<LA, LB, LC, LD>(R, a, P, lane);
   const gcptr<double> bprim = (gcptr<double>)a.bprim + (size_t)P.poff * kPrimPairStride;
   const uint2* pg = Pg::prog() + lane;
-  for (int j = t.j0 + w; j < t.j1; j += nw) {
+  for (int j = t.j0; j < t.j1; ++j) {
     const PairInfo K = load_pair((gcptr<PairInfo>)a.ket + j);
     const gcptr<double> kprim = (gcptr<double>)a.kprim + (size_t)K.poff * kPrimPairStride;
     coop_quartet<LA, LB, LC, LD>(R, pg, bprim, P.nprim, kprim, K.nprim, a.boys, P, K, lane);

@@ -294,10 +294,7 @@ __device__ __forceinline__ void contracted_quartet_f32_body(BP bprim, int nbp, K
 // Quartet evaluation is inlined into every kernel of a class: an
 // out-of-line body for the largest classes doubled their scratch (the
 // integral array then lives in the caller's private segment as well) and
-// the runtime could not provision it at full occupancy.  The two largest
-// classes ((dd|dp), (dd|dd): single-primitive d shells in every workload
-// here) keep FP64 in mixed mode, which halves their code and compile time.
-constexpr int kMaxNaccFp32 = 300;
+// the runtime could not provision it at full occupancy.
 
 template <int LA, int LB, int LC, int LD, typename BP, typename KP, typename TP>
 __device__ __forceinline__ void contracted_quartet(BP bprim, int nbp, KP kprim, int nkp, TP boys, double ABx,
@@ -306,11 +303,6 @@ __device__ __forceinline__ void contracted_quartet(BP bprim, int nbp, KP kprim, 
   contracted_quartet_body<LA, LB, LC, LD>(bprim, nbp, kprim, nkp, boys, ABx, ABy, ABz, CDx, CDy, CDz, out, sub,
                                           nsplit);
 }
-
-template <int LA, int LB, int LC, int LD>
-struct Fp32Allowed {
-  static constexpr bool value = EriClass<LA, LB, LC, LD>::nacc <= kMaxNaccFp32;
-};
 
 template <int LA, int LB, int LC, int LD, typename BP, typename KP>
 __device__ __forceinline__ void contracted_quartet_f32(BP bprim, int nbp, KP kprim, int nkp,
@@ -469,7 +461,7 @@ __global__ __launch_bounds__(256) void jk_kernel(JKArgs a) {
   if (active && (M.screen || M.mixed)) {
     const double dn = quartet_dnorm((gcptr<double>)M.Dn, ns, P, K);
     if (M.screen && dn * P.Q * K.Q < a.eps) active = false;
-    lo = Fp32Allowed<LA, LB, LC, LD>::value && M.mixed && dn * P.Qn * K.Qn < M.tau;
+    lo = M.mixed && dn * P.Qn * K.Qn < M.tau;
   }
   const uint64_t amask = __ballot(active);
   if (a.counts) {
@@ -490,14 +482,12 @@ __global__ __launch_bounds__(256) void jk_kernel(JKArgs a) {
   for (int k = 0; k < NA * NB; ++k) jab[k] = 0.0;
   if (active) {
     double out[NA * NB * NC * ND];
-    if constexpr (Fp32Allowed<LA, LB, LC, LD>::value) {
-      if (lo)
-        contracted_quartet_f32<LA, LB, LC, LD>((gcptr<float>)M.primf + (size_t)P.poff * kPrimPairStride, P.nprim,
-                                               (gcptr<float>)M.primf + (size_t)K.poff * kPrimPairStride, K.nprim,
-                                               a.boysf,
-                                               P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
-    }
-    if (!lo)
+    if (lo)
+      contracted_quartet_f32<LA, LB, LC, LD>((gcptr<float>)M.primf + (size_t)P.poff * kPrimPairStride, P.nprim,
+                                             (gcptr<float>)M.primf + (size_t)K.poff * kPrimPairStride, K.nprim,
+                                             a.boysf,
+                                             P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
+    else
       contracted_quartet<LA, LB, LC, LD>(prim + (size_t)P.poff * kPrimPairStride, P.nprim,
                                          prim + (size_t)K.poff * kPrimPairStride, K.nprim, a.boys,
                                          P.ABx, P.ABy, P.ABz, K.ABx, K.ABy, K.ABz, out);
@@ -825,12 +815,11 @@ __device__ __forceinline__ void jk_strip_body(const JKArgs& a, const Task& t, un
 
 template <int LA, int LB, int LC, int LD>
 __global__ __launch_bounds__(256, (StripWaves<LA, LB, LC, LD>::value)) void jk_strip_kernel(JKArgs a) {
-  constexpr bool kF32 = Fp32Allowed<LA, LB, LC, LD>::value;
   extern __shared__ double strip[];
   __shared__ double bpd[kMaxStripPrims * kPrimPairStride];
-  __shared__ float bpf[kF32 ? kMaxStripPrims * kPrimPairStride : 1];
+  __shared__ float bpf[kMaxStripPrims * kPrimPairStride];
   __shared__ unsigned int wg[3];
-  jk_strip_body<LA, LB, LC, LD, kF32, StripLdsBoys<LA, LB, LC, LD>::value>(
+  jk_strip_body<LA, LB, LC, LD, true, StripLdsBoys<LA, LB, LC, LD>::value>(
       a, a.tasks[blockIdx.x], a.counts ? a.counts + 3 * blockIdx.x : nullptr, strip, bpd, bpf, wg);
 }
 

@@ -24,9 +24,6 @@
 
 namespace lowdin {
 
-// Blocks up to this many integrals get fully unrolled element loops.
-constexpr int kStoreFullUnroll = 216;
-
 // Elements of one block have the same eight index images where the shells of
 // a pair are the same, or bra and ket are the same pair: ((a b) and (b a), (c d)
 // and (d c), (ab|cd) and (cd|ab)).  Their recursions round differently, and
@@ -109,10 +106,6 @@ __device__ __forceinline__ void store_images(double* A, size_t n, size_t i, size
 template <int LA, int LB, int LC, int LD>
 __global__ __launch_bounds__(256) void store_kernel(StoreArgs a) {
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-  // Element loops: fully unrolled for small blocks; for large ones the two
-  // outer levels stay loops, which keeps code size and compile time bounded.
-  constexpr bool kFull = NA * NB * NC * ND <= kStoreFullUnroll;
-  constexpr int U1 = kFull ? 6 : 1;
   const int wid = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
   if (wid >= a.ntasks) return;
   const Task t = a.tasks[wid];
@@ -139,9 +132,9 @@ __global__ __launch_bounds__(256) void store_kernel(StoreArgs a) {
   for (int i = 0; i < ND; ++i) nd[i] = nrm[K.bfb + i];
   join_images<false, NA, NB, NC, ND>(out, P.sa == P.sb, K.sa == K.sb, a.same_class && j == t.bra, a.drop, 0);
   int turn = 0;
-#pragma unroll U1
+#pragma unroll
   for (int ia = 0; ia < NA; ++ia)
-#pragma unroll U1
+#pragma unroll
     for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
       for (int ic = 0; ic < NC; ++ic)
@@ -295,9 +288,10 @@ __global__ __launch_bounds__(256) void it_strip_kernel(StoreArgs a) {
 
 // ------------------------------------- one wavefront per quartet (high L)
 // One lane per quartet kept these classes' blocks in scratch: (H2O)3 6-31G**
-// (dd|dd) 1060 -> 33 us, (dd|dp) 901 -> 31, the store 4.0 -> 0.56 ms.  Store (MODE 0) or transform (MODE 1, packed slabs as above, every update a
-// global atomic: these classes have few quartets): the lanes share the
-// elements of the (ab|cd) block in LDS.
+// (dd|dd) 1060 -> 33 us, (dd|dp) 901 -> 31, the store 4.0 -> 0.56 ms.  Store
+// (MODE 0) or transform (MODE 1, packed slabs as above, every update a global
+// atomic: these classes have few quartets): the lanes share the elements of the
+// (ab|cd) block in LDS.
 template <int LA, int LB, int LC, int LD, int MODE>
 __global__ __launch_bounds__(64) void store_coop_kernel(StoreArgs a) {
   using Pg = CoopProgram<LA, LB, LC, LD>;
@@ -367,11 +361,6 @@ __global__ __launch_bounds__(64) void store_coop_kernel(StoreArgs a) {
 template <int LA, int LB, int LC, int LD>
 __global__ __launch_bounds__(256) void coupling_store_kernel(CouplingStoreArgs a) {
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-  // Element loops: fully unrolled for small blocks; for large ones (the
-  // block lives in private memory anyway) the two outer levels stay loops,
-  // which keeps code size and compile time bounded.
-  constexpr bool kFull = NA * NB * NC * ND <= kStoreFullUnroll;
-  constexpr int U1 = kFull ? 6 : 1;
   const int wid = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
   if (wid >= a.ntasks) return;
   const Task t = a.tasks[wid];
@@ -396,9 +385,9 @@ __global__ __launch_bounds__(256) void coupling_store_kernel(CouplingStoreArgs a
 #pragma unroll
   for (int i = 0; i < ND; ++i) nd[i] = a.nket_norma[K.bfb + i];
   // drop (|raw| < drop dropped) and normalise
-#pragma unroll U1
+#pragma unroll
   for (int ia = 0; ia < NA; ++ia)
-#pragma unroll U1
+#pragma unroll
     for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
       for (int ic = 0; ic < NC; ++ic)
@@ -412,9 +401,9 @@ __global__ __launch_bounds__(256) void coupling_store_kernel(CouplingStoreArgs a
   if (a.mode == 0) {
     double* A = a.out;
     const size_t s1 = a.sx1, s2 = a.sx2, s3 = a.sy1;
-#pragma unroll U1
+#pragma unroll
     for (int ia = 0; ia < NA; ++ia)
-#pragma unroll U1
+#pragma unroll
       for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
         for (int ic = 0; ic < NC; ++ic)
@@ -438,9 +427,9 @@ __global__ __launch_bounds__(256) void coupling_store_kernel(CouplingStoreArgs a
   const size_t no = (size_t)a.n_o, no2 = no * no;
   if (a.bra_is_t) {
     // transformed pair (a b), other pair (c d)
-#pragma unroll U1
+#pragma unroll
     for (int ib = 0; ib < NB; ++ib)
-#pragma unroll U1
+#pragma unroll
       for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
         for (int id = 0; id < ND; ++id) {
@@ -453,9 +442,9 @@ __global__ __launch_bounds__(256) void coupling_store_kernel(CouplingStoreArgs a
             global_add(GG + (size_t)(P.bfb + ib) * no2 + (size_t)min(fc, fd) * no + max(fc, fd), s);
         }
     if (!bdiag) {
-#pragma unroll U1
+#pragma unroll
       for (int ia = 0; ia < NA; ++ia)
-#pragma unroll U1
+#pragma unroll
         for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
           for (int id = 0; id < ND; ++id) {
@@ -470,9 +459,9 @@ __global__ __launch_bounds__(256) void coupling_store_kernel(CouplingStoreArgs a
     }
   } else {
     // transformed pair (c d), other pair (a b)
-#pragma unroll U1
+#pragma unroll
     for (int id = 0; id < ND; ++id)
-#pragma unroll U1
+#pragma unroll
       for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib) {
@@ -485,9 +474,9 @@ __global__ __launch_bounds__(256) void coupling_store_kernel(CouplingStoreArgs a
             global_add(GG + (size_t)(K.bfb + id) * no2 + (size_t)min(fa, fb) * no + max(fa, fb), s);
         }
     if (!kdiag) {
-#pragma unroll U1
+#pragma unroll
       for (int ic = 0; ic < NC; ++ic)
-#pragma unroll U1
+#pragma unroll
         for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
           for (int ib = 0; ib < NB; ++ib) {
