@@ -25,67 +25,25 @@
 namespace lowdin {
 
 // Elements of one block have the same eight index images where the shells of
-// a pair are the same, or bra and ket are the same pair: ((a b) and (b a), (c d)
-// and (d c), (ab|cd) and (cd|ab)).  Their recursions round differently, and
-// lanes that share a block store them side by side, so they get one value (the
-// later element's, or the other's where that one was dropped) before any is
-// stored: all images of an integral hold the same bits, whatever the timing.
-// w: the raw block, in registers or (kShared) in LDS, where lane takes every 64th
-// element.  The norms of the four functions are multiplied in pairs, (a b) by
-// (c d), which rounds alike for all of them.
-__device__ __forceinline__ void join_elements(double& later, double& other, double drop) {
-  const double v = fabs(later) > drop ? later : other;
-  later = v;
-  other = v;
-}
-
-template <bool kShared>
-__device__ __forceinline__ void join_fence() {
-  if constexpr (kShared) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+// a pair are the same, or bra and ket are the same pair: (a b) and (b a), (c d)
+// and (d c), (ab|cd) and (cd|ab).  Their recursions round differently, and
+// lanes that share a block store it side by side, so only the last kept one of
+// them is stored: all images of an integral hold the same bits, whatever the
+// timing.  True where a later element than (ia ib|ic id) is stored for it.
+template <int NA, int NB, int NC, int ND>
+__device__ __forceinline__ bool stored_later(const double* w, int ia, int ib, int ic, int id, bool bdiag, bool kdiag,
+                                             bool same, double drop) {
+  const int e = ((ia * NB + ib) * NC + ic) * ND + id;
+  bool later = false;
+#pragma unroll
+  for (int t = 1; t < 8; ++t) {
+    const bool k = t & 1, b = t & 2, s = t & 4;   // swap c and d, a and b, bra and ket
+    if ((k && NC != ND) || (b && NA != NB) || (s && (NA != NC || NB != ND))) continue;
+    const int x = b ? ib : ia, y = b ? ia : ib, z = k ? id : ic, u = k ? ic : id;
+    const int f = s ? ((z * NB + u) * NC + x) * ND + y : ((x * NB + y) * NC + z) * ND + u;
+    if (f > e) later = later || ((!k || kdiag) && (!b || bdiag) && (!s || same) && fabs(w[f]) > drop);
   }
-}
-
-template <bool kShared, int NA, int NB, int NC, int ND>
-__device__ __forceinline__ void join_images(double* w, bool bdiag, bool kdiag, bool same, double drop, int lane) {
-  constexpr int N = NA * NB * NC * ND, kTurns = kShared ? (N + 63) / 64 : N, U = kShared ? 1 : N;
-  if constexpr (NC == ND) {
-    if (kdiag) {
-      join_fence<kShared>();
-#pragma unroll U
-      for (int t = 0; t < kTurns; ++t) {
-        const int e = kShared ? 64 * t + lane : t;
-        const int id = e % ND, ic = e / ND % NC, ab = e / (NC * ND);
-        if (e < N && ic > id) join_elements(w[e], w[(ab * NC + id) * ND + ic], drop);
-      }
-    }
-  }
-  if constexpr (NA == NB) {
-    if (bdiag) {
-      join_fence<kShared>();
-#pragma unroll U
-      for (int t = 0; t < kTurns; ++t) {
-        const int e = kShared ? 64 * t + lane : t;
-        const int cd = e % (NC * ND), ib = e / (NC * ND) % NB, ia = e / (NC * ND * NB);
-        if (e < N && ia > ib) join_elements(w[e], w[(ib * NB + ia) * NC * ND + cd], drop);
-      }
-    }
-  }
-  if constexpr (NA == NC && NB == ND) {
-    if (same) {
-      join_fence<kShared>();
-#pragma unroll U
-      for (int t = 0; t < kTurns; ++t) {
-        const int e = kShared ? 64 * t + lane : t;
-        const int id = e % ND, ic = e / ND % NC, ib = e / (NC * ND) % NB, ia = e / (NC * ND * NB);
-        // an order of the pairs that (a b) and (b a) agree on
-        const int ab = (max(ia, ib) * 8 + min(ia, ib)) * 8 + ia, cd = (max(ic, id) * 8 + min(ic, id)) * 8 + ic;
-        if (e < N && ab > cd) join_elements(w[e], w[((ic * ND + id) * NA + ia) * NB + ib], drop);
-      }
-    }
-  }
-  join_fence<kShared>();
+  return later;
 }
 
 // The eight index images of one kept integral of an intra-species quartet.
@@ -130,7 +88,11 @@ __global__ __launch_bounds__(256) void store_kernel(StoreArgs a) {
   for (int i = 0; i < NC; ++i) nc[i] = nrm[K.bfa + i];
 #pragma unroll
   for (int i = 0; i < ND; ++i) nd[i] = nrm[K.bfb + i];
-  join_images<false, NA, NB, NC, ND>(out, P.sa == P.sb, K.sa == K.sb, a.same_class && j == t.bra, a.drop, 0);
+  // only (c d) and (d c) can coincide: one comparison for half of the elements,
+  // by itself (in stored_later's form the spilling (dp|pp) takes 250-270 us of a
+  // (H2O)3 store instead of 205)
+  constexpr bool kKetOnly = NA != NB && NC == ND;
+  const bool bdiag = P.sa == P.sb, kdiag = K.sa == K.sb, same = a.same_class && j == t.bra;
   int turn = 0;
 #pragma unroll
   for (int ia = 0; ia < NA; ++ia)
@@ -141,10 +103,15 @@ __global__ __launch_bounds__(256) void store_kernel(StoreArgs a) {
 #pragma unroll
         for (int id = 0; id < ND; ++id) {
           const double v = out[((ia * NB + ib) * NC + ic) * ND + id];
-          const bool mine = (turn++ & ((1 << ls) - 1)) == sub;
+          bool mine = (turn++ & ((1 << ls) - 1)) == sub;
+          if constexpr (kKetOnly) {
+            if (ic < id) mine = mine && !(kdiag && fabs(out[((ia * NB + ib) * NC + id) * ND + ic]) > a.drop);
+          } else {
+            mine = mine && !stored_later<NA, NB, NC, ND>(out, ia, ib, ic, id, bdiag, kdiag, same, a.drop);
+          }
           if (mine && fabs(v) > a.drop)
             store_images(a.out, a.n, P.bfa + ia, P.bfb + ib, K.bfa + ic, K.bfb + id,
-                         v * ((na[ia] * nb[ib]) * (nc[ic] * nd[id])));
+                         v * na[ia] * nb[ib] * nc[ic] * nd[id]);
         }
 }
 
@@ -312,21 +279,20 @@ __global__ __launch_bounds__(64) void store_coop_kernel(StoreArgs a) {
     coop_quartet<LA, LB, LC, LD>(R, Pg::prog() + lane, prim + (size_t)P.poff * kPrimPairStride, P.nprim,
                                  prim + (size_t)K.poff * kPrimPairStride, K.nprim, a.boys, P, K, lane);
     double* out = R + Pg::kOut;
-    if constexpr (MODE == 0)
-      join_images<true, NA, NB, NC, ND>(out, P.sa == P.sb, K.sa == K.sb, a.same_class && j == t.bra, a.drop, lane);
+    const bool sab = P.sa != P.sb, scd = K.sa != K.sb;
+    const bool spk = !(a.same_class && j == t.bra);
     for (int e = lane; e < NA * NB * NC * ND; e += 64) {
       const int id = e % ND, ic = e / ND % NC, ib = e / (ND * NC) % NB, ia = e / (ND * NC * NB);
       const double v = out[e];
-      const double nn = (nrm[P.bfa + ia] * nrm[P.bfb + ib]) * (nrm[K.bfa + ic] * nrm[K.bfb + id]);
+      const double w = fabs(v) > a.drop ? v * nrm[P.bfa + ia] * nrm[P.bfb + ib] * nrm[K.bfa + ic] * nrm[K.bfb + id] : 0.0;
       if constexpr (MODE == 0) {
-        if (fabs(v) > a.drop) store_images(a.out, a.n, P.bfa + ia, P.bfb + ib, K.bfa + ic, K.bfb + id, v * nn);
+        if (w != 0.0 && !stored_later<NA, NB, NC, ND>(out, ia, ib, ic, id, !sab, !scd, !spk, a.drop))
+          store_images(a.out, a.n, P.bfa + ia, P.bfb + ib, K.bfa + ic, K.bfb + id, w);
       } else {
-        out[e] = fabs(v) > a.drop ? v * nn : 0.0;
+        out[e] = w;
       }
     }
     if constexpr (MODE == 1) {
-      const bool sab = P.sa != P.sb, scd = K.sa != K.sb;
-      const bool spk = !(a.same_class && j == t.bra);
       for (int e = lane; e < NC * ND * (NA + NB); e += 64) {   // (ab|cd), (ba|cd)
         const int x = e / (NC * ND), id = e % ND, ic = e / ND % NC;
         if (!scd && ic > id) continue;
