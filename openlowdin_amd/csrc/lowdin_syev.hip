@@ -4,8 +4,8 @@
 //
 // The orthogonalised Fock matrix of an iteration is small (two water
 // molecules in 6-31G**: 50), and a library call takes some hundred dependent
-// launches over it.  Measured, library / here: n = 25 0.64 / 0.17, 50 1.30 /
-// 0.57, 64 1.69 / 0.90 ms; 72 matrices at once take as long as one.  Past 64
+// launches over it.  Measured, library / here: n = 25 0.64 / 0.17, 50 1.29 /
+// 0.55, 64 1.70 / 0.88 ms; 72 matrices at once take as long as one.  Past 64
 // a row no longer fits a lane and the library changes its method: with two
 // rows per lane 75 1.16 / 1.32, 100 1.63 / 2.14 ms.  (Parallel Jacobi over the
 // same LDS: 50 0.49, 75 1.13 ms, with twice to four times the loss of
@@ -88,10 +88,16 @@ typedef double double4v __attribute__((ext_vector_type(4)));
 template <typename X, typename Y>
 __device__ __forceinline__ double4v tile_product(double4v c, int n, int I, int J, int lane, X x, Y y) {
   const int i = 16 * I + (lane & 15), j = 16 * J + (lane & 15);
-  for (int k0 = 0; k0 < n; k0 += 4) {
-    const int k = k0 + (lane >> 4);
-    const double a = i < n && k < n ? x(i, k) : 0.0, b = k < n && j < n ? y(k, j) : 0.0;
-    c = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  for (int k0 = 0; k0 < n; k0 += 16) {   // the same for all lanes
+    double a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = k0 + 4 * u + (lane >> 4);
+      a[u] = i < n && k < n ? x(i, k) : 0.0;
+      b[u] = k < n && j < n ? y(k, j) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], c, 0, 0, 0);
   }
   return c;
 }
@@ -252,7 +258,7 @@ __global__ __launch_bounds__(kSyevThreads) void syev_kernel(SyevArgs g) {
     if (w == 0) {
       const double dr = lane < n ? d[lane] : 0.0, er = lane < n - 1 ? e[lane] : 0.0;
       // [l, hi]: first block without a negligible e
-      const double dn = __shfl_down(dr, 1);   // of all lanes: it reads the neighbour's register
+      const double dn = lane < n - 1 ? d[lane + 1] : 0.0;
       const unsigned long long small =
           __ballot(lane >= n - 1 || fabs(er) <= fmax(2.220446049250313e-16 * (fabs(dr) + fabs(dn)), 1e-18));
       int hi = l;
