@@ -466,7 +466,7 @@ __global__ __launch_bounds__(256) void jk_kernel(JKArgs a) {
   const uint64_t amask = __ballot(active);
   if (a.counts) {
     // per-wave statistics: plain stores into this task's slot (summed by
-    // reduce_counts_kernel), no same-address atomics
+    // reduce_counts_multi_kernel), no same-address atomics
     unsigned int np = active ? (unsigned int)(P.nprim * K.nprim) : 0u;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) np += __shfl_xor(np, o, 64);

@@ -128,8 +128,8 @@ __global__ __launch_bounds__(256) void store_kernel(StoreArgs a) {
 //     all fit (n above 568 for (dd|), 1136 for (dp|)) the launch is repeated
 //     for the next ones; the first pass does the slabs of a and b.
 // Scattered over GG, one lane per quartet, these atomics bounded the
-// transform: C8H18 cc-pVDZ (n = 210) 11.2 ms; packed 3.5 ms (4 ms of kernels
-// over four streams, the (dp|pp) recursion and (ps|ss) longest).
+// transform: C8H18 cc-pVDZ (n = 210) 11.2 ms; packed 3.3 ms (9.6 ms of kernels
+// over four streams, (ds|pp), (ps|ss), (dd|ps) and (pp|pp) longest).
 template <int LA, int LB, int LC, int LD>
 __global__ __launch_bounds__(256) void it_strip_kernel(StoreArgs a) {
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256) void it_strip_kernel(StoreArgs a) {
 
 // ------------------------------------- one wavefront per quartet (high L)
 // One lane per quartet kept these classes' blocks in scratch: (H2O)3 6-31G**
-// (dd|dd) 1060 -> 33 us, (dd|dp) 901 -> 31, the store 4.0 -> 0.56 ms.  Store
+// (dd|dd) 1060 -> 33 us, (dd|dp) 901 -> 31, the store 4.0 -> 0.55 ms.  Store
 // (MODE 0) or transform (MODE 1, packed slabs as above, every update a global
 // atomic: these classes have few quartets): the lanes share the elements of the
 // (ab|cd) block in LDS.

@@ -14,7 +14,7 @@ struct MolDesc {
   const double* prim;      // PrimPair records
   const float* primf;      // the same records in FP32 (mixed precision)
   const double* D;         // n x n density
-  double* Dn;              // nshell x nshell block infinity norms (dnorm_batch writes them)
+  double* Dn;              // nshell x nshell block infinity norms (the prologue writes them)
   const ShellInfo* shells;
   const double* norma;
   double* Graw;            // n x n raw accumulator of everything but J_cd (symmetrised afterwards)
