@@ -20,7 +20,7 @@ def test_tuned_build_is_not_slower_than_the_default():
 
     def least(h):
         t = []
-        for _ in range(12):
+        for _ in range(5):
             t0 = time.perf_counter()
             h.compute_2body_device(dD.ptr, dG.ptr, -0.5)
             t.append(time.perf_counter() - t0)
@@ -31,8 +31,12 @@ def test_tuned_build_is_not_slower_than_the_default():
         x.init_2body_ints()
     g.compute_2body_device(dD.ptr, dG.ptr, -0.5)
     g.autotune(dD.ptr, dG.ptr, -0.5, reps=1)
-    untuned, Gu = least(h)
-    tuned, Gt = least(g)
+    untuned = tuned = 1e9
+    for _ in range(4):          # in turn, so that a slow spell of the machine meets both
+        t, Gu = least(h)
+        untuned = min(untuned, t)
+        t, Gt = least(g)
+        tuned = min(tuned, t)
     h.close()
     g.close()
     assert np.max(np.abs(Gt - Gu)) < 1e-12 * max(1.0, np.max(np.abs(Gu)))
